@@ -416,6 +416,9 @@ struct Problem {
   void* ws;
   size_t ws_bytes;
   bool noalloc = false;  // mi_gemm_noalloc: the library's static scratch is the workspace
+  // A / B is a library buffer whose rows are readable, and zero, up to a whole 16-byte
+  // chunk past its contiguous extent (the gradient chunk of mi_lm_head_xent)
+  bool pad_a = false, pad_b = false;
 };
 
 int validate(const Problem& P) {
@@ -565,8 +568,13 @@ int run(const Problem& P, hipStream_t stream) {
   const int esz = P.dtype_in == MI_BF16 ? 2 : 4;
   const int64_t a_rows = P.M, b_rows = P.N;
   const int64_t a_contig = P.transA ? P.M : P.K, b_contig = P.transB ? P.K : P.N;
-  const int64_t extA = P.K == 0 ? 0 : (P.transA ? (P.K - 1) * P.lda + P.M : (P.M - 1) * P.lda + P.K) * esz;
-  const int64_t extB = P.K == 0 ? 0 : (P.transB ? (P.N - 1) * P.ldb + P.K : (P.K - 1) * P.ldb + P.N) * esz;
+  // A padded operand's last chunk may straddle its edge: along K the zeros add nothing
+  // (the other operand is zero-filled or zero there too), along M or N it only feeds
+  // outputs that are not stored.
+  const int64_t a_ext = P.pad_a ? cdiv(a_contig, CH) * CH : a_contig;
+  const int64_t b_ext = P.pad_b ? cdiv(b_contig, CH) * CH : b_contig;
+  const int64_t extA = P.K == 0 ? 0 : ((P.transA ? P.K : P.M) - 1) * P.lda * esz + a_ext * esz;
+  const int64_t extB = P.K == 0 ? 0 : ((P.transB ? P.N : P.K) - 1) * P.ldb * esz + b_ext * esz;
   const int64_t lim = (int64_t)1 << 31;
   auto span_ok = [&](bool kc, int64_t rows, int64_t ld) {
     // largest offset formed: a row/k line one tile (<= 512 rows, <= 64 k) past the edge
@@ -574,7 +582,7 @@ int run(const Problem& P, hipStream_t stream) {
                            : (P.K + 64) * ld * esz + (rows + 512) * esz;
     return far < lim;
   };
-  const bool fast = vecA && vecB && mult(a_contig) && mult(b_contig) && extA < lim && extB < lim &&
+  const bool fast = vecA && vecB && mult(a_ext) && mult(b_ext) && extA < lim && extB < lim &&
                     span_ok(!P.transA, a_rows, P.lda) && span_ok(P.transB != 0, b_rows, P.ldb);
 
   // SiLU-gate prologue as its own pass when the workspace holds SiLU(A) * A2 (bf16,
@@ -1390,8 +1398,10 @@ size_t lm_fixed_bytes(int64_t rows, int64_t hidden, int64_t chunk, bool dx_acc) 
 
 int lm_gemm(hipStream_t st, int tA, int tB, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
             const void* B, int64_t ldb, float beta, void* C, int64_t ldc, int32_t dtype_c, void* ws,
-            size_t ws_bytes) {
+            size_t ws_bytes, bool pad_a = false, bool pad_b = false) {
   Problem P;
+  P.pad_a = pad_a;
+  P.pad_b = pad_b;
   P.transA = tA; P.transB = tB;
   P.M = M; P.N = N; P.K = K;
   P.alpha = 1.0f; P.beta = beta;
@@ -1492,7 +1502,11 @@ int mi_lm_head_xent(void* stream, const void* X, int64_t ldx, const void* W, int
   int r = herr(launch_xent_chunk_finish((int)rows, (int)vocab, targets, run_m, run_s, xy, scale, row_loss, st));
   if (r == MI_OK && loss_out) r = herr(launch_xent_mean(row_loss, (int)rows, scale, loss_out, st));
   if (r != MI_OK || (!dX && !dW)) return r;
-  // pass 2, last chunk first: its logits are still in L; every other chunk is recomputed
+  // pass 2, last chunk first: its logits are still in L; every other chunk is recomputed.
+  // The gradient kernel leaves zeros up to a whole 16-byte vector past column n, so a chunk
+  // of any width keeps the direct-to-LDS kernels wherever L is the operand that n bounds
+  // (2048 x 2048 -> 32001: the last chunk's 7425 columns took the element-granular
+  // loader, 346 us for dX and 355 for dW; the whole call went from 1645 to 1055 us).
   void* dx_c = dx_acc ? (void*)acc : dX;
   const int64_t dx_ld = dx_acc ? hidden : lddx;
   const int32_t dx_t = dx_acc ? MI_F32 : dx_dtype;
@@ -1507,14 +1521,14 @@ int mi_lm_head_xent(void* stream, const void* X, int64_t ldx, const void* W, int
       r = w_layout == 0 ? lm_gemm(st, 0, 1, rows, hidden, n, L, ldl, w16 + c0, ldw, bx, dx_c, dx_ld, dx_t, gws,
                                   gws_bytes)
                         : lm_gemm(st, 0, 0, rows, hidden, n, L, ldl, w16 + c0 * ldw, ldw, bx, dx_c, dx_ld, dx_t,
-                                  gws, gws_bytes);
+                                  gws, gws_bytes, true);
       if (r != MI_OK) return r;
     }
     if (dW) {  // dW's chunk = dw_beta dW's chunk + X^T dL_c (layout 0) or dL_c^T X (layout 1)
       r = w_layout == 0 ? lm_gemm(st, 1, 0, hidden, n, rows, X, ldx, L, ldl, dw_beta,
-                                  (char*)dW + c0 * esw, lddw, dw_dtype, gws, gws_bytes)
+                                  (char*)dW + c0 * esw, lddw, dw_dtype, gws, gws_bytes, false, true)
                         : lm_gemm(st, 1, 0, n, hidden, rows, L, ldl, X, ldx, dw_beta,
-                                  (char*)dW + c0 * lddw * esw, lddw, dw_dtype, gws, gws_bytes);
+                                  (char*)dW + c0 * lddw * esw, lddw, dw_dtype, gws, gws_bytes, true);
       if (r != MI_OK) return r;
     }
   }

@@ -275,37 +275,27 @@ __global__ void __launch_bounds__(256) xent_chunk_stats_kernel(const uint16_t* L
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint16_t* lrow = L + (int64_t)row * ldl;
   float m = -INFINITY, s = 0.0f;
-  if ((n & 7) == 0 && (ldl & 7) == 0) {  // 16-byte vectors of 8 logits, one rescale per vector
-    for (int v = tid * 8; v < n; v += 256 * 8) {
-      const xu32x4_t q = *(const xu32x4_t*)(lrow + v);
-      float x[8], mx = -INFINITY;
+  // 16-byte vectors of 8 logits, one rescale per vector; columns past n count as -inf
+  // (the row holds whole vectors: ldl is a multiple of 8 and at least n)
+  for (int v = tid * 8; v < n; v += 256 * 8) {
+    const xu32x4_t q = *(const xu32x4_t*)(lrow + v);
+    float x[8], mx = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[e] = elem_of<true>(q, e);
-        mx = fmaxf(mx, x[e]);
-      }
-      if (mx > m) {
-        s = m == -INFINITY ? s * 0.0f : s * __builtin_amdgcn_exp2f((m - mx) * XENT_L2E);  // keeps a NaN
-        m = mx;
-      }
-      if (m != -INFINITY) {
-        const float mneg = -m * XENT_L2E;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], XENT_L2E, mneg));
-      } else {  // every logit so far is -inf or NaN (fmaxf skips NaN): add the NaNs
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += x[e] == -INFINITY ? 0.0f : x[e];
-      }
+    for (int e = 0; e < 8; ++e) {
+      x[e] = v + e < n ? elem_of<true>(q, e) : -INFINITY;
+      mx = fmaxf(mx, x[e]);
     }
-  } else {
-    for (int v = tid; v < n; v += 256) {
-      const float x = bf16_bits_to_f32(lrow[v]);
-      if (x > m) {
-        s = (m == -INFINITY ? s * 0.0f : s * __builtin_amdgcn_exp2f((m - x) * XENT_L2E)) + 1.0f;  // keeps a NaN
-        m = x;
-      } else if (x != -INFINITY) {
-        s += __builtin_amdgcn_exp2f((x - m) * XENT_L2E);  // NaN x propagates
-      }
+    if (mx > m) {
+      s = m == -INFINITY ? s * 0.0f : s * __builtin_amdgcn_exp2f((m - mx) * XENT_L2E);  // keeps a NaN
+      m = mx;
+    }
+    if (m != -INFINITY) {
+      const float mneg = -m * XENT_L2E;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], XENT_L2E, mneg));
+    } else {  // every logit so far is -inf or NaN (fmaxf skips NaN): add the NaNs
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += x[e] == -INFINITY ? 0.0f : x[e];
     }
   }
 #pragma unroll
@@ -349,7 +339,8 @@ __global__ void __launch_bounds__(256) xent_chunk_finish_kernel(int rows, int vo
   run_s[r] = scale / S;
 }
 
-// Gradient of one chunk in place: L[r][v] = scale * (exp(x - m) / s - [c0 + v == y]).
+// Gradient of one chunk in place: L[r][v] = scale * (exp(x - m) / s - [c0 + v == y]), and
+// zeros in the columns past n of the row's last 16-byte vector (ldl is a multiple of 8).
 __global__ void __launch_bounds__(256) xent_chunk_grad_kernel(uint16_t* L, int64_t ldl, int n, int c0,
                                                               const uint32_t* targets, const float* run_m,
                                                               const float* run_inv, float scale) {
@@ -357,25 +348,17 @@ __global__ void __launch_bounds__(256) xent_chunk_grad_kernel(uint16_t* L, int64
   uint16_t* lrow = L + (int64_t)row * ldl;
   const float mneg = -run_m[row] * XENT_L2E, inv = run_inv[row];
   const uint32_t yc = targets[row] - (uint32_t)c0;  // the target's column in the chunk (or past n)
-  const bool vec = (n & 7) == 0 && (ldl & 7) == 0;  // 16-byte rows of 8 logits
-  if (vec) {
-    for (int v = threadIdx.x * 8; v < n; v += 256 * 8) {
-      xu32x4_t q = *(const xu32x4_t*)(lrow + v);
-      float g[8];
+  for (int v = threadIdx.x * 8; v < n; v += 256 * 8) {
+    const xu32x4_t q = *(const xu32x4_t*)(lrow + v);
+    float g[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        g[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(elem_of<true>(q, e), XENT_L2E, mneg)) * inv;
-        if ((uint32_t)(v + e) == yc) g[e] -= scale;
-      }
-      *(xu32x4_t*)(lrow + v) = xu32x4_t{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]),
-                                        pack_bf16x2(g[4], g[5]), pack_bf16x2(g[6], g[7])};
+    for (int e = 0; e < 8; ++e) {
+      g[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(elem_of<true>(q, e), XENT_L2E, mneg)) * inv;
+      if ((uint32_t)(v + e) == yc) g[e] -= scale;
+      if (v + e >= n) g[e] = 0.0f;
     }
-  } else {
-    for (int v = threadIdx.x; v < n; v += 256) {
-      float g = __builtin_amdgcn_exp2f(__builtin_fmaf(bf16_bits_to_f32(lrow[v]), XENT_L2E, mneg)) * inv;
-      if ((uint32_t)v == yc) g -= scale;
-      lrow[v] = (uint16_t)f32_to_bf16_rne(g);
-    }
+    *(xu32x4_t*)(lrow + v) = xu32x4_t{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]),
+                                      pack_bf16x2(g[4], g[5]), pack_bf16x2(g[6], g[7])};
   }
 }
 

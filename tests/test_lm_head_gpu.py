@@ -137,6 +137,28 @@ def test_lm_head_xent_vs_unfused_small(mi, dev, oracle, layout):
     check(host(dW1), host(dW2), TOL_BF16, "dW vs unfused")
 
 
+# rows, hidden, vocab, chunk, layout: chunks whose width is not whole 16-byte vectors (by 1, 4
+# and 7 columns), as one chunk, as a last chunk and as every chunk
+@pytest.mark.parametrize("rows,hidden,vocab,chunk,layout",
+                         [(40, 64, 1001, 0, 1), (130, 128, 2052, 1024, 1), (64, 96, 999, 101, 1),
+                          (40, 64, 1001, 0, 0), (96, 128, 2055, 1024, 0), (7, 8, 9, 5, 1)])
+def test_chunk_width_off_vectors(mi, dev, oracle, rows, hidden, vocab, chunk, layout):
+    """The chunk's zero-padded rows against the separate calls on a packed logits matrix."""
+    import torch
+
+    x, w, t = _problem(oracle, rows, hidden, vocab, layout, 960 + vocab % 7)
+    X, W, T = _tensors(dev, x, w, t)
+    dW1 = torch.zeros(W.shape, dtype=torch.float32, device=dev)
+    dW2 = torch.zeros_like(dW1)
+    need = mi.lm_head_xent_workspace_size(rows, hidden, vocab, chunk)
+    ws = torch.full((need,), 0xff, dtype=torch.uint8, device=dev)  # every unwritten value a NaN
+    l1, r1, dX1 = mi.lm_head_xent(X, W, T, w_layout=layout, chunk=chunk, dW=dW1, workspace=ws)
+    l2, r2, dX2 = _unfused(mi, X, W, T, layout, 0.0, dW2)
+    _loss_close(host(r1), host(r2), 2e-3)
+    check(host(dX1), host(dX2), TOL_BF16, "dX vs unfused")
+    check(host(dW1), host(dW2), TOL_BF16, "dW vs unfused")
+
+
 def test_chunk_size_and_determinism(mi, dev, oracle):
     """Chunks of 8192, 2048 and one chunk agree; repeated calls give the same bits."""
     rows, hidden, vocab = 512, 256, 20000
