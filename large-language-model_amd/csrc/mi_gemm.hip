@@ -401,6 +401,15 @@ bool rows_overlap(const void* a, const void* b, int64_t bytes) {
   return a0 < b0 + (uintptr_t)bytes && b0 < a0 + (uintptr_t)bytes;
 }
 
+// Whether the direct-to-LDS kernels take this K without a workspace: a K-contiguous
+// operand whose K is not whole 16-byte chunks has a straddling chunk to zero.  Without a
+// workspace such a single problem keeps the register-staged kernel, the plan that
+// mi_gemm_describe reports for it; with one, and in a batch, it takes the direct-to-LDS
+// kernels (fp32 forward, dX and dW of 1500 x 1343 x 811 in us: 282 -> 141; 77 x 1343 x
+// 811: 92 -> 44; bf16 2000 x 3144 x 942, rows of whole dwords: 721 -> 87).
+constexpr size_t kTailWorkspace = 256;  // what mi_gemm_workspace_size asks for then, without a split
+bool tail_ok(int transA, int transB, int64_t K, int64_t ch) { return (transA && !transB) || K % ch == 0; }
+
 struct Problem {
   int transA, transB;
   int64_t M, N, K;
@@ -582,8 +591,22 @@ int run(const Problem& P, hipStream_t stream) {
                            : (P.K + 64) * ld * esz + (rows + 512) * esz;
     return far < lim;
   };
-  const bool fast = vecA && vecB && mult(a_ext) && mult(b_ext) && extA < lim && extB < lim &&
-                    span_ok(!P.transA, a_rows, P.lda) && span_ok(P.transB != 0, b_rows, P.ldb);
+  const bool spanA = extA < lim && span_ok(!P.transA, a_rows, P.lda);
+  const bool spanB = extB < lim && span_ok(P.transB != 0, b_rows, P.ldb);
+  bool fast = vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB;
+  // The direct-to-LDS kernels (every bf16 mode but the prologue, plain fp32) need no
+  // more than 4-byte alignment: a buffer load's address and its bounds check work in dwords.
+  // A row-contiguous chunk that straddles the matrix edge feeds outputs that are not
+  // stored; a K-contiguous one is zeroed past K in LDS (tail_ok).
+  const bool dlds = P.dtype_in == MI_BF16 ? mode != MODE_PROLOGUE : mode == MODE_PLAIN;
+  if (!fast && dlds && spanA && spanB) {
+    auto dw = [&](const void* q, int64_t ld, int64_t o, int64_t i, int64_t sg) {
+      return ((uintptr_t)q & 3u) == 0 && (esz == 4 || (ld % 2 == 0 && o % 2 == 0 && i % 2 == 0 && sg % 2 == 0));
+    };
+    fast = dw(P.A, P.lda, b.a_outer, b.a_inner, b.seg_a) && dw(P.B, P.ldb, b.b_outer, b.b_inner, b.seg_b) &&
+           (!P.ep.B2 || ((uintptr_t)P.ep.B2 & 3u) == 0) &&
+           (tail_ok(P.transA, P.transB, P.K, CH) || b.batch > 1 || (P.ws && P.ws_bytes > 0));
+  }
 
   // SiLU-gate prologue as its own pass when the workspace holds SiLU(A) * A2 (bf16,
   // one matrix, 16-byte rows): the activation is written once and the GEMM runs
@@ -687,11 +710,11 @@ int run(const Problem& P, hipStream_t stream) {
   p.c_bf16 = P.dtype_c == MI_BF16;
   p.bias_bf16 = P.ep.bias_dtype == MI_BF16;
   p.r_bf16 = P.ep.residual_dtype == MI_BF16;
-  p.vecA = vecA;
-  p.vecB = vecB;
   p.cvec = cvec;
-  p.extA = (uint32_t)(fast ? extA : 0);
-  p.extB = (uint32_t)(fast ? extB : 0);
+  // whole dwords: the buffer's bounds check would drop the dword that holds a last odd
+  // bf16 element (the dword itself is aligned, so it lies in the element's page)
+  p.extA = (uint32_t)(spanA ? (extA + 3) / 4 * 4 : 0);
+  p.extB = (uint32_t)(spanB ? (extB + 3) / 4 * 4 : 0);
   p.krot = rotate_k(P, plan) ? 1 : 0;
   p.group_m = group_rows(P, plan);
 
@@ -841,12 +864,13 @@ const char* mi_version(void) { return "mi_gemm 0.1 (gfx950)"; }
 
 size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int64_t K,
                               int32_t dtype_in, int32_t dtype_c, int64_t batch) {
-  (void)transA; (void)transB; (void)dtype_c;
+  (void)dtype_c;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
   int cus = 256;
   if (init_devices() == MI_OK) cus = current_cus();
   const Plan pl = make_plan(dtype_in, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, true);
-  return pl.splits > 1 ? (size_t)pl.splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float) : 0;
+  if (pl.splits > 1) return (size_t)pl.splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float);
+  return batch == 1 && !tail_ok(transA, transB, K, dtype_in == MI_BF16 ? 8 : 4) ? kTailWorkspace : 0;
 }
 
 int mi_gemm(void* stream, int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
@@ -1552,11 +1576,16 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   if (init_devices() == MI_OK) cus = current_cus();
   const int mode = epi_mode == 1 ? MODE_DUAL : (epi_mode == 2 ? MODE_PROLOGUE : MODE_PLAIN);
   const int64_t ws = (int64_t)(workspace_bytes / sizeof(float));
-  // packed operands (leading dimension = contiguous extent), 16-byte-aligned bases: the
-  // 16-byte loaders need the contiguous extents in whole 16-byte chunks, as run() checks
+  // packed operands (leading dimension = contiguous extent), 16-byte-aligned bases, as
+  // run() checks them: rows of whole 16-byte chunks, or for the direct-to-LDS kernels of
+  // whole dwords
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
-  const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0);
+  const bool dlds = dtype_in == MI_BF16 ? mode != MODE_PROLOGUE : mode == MODE_PLAIN;
+  const int64_t dw = dtype_in == MI_BF16 ? 2 : 1;
+  const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) ||
+                    (dlds && a_contig % dw == 0 && b_contig % dw == 0 &&
+                     (tail_ok(transA, transB, K, ch) || batch > 1 || ws > 0));
   const Plan pl = make_plan(dtype_in, M, N, K, batch, mode, ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;

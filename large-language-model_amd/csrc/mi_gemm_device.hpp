@@ -57,7 +57,6 @@ struct Params {
   float mask_value;
   float alpha, beta;
   int c_bf16, bias_bf16, r_bf16;
-  int vecA, vecB;  // 16-byte global loads legal for A (and A2) / B (and B2)
   int cvec;        // 4-wide C / R / bias accesses legal
   uint32_t extA, extB;  // byte extent of one batch/segment matrix of A (A2) / B (B2)
   const float* row_scale;  // optional [M] fp32 factor on row m of alpha * acc (a folded RMSNorm)
@@ -110,12 +109,12 @@ struct ElemTraits;
 template <>
 struct ElemTraits<float> {
   static constexpr int CH = 4;  // elements per 16-byte chunk
-  __device__ static uint32_t bits(const void* p, int64_t i) { return ((const uint32_t*)p)[i]; }
+  typedef uint32_t bits_t;
 };
 template <>
 struct ElemTraits<__bf16> {
   static constexpr int CH = 8;
-  __device__ static uint32_t bits(const void* p, int64_t i) { return ((const uint16_t*)p)[i]; }
+  typedef uint16_t bits_t;
 };
 
 // Pack CH scalar bit patterns into a 16-byte chunk.
@@ -132,15 +131,17 @@ __device__ __forceinline__ u32x4_t pack_chunk(const uint32_t* e) {
 }
 
 // Load the 16-byte chunk of CH consecutive elements starting at element index
-// `i` of `p`, `n_ok` of which are in bounds (0..CH).  vec: the chunk is
-// 16-byte aligned and the fast path may be used.
+// `i` of `p`, `n_ok` of which are in bounds (0..CH), element by element.
 template <typename T>
-__device__ __forceinline__ u32x4_t load_chunk(const void* p, int64_t i, int n_ok, bool vec) {
+__device__ __forceinline__ u32x4_t load_chunk(const void* p, int64_t i, int n_ok) {
   constexpr int CH = ElemTraits<T>::CH;
-  if (n_ok >= CH && vec) return *(const u32x4_t*)((const T*)p + i);
+  // operand pointers passed through scalar registers have lost their address space, and a
+  // flat load would count as an LDS access too
+  typedef __attribute__((address_space(1))) const typename ElemTraits<T>::bits_t gbits_t;
+  gbits_t* g = (gbits_t*)(uintptr_t)p + i;
   uint32_t e[CH];
 #pragma unroll
-  for (int j = 0; j < CH; ++j) e[j] = (j < n_ok) ? ElemTraits<T>::bits(p, i + j) : 0u;
+  for (int j = 0; j < CH; ++j) e[j] = (j < n_ok) ? (uint32_t)g[j] : 0u;
   return pack_chunk<T>(e);
 }
 
@@ -176,7 +177,11 @@ __device__ __forceinline__ u32x4_t swiglu_chunk(u32x4_t g, u32x4_t u) {
 //   one branch-free buffer_load_dwordx4.  Requires every chunk fully inside or
 //   fully outside the matrix, 16-byte alignment and 31-bit byte offsets (checked
 //   on the host).
-// !FAST: element-granular bounds for any shape, leading dimension or alignment.
+// !FAST: any shape, leading dimension or alignment.  A K tile that lies inside the
+//   operand (see inner_) is read with branch-free 16-byte loads at the elements' own
+//   alignment, rows past the matrix edge clamped to its last row (they only feed
+//   outputs that are not stored); the last K tile, and operands whose byte offsets
+//   exceed 31 bits, take element-granular bounds.
 
 constexpr uint32_t kBufOOB = 0x80000000u;          // offset past any extent < 2^31
 constexpr int kBufFlags = 0x00020000;               // raw-buffer dword3 for gfx9-family
@@ -227,13 +232,14 @@ struct TileLoader {
   int koff;                       // KC: this thread's chunk column * CH
   int rows_, row0_;
   int64_t ld_;
+  uint32_t goff[FAST ? 1 : (KC ? NCK : NBLK)];  // !FAST: byte offsets inside a K tile, rows clamped
+  bool inner_;                                  // !FAST: the tile's loads need no bounds
   // per K tile
   __amdgpu_buffer_rsrc_t rs, rs2;
   const void* base_;
   const void* base2_;
   uint32_t kv0, kmask;
   int k0_, kseg_;
-  bool vec_;
 
   __device__ __forceinline__ void init(int64_t ld, int rows, int row0) {
     const int tid = threadIdx.x;
@@ -254,6 +260,20 @@ struct TileLoader {
           boff[i] = (b < NBLK_TOT && grow < rows) ? (uint32_t)(grow * ESZ + kb * CH * ldb) : kBufOOB;
         }
       }
+    } else if constexpr (KC) {
+#pragma unroll
+      for (int u = 0; u < NCK; ++u) {
+        const int idx = tid + NT * u;
+        const int grow = row0 + (idx < R * 8 ? idx >> 3 : 0);
+        goff[u] = (uint32_t)(grow < rows ? grow : rows - 1) * (uint32_t)(ld * ESZ) + (idx & 7) * 16;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NBLK; ++i) {
+        const int b = tid + NT * i < NBLK_TOT ? tid + NT * i : NBLK_TOT - 1;
+        const int grow = row0 + (b % (R / CH)) * CH, kb = b / (R / CH);
+        goff[i] = (uint32_t)(grow < rows ? grow : rows - 1) * ESZ + (uint32_t)(kb * CH) * (uint32_t)(ld * ESZ);
+      }
     }
   }
 
@@ -261,11 +281,10 @@ struct TileLoader {
   // and K segment, ext their byte extent, k0 the tile's first K, kseg the K extent.
   // live = false turns every load of the tile into an out-of-range no-op.
   __device__ __forceinline__ void set_tile(const void* base, const void* base2, uint32_t ext, int k0,
-                                           int kseg, bool vec, bool live) {
+                                           int kseg, bool live) {
     k0_ = k0;
     kseg_ = live ? kseg : 0;
     if constexpr (FAST) {
-      (void)vec;
       rs = make_rsrc(base, ext);
       if constexpr (PRO) rs2 = make_rsrc(base2, ext);
       // offsets stay below 2^31, so OR-ing the top bit moves a chunk out of range
@@ -276,11 +295,26 @@ struct TileLoader {
         kmask = live ? 0u : kBufOOB;
       }
     } else {
-      (void)ext;
       base_ = base;
       base2_ = base2;
-      vec_ = vec;
+      // ext: the operand's byte extent, 0 when an offset could exceed 31 bits.  A
+      // row-contiguous chunk may run past the last row into the next k line, which
+      // exists for every k line of the tile but the operand's last.
+      const int kend = k0 + 8 * CH;
+      inner_ = live && ext != 0 &&
+               (KC ? kend <= kseg
+                   : (kend <= kseg && row0_ + R <= rows_) || (kend < kseg && ld_ >= CH));
     }
+  }
+
+  // !FAST: 16 bytes at a byte offset of the K tile k0_ of `base`.
+  __device__ __forceinline__ u32x4_t load_inner(const void* base, int64_t k_bytes, uint32_t off) const {
+    typedef __attribute__((address_space(1))) const char gchar_t;
+    typedef __attribute__((address_space(1))) const typename ElemTraits<T>::bits_t gbits_t;
+    gchar_t* tile = (gchar_t*)(uintptr_t)base + k_bytes;
+    u32x4_t v;
+    __builtin_memcpy(&v, (gbits_t*)(tile + off), 16);
+    return v;
   }
 
   __device__ __forceinline__ void load_unit(int u) {
@@ -297,6 +331,12 @@ struct TileLoader {
         st[u] = buf_load16(rs, vo);
         if constexpr (PRO) st2[u] = buf_load16(rs2, vo);
       }
+    } else if (inner_) {
+      const int64_t ldb64 = ld_ * ESZ;
+      const int64_t kb = KC ? (int64_t)k0_ * ESZ : (k0_ + u % CH) * ldb64;
+      const uint32_t off = goff[KC ? u : u / CH];
+      st[u] = load_inner(base_, kb, off);
+      if constexpr (PRO) st2[u] = load_inner(base2_, kb, off);
     } else {
       if constexpr (KC) {
         const int idx = tid + NT * u;
@@ -305,8 +345,8 @@ struct TileLoader {
         int n_ok = (grow < rows_ && idx < R * 8) ? kseg_ - gk : 0;
         n_ok = n_ok < 0 ? 0 : (n_ok > CH ? CH : n_ok);
         const int64_t off = (int64_t)grow * ld_ + gk;
-        st[u] = load_chunk<T>(base_, off, n_ok, vec_);
-        if constexpr (PRO) st2[u] = load_chunk<T>(base2_, off, n_ok, vec_);
+        st[u] = load_chunk<T>(base_, off, n_ok);
+        if constexpr (PRO) st2[u] = load_chunk<T>(base2_, off, n_ok);
       } else {
         const int i = u / CH, kk = u % CH;
         const int b = tid + NT * i;
@@ -317,8 +357,8 @@ struct TileLoader {
         const int gk = k0_ + kb * CH + kk;
         const int nk = (gk < kseg_) ? n_ok : 0;
         const int64_t off = (int64_t)gk * ld_ + grow;
-        st[u] = load_chunk<T>(base_, off, nk, vec_);
-        if constexpr (PRO) st2[u] = load_chunk<T>(base2_, off, nk, vec_);
+        st[u] = load_chunk<T>(base_, off, nk);
+        if constexpr (PRO) st2[u] = load_chunk<T>(base2_, off, nk);
       }
     }
   }
@@ -623,10 +663,10 @@ __global__ void __launch_bounds__(256)
     const int seg = itc / per_seg;
     const int k0 = (klo + (itc - seg * per_seg)) * KT;
     la.set_tile(Ab + (int64_t)seg * p.segA, PRO ? (const void*)(A2b + (int64_t)seg * p.segA) : nullptr,
-                p.extA, k0, p.K, p.vecA, live);
-    lb.set_tile(Bb + (int64_t)seg * p.segB, nullptr, p.extB, k0, p.K, p.vecB, live);
+                p.extA, k0, p.K, live);
+    lb.set_tile(Bb + (int64_t)seg * p.segB, nullptr, p.extB, k0, p.K, live);
     if constexpr (MODE == MODE_DUAL)
-      lb2.set_tile(B2b + (int64_t)seg * p.segB, nullptr, p.extB, k0, p.K, p.vecB, live);
+      lb2.set_tile(B2b + (int64_t)seg * p.segB, nullptr, p.extB, k0, p.K, live);
   };
   constexpr int NLA = TileLoader<T, BM, AK, PRO, FAST>::NUNIT;
   constexpr int NLB = TileLoader<T, BN, BK, false, FAST>::NUNIT;

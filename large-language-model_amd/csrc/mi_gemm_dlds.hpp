@@ -235,6 +235,20 @@ struct DldsOperand {
         16, (int)vo, 0, 0, 0);
   }
 
+  // Zero the elements past the K extent in the chunk that straddles it (chunk c of every
+  // row of stage J, whose first nv elements are inside): the DMA has filled them with
+  // what follows the row in memory.
+  template <int J>
+  __device__ __forceinline__ void zero_tail(uint32_t region, int c, int nv) const {
+    static_assert(KC, "only a K-contiguous operand has a straddling chunk");
+    typedef std::conditional_t<ES == 2, uint16_t, uint32_t> bits_t;
+    typedef __attribute__((address_space(3))) volatile bits_t lds_bits_t;
+    for (int r = threadIdx.x; r < R; r += 64 * NW) {
+      const uint32_t a = region + (uint32_t)(J * BYTES + r * (BK * ES) + 16 * kc_swz<NCH>(r, c));
+      for (int e = nv; e < EPC; ++e) *(lds_bits_t*)(uintptr_t)(a + (uint32_t)(e * ES)) = 0;
+    }
+  }
+
   // MFMA fragment f (rows w0+32f .. +31 of the wave tile), K substep S of stage J,
   // as 8 bf16 per lane.  In a K-contiguous tile fragments f and f+2 share the
   // swizzle, 64 rows apart; a row-contiguous tile steps 16 k-rows per substep.
@@ -274,8 +288,8 @@ struct DldsOperand {
 };
 
 // Kernel variants (VAR bits): the K segment length is not a multiple of BK
-// (K-contiguous operands then mask the chunks past the segment end), and the
-// problem takes the direct epilogue (every tile full, epilogue alpha / SiLU
+// (K-contiguous operands then mask the chunks past the segment end, and zero the rest
+// of a chunk that straddles it in LDS), and the problem takes the direct epilogue (every tile full, epilogue alpha / SiLU
 // gate, beta*C and the output conversion only, no split-K).  One kernel holding
 // both epilogues would need the accumulators in two places at once.
 enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4 };
@@ -454,6 +468,27 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     else ob.template load<JF, KTB>(o - OpA::NU - OpB::NU, t.rb2, t.k0, ob2.dma);
   };
 
+  // The K tile whose last chunk straddles the K extent (K not a whole number of 16-byte
+  // chunks): once its DMA has landed, the chunk's elements past K are zeroed in LDS, behind
+  // one more barrier.  c_kt follows the K tile that the next barrier makes visible.
+  constexpr int EPC = 16 / ES;
+  int c_kt = uniform(it0 - d_seg * per_seg + rot);
+  const int tail_nv = p.K % EPC;
+  const int tail_kt = tail_nv ? kt_seg - 1 - klo : -1;
+  auto zero_tail = [&](auto J_c) __attribute__((always_inline)) {
+    constexpr int J = decltype(J_c)::value;
+    if constexpr (KTAIL) {
+      if (c_kt == tail_kt) {
+        const int c = (p.K - (kt_seg - 1) * BK) / EPC;
+        if constexpr (AK) oa.template zero_tail<J>(lds0 + A_REG, c, tail_nv);
+        if constexpr (BKC) ob.template zero_tail<J>(lds0 + B_REG, c, tail_nv);
+        if constexpr (BKC && DUAL) ob.template zero_tail<J>(lds0 + B2_REG, c, tail_nv);
+        lds_ring_barrier();
+      }
+      if (++c_kt == per_seg) c_kt = 0;
+    }
+  };
+
   // EARLY (two stages of four substeps): each substep has its own fragment set,
   // so a K tile's fragments are all read by the end of its second substep and
   // its stage is free from then on; otherwise substep s uses set s & 1.
@@ -587,6 +622,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   }
   lds_ring_barrier();
   if (it0 < it1) {
+    zero_tail(ic<0>{});
 #pragma unroll
     for (int o = 0; o < NREAD; ++o) read_op(o, ic<0>{}, ic<0>{}, 0);
     if constexpr (EARLY) {
@@ -621,6 +657,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     }
     wait_vmcnt<VM_WAIT>();
     lds_ring_barrier();
+    zero_tail(ic<JN>{});
     substep(ic<NSUB - 1>{}, ic<0>{}, ic<JN>{}, DmaLast{}, ic<JF>{}, t);
   };
   // EARLY: substeps 0 and 1 of tile it read sets 2 and 3 (the rest of tile it);
@@ -636,6 +673,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     substep4(ic<1>{}, ic<3>{}, ic<3>{}, ic<J>{}, ic<0>{}, ic<J>{}, t);
     wait_vmcnt<0>();
     lds_ring_barrier();
+    zero_tail(ic<JN>{});
     // The substeps that issue the next tile's DMA run at raised wave priority: the
     // wave that leaves the barrier first keeps the SIMD's issue slot for its MFMAs,
     // reads and DMA instead of alternating with its partner wave instruction by

@@ -679,3 +679,49 @@ def test_cpp_bridge_program():
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     print(r.stdout)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("bf16,pad", [(True, 0), (True, 1), (True, 2), (False, 0), (False, 1)])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)], ids=["NN", "NT", "TN", "TT"])
+def test_unaligned_operands(mi, dev, bf16, pad, tA, tB):
+    """Operands off 16-byte alignment on both their kernels (with a workspace or in a batch the
+    direct-to-LDS ones where rows are whole dwords, else the register-staged one): sizes around
+    a 16-byte chunk, a K tile and an output tile, leading dimensions `pad` past the row, a
+    base one dword (or, bf16 with odd rows, one element) off, NaN in every gap around and
+    between the rows, one row of A infinite. Integer products, bit for bit."""
+    import torch
+
+    dt = torch.bfloat16 if bf16 else torch.float32
+    ch = 8 if bf16 else 4
+    rng = np.random.default_rng(7 + 2 * tA + tB + 10 * pad)
+    ws = torch.empty(8 << 20, dtype=torch.float32, device=dev)
+
+    def place(mats, ld, off):  # the matrices in one NaN-filled buffer, `off` elements in
+        rows, cols = mats[0].shape
+        buf = torch.full((off + len(mats) * rows * ld + 64,), float("nan"), dtype=dt, device=dev)
+        for i, m in enumerate(mats):
+            v = buf[off + i * rows * ld: off + (i + 1) * rows * ld].view(rows, ld)
+            v[:, :cols] = torch.from_numpy(m).to(dev, dt)
+        return buf[off:]
+
+    for M, N, K in [(1, 1, 3), (33, 7, 5), (63, 65, 31), (130, 70, 33), (129, 190, 331), (257, 96, ch * 64 + 1),
+                    (96, 130, ch * 8 - 1), (70, 259, 2050)]:
+        for nb, with_ws in [(1, True), (1, False), (3, False)]:
+            a = rng.integers(-4, 5, (nb, M, K)).astype(np.float32)
+            b = rng.integers(-4, 5, (nb, K, N)).astype(np.float32)
+            b[b == 0] = 1.0  # an infinity times zero would hide which row it came from
+            ref = np.stack([a[i].astype(np.int64) @ b[i].astype(np.int64) for i in range(nb)]).astype(np.float64)
+            hot = M // 2  # a row of infinities next to the rows that must stay finite
+            a[:, hot] = np.inf
+            As, Bs = [layout(m, tA) for m in a], [layout(m, tB) for m in b]
+            lda, ldb = As[0].shape[1] + pad, Bs[0].shape[1] + pad
+            off = 1 if not bf16 or lda % 2 or ldb % 2 else 2
+            A, B = place(As, lda, off), place(Bs, ldb, off)
+            C = torch.full((nb, M, N), 5.0, dtype=torch.float32, device=dev)
+            bt = mi.make_batch(nb, 1, a=(As[0].shape[0] * lda, 0, 1), b=(Bs[0].shape[0] * ldb, 0, 1), c=(M * N, 0, 1))
+            mi.gemm_batched(A, B, C, M, N, K, bt, transA=tA, transB=tB, lda=lda, ldb=ldb,
+                            workspace=ws if with_ws else None)
+            got = host(C)
+            keep = np.arange(M) != hot
+            assert np.array_equal(got[:, keep], ref[:, keep]), (M, N, K, nb, with_ws)
+            assert not np.isfinite(got[:, hot]).any(), (M, N, K, nb, with_ws)
