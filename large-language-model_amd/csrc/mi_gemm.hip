@@ -24,6 +24,7 @@
 #include "mi_norm.hpp"
 #include "mi_convert.hpp"
 #include "mi_gemm_kernels.hpp"
+#include "mi_skinny.hpp"
 
 using namespace mig;
 
@@ -338,11 +339,26 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
   return plan_for(CFG_S, best);
 }
 
+// Products of few rows with op(A) not transposed, in whole 16-byte chunks of K: the kernels
+// of mi_skinny.hip, which read B once at the rate HBM gives (a layer's products on 8 rows:
+// 128-row tiles split along K spent 99 us of which 45 in the dual product's 44 workgroups).
+bool skinny_fits(int transA, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t segs, int causal, int mode,
+                 int64_t ch) {
+  return !transA && M <= SKINNY_MAX_M && (M <= 32 || N * K * (16 / ch) <= SKINNY_WIDE_BYTES) && K % ch == 0 &&
+         batch == 1 && segs == 1 && causal == MI_CAUSAL_NONE && mode != MODE_PROLOGUE;
+}
+Plan skinny_as_plan(const SkinnyPlan& sk) { return Plan{CFG_SKINNY, sk.splits, 1, sk.strips}; }
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Text of a plan, as mi_gemm_describe and the profiler records show it.
 void describe_plan(char* buf, size_t len, int dtype_in, bool fast, const Plan& pl, int transA,
                    int transB, int64_t batch) {
+  if (pl.cfg == CFG_SKINNY) {
+    std::snprintf(buf, len, "skinny %s N%s split%d strips%d", dtype_in == MI_BF16 ? "bf16" : "f32",
+                  transB ? "T" : "N", pl.splits, pl.tiles_n);
+    return;
+  }
   const CfgShape sh = shape_of(dtype_in, pl.cfg);
   const char* kind = (dtype_in == MI_BF16 && fast && pl.cfg != CFG_PRO)
                          ? (pl.cfg == CFG_W || pl.cfg == CFG_V ? "dlds-kg2" : "dlds")
@@ -593,20 +609,20 @@ int run(const Problem& P, hipStream_t stream) {
   };
   const bool spanA = extA < lim && span_ok(!P.transA, a_rows, P.lda);
   const bool spanB = extB < lim && span_ok(P.transB != 0, b_rows, P.ldb);
-  bool fast = vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB;
-  // The direct-to-LDS kernels (every bf16 mode but the prologue, plain fp32) need no
-  // more than 4-byte alignment: a buffer load's address and its bounds check work in dwords.
-  // A row-contiguous chunk that straddles the matrix edge feeds outputs that are not
-  // stored; a K-contiguous one is zeroed past K in LDS (tail_ok).
+  // The skinny and the direct-to-LDS kernels (every bf16 mode but the prologue, plain fp32)
+  // need no more than 4-byte alignment: a buffer load's address and its bounds check work in
+  // dwords.  A row-contiguous chunk that straddles the matrix edge feeds outputs that are
+  // not stored; a K-contiguous one is zeroed past K in LDS (tail_ok).
+  auto dw = [&](const void* q, int64_t ld, int64_t o, int64_t i, int64_t sg) {
+    return ((uintptr_t)q & 3u) == 0 && (esz == 4 || (ld % 2 == 0 && o % 2 == 0 && i % 2 == 0 && sg % 2 == 0));
+  };
+  const bool dwords = spanA && spanB && dw(P.A, P.lda, b.a_outer, b.a_inner, b.seg_a) &&
+                      dw(P.B, P.ldb, b.b_outer, b.b_inner, b.seg_b) && (!P.ep.B2 || ((uintptr_t)P.ep.B2 & 3u) == 0);
   const bool dlds = P.dtype_in == MI_BF16 ? mode != MODE_PROLOGUE : mode == MODE_PLAIN;
-  if (!fast && dlds && spanA && spanB) {
-    auto dw = [&](const void* q, int64_t ld, int64_t o, int64_t i, int64_t sg) {
-      return ((uintptr_t)q & 3u) == 0 && (esz == 4 || (ld % 2 == 0 && o % 2 == 0 && i % 2 == 0 && sg % 2 == 0));
-    };
-    fast = dw(P.A, P.lda, b.a_outer, b.a_inner, b.seg_a) && dw(P.B, P.ldb, b.b_outer, b.b_inner, b.seg_b) &&
-           (!P.ep.B2 || ((uintptr_t)P.ep.B2 & 3u) == 0) &&
-           (tail_ok(P.transA, P.transB, P.K, CH) || b.batch > 1 || (P.ws && P.ws_bytes > 0));
-  }
+  const bool fast = (vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB) ||
+                    (dwords && dlds &&
+                     (tail_ok(P.transA, P.transB, P.K, CH) || b.batch > 1 || (P.ws && P.ws_bytes > 0)));
+  const bool skinny = dwords && skinny_fits(P.transA, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode, CH);
 
   // SiLU-gate prologue as its own pass when the workspace holds SiLU(A) * A2 (bf16,
   // one matrix, 16-byte rows): the activation is written once and the GEMM runs
@@ -643,8 +659,13 @@ int run(const Problem& P, hipStream_t stream) {
   // mi_gemm_noalloc: the plan mi_gemm makes with unlimited workspace, refused when
   // its partials would not fit the scratch array (so both entry points run the same
   // kernels on the same problem)
-  Plan plan = make_plan(P.dtype_in, P.M, P.N, Ktot, b.batch, mode, allow_split || P.noalloc,
-                        P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
+  // a dual product's partials are no part of what mi_gemm_workspace_size promises, so
+  // mi_gemm_noalloc runs it as mi_gemm does without a workspace
+  const SkinnyPlan sk = skinny_plan(P.dtype_in == MI_BF16, P.transB != 0, mode == MODE_DUAL, P.M, P.N, P.K,
+                                    allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0);
+  Plan plan = skinny ? skinny_as_plan(sk)
+                     : make_plan(P.dtype_in, P.M, P.N, Ktot, b.batch, mode, allow_split || P.noalloc,
+                                 P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
   if (P.noalloc && plan.splits > 1 && (int64_t)plan.splits * P.M * P.N * b.batch > ws_elems)
     return fail(MI_ERR_WORKSPACE,
                 "mi_gemm_noalloc: split-K by %d needs %lld bytes of scratch, above its %lld-byte "
@@ -667,8 +688,9 @@ int run(const Problem& P, hipStream_t stream) {
   if (P.ep.row_scale && fast_epi)
     epi_kind = (P.dtype_in == MI_BF16 && fast && !P.transA && P.K % kstep == 0 &&
                 (plan.cfg == CFG_L || plan.cfg == CFG_M || plan.cfg == CFG_S)) ? 2 : 0;
-  KernelFn fn = pick_kernel(P.dtype_in, P.transA, P.transB, plan.cfg, fast, P.K % kstep != 0, epi_kind);
-  if (!fn) return fail(MI_ERR_UNSUPPORTED, "no kernel for this layout / mode");
+  KernelFn fn = skinny ? nullptr
+                       : pick_kernel(P.dtype_in, P.transA, P.transB, plan.cfg, fast, P.K % kstep != 0, epi_kind);
+  if (!fn && !skinny) return fail(MI_ERR_UNSUPPORTED, "no kernel for this layout / mode");
 
   Params p;
   std::memset(&p, 0, sizeof(p));
@@ -715,8 +737,8 @@ int run(const Problem& P, hipStream_t stream) {
   // bf16 element (the dword itself is aligned, so it lies in the element's page)
   p.extA = (uint32_t)(spanA ? (extA + 3) / 4 * 4 : 0);
   p.extB = (uint32_t)(spanB ? (extB + 3) / 4 * 4 : 0);
-  p.krot = rotate_k(P, plan) ? 1 : 0;
-  p.group_m = group_rows(P, plan);
+  p.krot = !skinny && rotate_k(P, plan) ? 1 : 0;
+  p.group_m = skinny ? 1 : group_rows(P, plan);
 
   const int64_t nblocks = (int64_t)plan.tiles_m * plan.tiles_n * plan.splits * b.batch;
   if (nblocks > INT32_MAX) return fail(MI_ERR_SHAPE, "too many tiles");
@@ -741,10 +763,15 @@ int run(const Problem& P, hipStream_t stream) {
       g_prof_free[pe.dev].push_back(pe.e1);
     }
   };
-  hipLaunchKernelGGL(fn, dim3((unsigned)nblocks), dim3((unsigned)ts.threads), 0, stream, p);
-  hipError_t e = hipGetLastError();
+  hipError_t e;
+  if (skinny) {
+    e = launch_skinny(p, sk, P.dtype_in == MI_BF16, P.transB != 0, mode == MODE_DUAL, stream);
+  } else {
+    hipLaunchKernelGGL(fn, dim3((unsigned)nblocks), dim3((unsigned)ts.threads), 0, stream, p);
+    e = hipGetLastError();
+  }
   if (e != hipSuccess) return drop_events(), fail(MI_ERR_HIP, "gemm launch: %s", hipGetErrorString(e));
-  if (plan.splits > 1) {
+  if (plan.splits > 1 && !skinny) {
     const int64_t work = b.batch * P.M * ((P.N + 3) / 4);
     const int64_t grid = std::min<int64_t>(cdiv(work, 256), 8 * (int64_t)current_cus());
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)grid), dim3(256), 0, stream, p);
@@ -869,8 +896,15 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
   int cus = 256;
   if (init_devices() == MI_OK) cus = current_cus();
   const Plan pl = make_plan(dtype_in, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, true);
-  if (pl.splits > 1) return (size_t)pl.splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float);
-  return batch == 1 && !tail_ok(transA, transB, K, dtype_in == MI_BF16 ? 8 : 4) ? kTailWorkspace : 0;
+  size_t need = pl.splits > 1 ? (size_t)pl.splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float) : 0;
+  const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
+  if (skinny_fits(transA, M, N, K, batch, 1, MI_CAUSAL_NONE, MODE_PLAIN, ch)) {
+    // operands that rule the skinny kernels out take the tile plan, so room for either
+    const SkinnyPlan sk = skinny_plan(dtype_in == MI_BF16, transB != 0, false, M, N, K, INT64_MAX / 8);
+    if (sk.splits > 1) need = std::max(need, (size_t)sk.splits * (size_t)M * (size_t)N * sizeof(float));
+  }
+  if (need) return need;
+  return batch == 1 && !tail_ok(transA, transB, K, ch) ? kTailWorkspace : 0;
 }
 
 int mi_gemm(void* stream, int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
@@ -1583,10 +1617,12 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
   const bool dlds = dtype_in == MI_BF16 ? mode != MODE_PROLOGUE : mode == MODE_PLAIN;
   const int64_t dw = dtype_in == MI_BF16 ? 2 : 1;
+  const bool dwords = a_contig % dw == 0 && b_contig % dw == 0;
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) ||
-                    (dlds && a_contig % dw == 0 && b_contig % dw == 0 &&
-                     (tail_ok(transA, transB, K, ch) || batch > 1 || ws > 0));
-  const Plan pl = make_plan(dtype_in, M, N, K, batch, mode, ws > 0, ws, cus, fast);
+                    (dwords && dlds && (tail_ok(transA, transB, K, ch) || batch > 1 || ws > 0));
+  const Plan pl = (K == 0 || dwords) && skinny_fits(transA, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
+                      ? skinny_as_plan(skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws))
+                      : make_plan(dtype_in, M, N, K, batch, mode, ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

@@ -725,3 +725,34 @@ def test_unaligned_operands(mi, dev, bf16, pad, tA, tB):
             keep = np.arange(M) != hot
             assert np.array_equal(got[:, keep], ref[:, keep]), (M, N, K, nb, with_ws)
             assert not np.isfinite(got[:, hot]).any(), (M, N, K, nb, with_ws)
+
+
+@pytest.mark.parametrize("bf16", [True, False], ids=["bf16", "f32"])
+@pytest.mark.parametrize("tB", [0, 1], ids=["NN", "NT"])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+def test_few_rows(mi, dev, oracle, bf16, tB, M):
+    """Products of few rows (mi_skinny.hip) at the edges of its 16-row blocks: strips cut by N,
+    K below one step, a K step cut by K, one workgroup's K, K in parts with a workspace, no
+    workspace, the dual product, and the epilogues. Small integers bit for bit."""
+    import torch
+
+    ch = 8 if bf16 else 4
+    ws = torch.full((4 << 20,), float("nan"), dtype=torch.float32, device=dev)
+    for i, (N, K, kw) in enumerate([(64, ch, {}), (130, 5 * ch, dict(bias=True)), (2, 768, dict(residual=True)),
+                                    (66, 2048 + ch, dict(beta=0.5, alpha=2.0, pad=(8, 8, 4))), (1026, 2040, dict(dual=True)),
+                                    (200, 4096, dict(bias=True, residual=True, beta=-1.0)),
+                                    (258, 136, dict(dual=True, pad=(4, 4, 0)))]):
+        for w in (ws, None):
+            plan = mi.describe(0, tB, M, N, K, mi.MI_BF16 if bf16 else mi.MI_F32, epi_mode=int(kw.get("dual", 0)),
+                               workspace_bytes=ws.numel() * 4 if w is not None else 0)
+            assert plan.startswith("skinny"), plan
+            got, ref = _run(mi, dev, oracle, M, N, K, 0, tB, bf16, seed=400 + 10 * i, ws=w, **kw)
+            check(got, ref, _tol(bf16), f"few rows {M}x{N}x{K} NT={tB} {kw} ws={w is not None}")
+    rng = np.random.default_rng(M)
+    for N, K in [(96, 3072), (160, 64)]:
+        a = rng.integers(-4, 5, (M, K)).astype(np.float32)
+        b = rng.integers(-4, 5, (K, N)).astype(np.float32)
+        C = torch.zeros((M, N), dtype=torch.float32, device=dev)
+        for w in (ws, None):
+            mi.gemm(to_dev(a, dev, bf16), to_dev(layout(b, tB), dev, bf16), C, M, N, K, transB=bool(tB), workspace=w)
+            assert np.array_equal(C.cpu().numpy(), a.astype(np.int64) @ b.astype(np.int64)), (N, K)
