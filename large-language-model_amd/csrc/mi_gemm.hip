@@ -218,9 +218,9 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 //     a training step, S also beats L1 on 2048x5632x8192 (931-951 vs 913): the
 //     second workgroup on a CU hides the first one's C read-modify-write, which
 //     L tiles all do at once (in a hot-cache loop L1 leads, 1143 vs 1038);
-//   * when even S tiles leave half the CUs idle, K is split over S tiles, given
-//     a workspace -- also for S tiles chosen by the fill rule and for the
-//     register-staged loader (unaligned operands);
+//   * when even S tiles leave half the CUs idle: W tiles, or given a workspace W tiles
+//     with K split where that pays; for the register-staged loader (unaligned operands) K
+//     is split over S tiles;
 //   * fp32: 64x128 or 64x64 direct-to-LDS tiles with K split to about three
 //     units per CU (16-byte-aligned operands), 128x128 register-staged tiles
 //     split below 5/8 of a wave (element-granular loader); the rules at the fp32
@@ -258,6 +258,24 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
       if (frac > 0.0 && frac <= 0.5 && tilesS >= cus) return plan_for(CFG_S, 1);
       return plan_for(CFG_L, 1);
     }
+    // Grids of S tiles that leave half the CUs idle (a quarter at short K): W tiles, whose two wave groups keep a
+    // lone workgroup's CU busy, split along K only where the shorter loop pays for the
+    // second launch and the partials.  Time in us of a plan: 7.5 + 0.36 per K tile of 64, and
+    // split 4.5 + the partials at 3 TB/s (500 x 768 x 2304 NT: W split 1 / 2 / 3 / 4 17.9 /
+    // 17.0 / 15.8 / 16.8, S split 8 18.9; 2000 x 768 x 2304: W 18.4, W split 2 22.9, S split 2
+    // 26.0; 768 x 2304 x 500 TN: W 11.5, S 11.5, S split 2 20.7; 500 x 2304 x 768: W 11.1, S
+    // split 3 19.4; 1000 x 2304 x 768, 144 tiles: W 11.7, S 13.0).
+    if (fast && (tilesS * 2 < cus || (Ktot < 1024 && tilesS * 4 <= 3 * cus))) {
+      const double kt = (double)cdiv(Ktot, 64);
+      int best = 1;
+      double best_t = 0.36 * kt;
+      for (int sp = 2; allow_split && sp <= std::min<int64_t>(8, cus / tilesS); ++sp) {
+        if (Ktot < 256 * (int64_t)sp || (int64_t)sp * M * N * batch > ws_limit_elems) continue;
+        const double t = 0.36 * kt / sp + 4.5 + 8.0 * (double)(sp * M * N * batch) / 3e6;
+        if (t < best_t) best = sp, best_t = t;
+      }
+      return plan_for(CFG_W, best);
+    }
     // Below one wave of L tiles (long K): one partial round of L tiles or of 256x192
     // tiles (M), 128x128 tiles two 4-wave workgroups per CU (S), or one 8-wave
     // workgroup per CU that splits every K tile between two wave groups (W,
@@ -267,7 +285,9 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
     // 177 (176), W 184, S 189; 5632x2048: M 164, L 172; 2048x3072: S 123, M 130, L
     // 165; 2048x2048: W 69, S 73, M 135, L 153).  M needs N in 64-column blocks.
     if (tilesS * 2 >= cus || !allow_split) {
-      if (fast && !sparse_L && Ktot >= 1024) {
+      // a short K favours the S tiles' small fixed cost while they fit one round (2048 x 2048 x
+      // 1000 TN: S 14.8 us, W 17.2; 2048 x 5632 x 1000, more than one round: S 33.6, M 29.6)
+      if (fast && !sparse_L && (Ktot >= 1024 || tilesS > 2 * cus)) {
         const double cW = (double)cdiv(tilesS, cus);
         const int64_t full2 = tilesS / (2 * cus), rem = tilesS - full2 * 2 * cus;
         const double cS = 1.8 * (double)full2 + (rem > cus ? 1.8 : rem > 0 ? 1.1 : 0.0);
@@ -678,13 +698,15 @@ int run(const Problem& P, hipStream_t stream) {
     return fail(MI_ERR_WORKSPACE, "split-K by %d needs %lld floats of workspace, %lld given",
                 plan.splits, (long long)plan.splits * P.M * P.N * b.batch, (long long)ws_elems);
   const CfgShape ts = shape_of(P.dtype_in, plan.cfg);
-  // the direct epilogue works in whole 32x32 blocks (an edge tile skips those past M, N)
+  // the direct epilogue: whole 32x32 blocks (those past M, N skipped), or cut ones in
+  // quads of columns (epi_kind 3)
+  const bool whole = P.M % 32 == 0 && P.N % 32 == 0;
   const bool fast_epi = plan.splits == 1 && !P.ep.bias && !P.ep.residual && cvec &&
-                        b.causal != MI_CAUSAL_OUT_LOWER && P.M % 32 == 0 && P.N % 32 == 0;
+                        b.causal != MI_CAUSAL_OUT_LOWER && (whole || (P.N % 4 == 0 && !P.ep.row_scale));
   const int64_t kstep = P.dtype_in != MI_BF16 ? 32 : plan.cfg == CFG_W || plan.cfg == CFG_V ? MI_W_BK : 64;
   // with a row scale the direct epilogue has a variant of its own (A K-contiguous on the
   // 256x256, 256x192 and 128x128 tiles); elsewhere the general epilogue applies it
-  int epi_kind = fast_epi ? 1 : 0;
+  int epi_kind = !fast_epi ? 0 : whole ? 1 : 3;
   if (P.ep.row_scale && fast_epi)
     epi_kind = (P.dtype_in == MI_BF16 && fast && !P.transA && P.K % kstep == 0 &&
                 (plan.cfg == CFG_L || plan.cfg == CFG_M || plan.cfg == CFG_S)) ? 2 : 0;

@@ -292,7 +292,7 @@ struct DldsOperand {
 // of a chunk that straddles it in LDS), and the problem takes the direct epilogue (every tile full, epilogue alpha / SiLU
 // gate, beta*C and the output conversion only, no split-K).  One kernel holding
 // both epilogues would need the accumulators in two places at once.
-enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4 };
+enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4, DLDS_EDGE = 8 };
 
 // GEMM of WGM x WGN waves, wave tile (BM/WGM) x (BN/WGN) of 32x32 MFMA blocks: bf16
 // (ES = 2, one 32x32x16 MFMA per block and substep) or fp32 (ES = 4, four 32x32x2).
@@ -312,6 +312,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   // a variant of its own, so that the plain GEMMs carry no row-scale code (+0.45 % on the
   // configuration-3 set, one box)
   constexpr bool ROWSCALE = (VAR & DLDS_ROWSCALE) != 0;
+  // EDGE: M or N is not whole 32x32 blocks, so the direct epilogue guards its rows and quads
+  // of columns; a variant of its own, since the guards cost the whole-block GEMMs 1 %
+  // (configuration-3 set 1903 -> 1924 us)
+  constexpr bool EDGE = (VAR & DLDS_EDGE) != 0;
   constexpr int NWG = WGM * WGN;          // waves of one K group
   constexpr int NWAVE = NWG * KG;         // waves of the workgroup
   constexpr int WTM = BM / WGM, WTN = BN / WGN;
@@ -761,17 +765,20 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
       if constexpr (ROWSCALE) return value(i, j, q, e) * rsv[i];
       else return value(i, j, q, e);
     };
-    // M and N multiples of 32, epilogue alpha (SiLU gate), beta*C and the output
+    // N a multiple of 4, epilogue alpha (SiLU gate), beta*C and the output
     // conversion.  Each 32x32 MFMA block goes through a wave-private LDS patch (rows
     // padded by 4 floats) and back out row-major, so a store instruction writes 8
     // rows of 32 contiguous columns (64 or 128 bytes per row) instead of 32 rows of
-    // 16 bytes.  A block is wholly inside the matrix or wholly past its edge (an
-    // edge tile's extra blocks are skipped).  One barrier first: the patches reuse
-    // the ring's LDS (the barrier is in store_tile, after the first beta loads).
+    // 16 bytes.  Blocks wholly past the edge are skipped; a cut block (EDGE) is stored by
+    // the lanes whose row and columns are inside (the engine's block on 1000 tokens: 465
+    // us with the general epilogue, 453 with this one).  One barrier first: the patches
+    // reuse the ring's LDS (the barrier is in store_tile, after the first beta loads).
     constexpr int PP = 36;  // patch pitch (floats)
     static_assert(NWAVE * 32 * PP * 4 <= LDS_BYTES, "epilogue patches fit the ring");
     float* patch = reinterpret_cast<float*>(smem) + wave * (32 * PP);
     const float beta = p.beta;
+    // whether the quad of columns col of a row is inside a cut block
+    auto in = [&](int row, int col) __attribute__((always_inline)) { return !EDGE || (row < p.M && col < p.N); };
     const int r_in = lane & 31, h_in = lane >> 5;
     const int r_out = lane >> 3, c_out = (lane & 7) * 4;  // + 8 rows per step
     // BF: bf16 C; BETA: beta*C is added.  Both uniform, hoisted out of the tile.
@@ -802,6 +809,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
           if (!inside(j)) continue;
 #pragma unroll
           for (int st = 0; st < 4; ++st) {
+            if (!in((int)row_of(i) + 8 * st, col_of(j))) continue;
             const int64_t ci = (row_of(i) + 8 * st) * p.ldc + col_of(j);
             // non-temporal: the old C is read once (configuration-3 set with its fp32 beta = 1
             // weight gradients 1144-1146 -> 1163-1164 TFLOP/s, one box)
@@ -843,7 +851,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
             for (int st = 0; st < 8; ++st) {
               const f32x4_t v = *reinterpret_cast<const f32x4_t*>(patchw + (rw_out + 4 * st) * PPW + cw_out);
               const int64_t ci = (roww + 4 * st) * p.ldc + colw;
-              if (ok)
+              if (ok && in((int)roww + 4 * st, colw))
                 __builtin_nontemporal_store(u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])},
                                             (u32x2_t*)((uint16_t*)Cz + ci));
             }
@@ -867,6 +875,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
           for (int st = 0; st < 4; ++st) {
             f32x4_t v = *reinterpret_cast<const f32x4_t*>(patch + (r_out + 8 * st) * PP + c_out);
             const int64_t ci = (row0 + 8 * st) * p.ldc + col;
+            if (!in((int)row0 + 8 * st, col)) continue;
             if constexpr (BF) {
               if constexpr (BETA) {
                 const u32x2_t o = old[i & 1][j][st];

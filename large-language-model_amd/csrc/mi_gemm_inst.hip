@@ -137,6 +137,7 @@ KernelFn MI_PICK_NAME(MI_DTN, MI_TA, MI_TB)(int cfg, bool fast, bool ktail, int 
         if (ktail) return dlds_kernel<AK, BK, DLDS_KTAIL>(cfg);
       }
       if (fast_epi == 2) return dlds_kernel<AK, BK, DLDS_FAST_EPI | DLDS_ROWSCALE>(cfg);
+      if (fast_epi == 3) return dlds_kernel<AK, BK, DLDS_FAST_EPI | DLDS_EDGE>(cfg);
       return fast_epi ? dlds_kernel<AK, BK, DLDS_FAST_EPI>(cfg) : dlds_kernel<AK, BK, 0>(cfg);
     }
     switch (cfg) {
@@ -150,6 +151,7 @@ KernelFn MI_PICK_NAME(MI_DTN, MI_TA, MI_TB)(int cfg, bool fast, bool ktail, int 
       if constexpr (AK || BK) {
         if (ktail) return dlds32_kernel<AK, BK, DLDS_KTAIL>(cfg);
       }
+      if (fast_epi == 3) return dlds32_kernel<AK, BK, DLDS_FAST_EPI | DLDS_EDGE>(cfg);
       return fast_epi ? dlds32_kernel<AK, BK, DLDS_FAST_EPI>(cfg) : dlds32_kernel<AK, BK, 0>(cfg);
     }
 #endif

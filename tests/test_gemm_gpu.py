@@ -756,3 +756,34 @@ def test_few_rows(mi, dev, oracle, bf16, tB, M):
         for w in (ws, None):
             mi.gemm(to_dev(a, dev, bf16), to_dev(layout(b, tB), dev, bf16), C, M, N, K, transB=bool(tB), workspace=w)
             assert np.array_equal(C.cpu().numpy(), a.astype(np.int64) @ b.astype(np.int64)), (N, K)
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)], ids=["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("bf16,M,N,K,want", [
+    (True, 4095, 4092, 128, "256x256"), (True, 1530, 8196, 64, "256x256"), (True, 2047, 5632, 1024, "256x192"),
+    (True, 1000, 5632, 1024, "128x192"), (True, 999, 2052, 1088, "128x128"), (True, 65, 68, 192, "128x128"),
+    (True, 2047, 2052, 256, "128x128"), (False, 300, 260, 96, "64x64"), (False, 2047, 772, 64, "64x128")])
+def test_cut_blocks(mi, dev, bf16, M, N, K, want, tA, tB):
+    """The direct epilogue on outputs that are not whole 32x32 blocks (every tile shape): bf16
+    and fp32 C, with and without beta, NaN in the gaps between C's rows and after its
+    last, which must stay. Integer products, bit for bit in fp32."""
+    import torch
+
+    plan = mi.describe(tA, tB, M, N, K, mi.MI_BF16 if bf16 else mi.MI_F32)
+    assert want in plan or tA or tB, plan
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    a = torch.randint(-2, 3, (M, K), generator=g, device=dev)
+    b = torch.randint(-2, 3, (K, N), generator=g, device=dev)
+    ref = a.double() @ b.double()
+    A = (a.T if tA else a).contiguous().to(dt)
+    B = (b.T if tB else b).contiguous().to(dt)
+    for cdt in (torch.float32, torch.bfloat16):
+        for beta in (0.0, 2.0):
+            buf = torch.full((M + 1, N + 12), float("nan"), dtype=cdt, device=dev)
+            C = buf[:M, :N]
+            C.fill_(3.0)
+            mi.gemm(A, B, C, M, N, K, transA=tA, transB=tB, beta=beta, ldc=N + 12)
+            want_c = (ref + 3.0 * beta).to(cdt)
+            assert torch.equal(C, want_c), (cdt, beta, (C.double() - want_c.double()).abs().max().item())
+            assert buf[M].isnan().all() and buf[:M, N:].isnan().all()
