@@ -232,7 +232,22 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
     const CfgShape s = shape_of(dtype_in, cfg);
     return Plan{cfg, sp, (int)cdiv(M, s.bm), (int)cdiv(N, s.bn)};
   };
-  if (mode == MODE_DUAL) return plan_for(CFG_DUAL, 1);
+  if (mode == MODE_DUAL) {
+    // The cost model of the plain tiles below (units of one W tile per round) on tiles of the
+    // same area; 192x128 tiles (M, 2.08) stand where the plain products have 256x192.  us, K
+    // 2048 to N = 5632: M = 2048 L 101 M 84-91 S 99 W 109 (four waves of 128x64 of each on a
+    // K tile of 32: 124), 8192 L 315 M 322, 1000 L 48 S 56 M 75, 500 S 34 M 37, 100 W 20 S 28.
+    if (!fast) return plan_for(CFG_DUAL, 1);
+    if (dtype_in != MI_BF16) return plan_for(CFG_DUAL_S, 1);
+    const int64_t tL = cdiv(M, 256) * cdiv(N, 128) * batch, tS = cdiv(M, 128) * cdiv(N, 64) * batch;
+    const int64_t full2 = tS / (2 * cus), rem = tS - full2 * 2 * cus;
+    const double cL = 2.6 * (double)cdiv(tL, cus), cW = (double)cdiv(tS, cus);
+    const double cS = 1.8 * (double)full2 + (rem > cus ? 1.8 : rem > 0 ? 1.1 : 0.0);
+    const double cM = 2.08 * (double)cdiv(cdiv(M, 192) * cdiv(N, 128) * batch, cus);
+    if (cM < cL && cM <= cW && cM <= cS) return plan_for(CFG_DUAL_M, 1);
+    if (cL <= cW && cL <= cS) return plan_for(CFG_DUAL, 1);
+    return plan_for(cW < cS ? CFG_DUAL_W : CFG_DUAL_S, 1);
+  }
   if (mode == MODE_PROLOGUE) return plan_for(CFG_PRO, 1);
   const CfgShape L = shape_of(dtype_in, CFG_L), S = shape_of(dtype_in, CFG_S);
   const int64_t tilesL = cdiv(M, L.bm) * cdiv(N, L.bn) * batch;
@@ -381,9 +396,10 @@ void describe_plan(char* buf, size_t len, int dtype_in, bool fast, const Plan& p
   }
   const CfgShape sh = shape_of(dtype_in, pl.cfg);
   const char* kind = (dtype_in == MI_BF16 && fast && pl.cfg != CFG_PRO)
-                         ? (pl.cfg == CFG_W || pl.cfg == CFG_V ? "dlds-kg2" : "dlds")
-                     : (dtype_in != MI_BF16 && fast && (pl.cfg == CFG_V || pl.cfg == CFG_M)) ? "dlds"
-                                                                                           : "regstage";
+                         ? (pl.cfg == CFG_W || pl.cfg == CFG_V || pl.cfg == CFG_DUAL_W ? "dlds-kg2" : "dlds")
+                     : (dtype_in != MI_BF16 && fast && (pl.cfg == CFG_V || pl.cfg == CFG_M || pl.cfg == CFG_DUAL_S))
+                         ? "dlds"
+                         : "regstage";
   std::snprintf(buf, len, "%s %s %dx%d %s%s split%d tiles%lld", kind,
                 dtype_in == MI_BF16 ? "bf16" : "f32", sh.bm, sh.bn, transA ? "T" : "N",
                 transB ? "T" : "N", pl.splits, (long long)pl.tiles_m * pl.tiles_n * batch);
@@ -629,8 +645,7 @@ int run(const Problem& P, hipStream_t stream) {
   };
   const bool spanA = extA < lim && span_ok(!P.transA, a_rows, P.lda);
   const bool spanB = extB < lim && span_ok(P.transB != 0, b_rows, P.ldb);
-  // The skinny and the direct-to-LDS kernels (every bf16 mode but the prologue, plain fp32)
-  // need no more than 4-byte alignment: a buffer load's address and its bounds check work in
+  // The skinny and the direct-to-LDS kernels (every mode but the prologue) need no more than 4-byte alignment: a buffer load's address and its bounds check work in
   // dwords.  A row-contiguous chunk that straddles the matrix edge feeds outputs that are
   // not stored; a K-contiguous one is zeroed past K in LDS (tail_ok).
   auto dw = [&](const void* q, int64_t ld, int64_t o, int64_t i, int64_t sg) {
@@ -638,7 +653,7 @@ int run(const Problem& P, hipStream_t stream) {
   };
   const bool dwords = spanA && spanB && dw(P.A, P.lda, b.a_outer, b.a_inner, b.seg_a) &&
                       dw(P.B, P.ldb, b.b_outer, b.b_inner, b.seg_b) && (!P.ep.B2 || ((uintptr_t)P.ep.B2 & 3u) == 0);
-  const bool dlds = P.dtype_in == MI_BF16 ? mode != MODE_PROLOGUE : mode == MODE_PLAIN;
+  const bool dlds = mode != MODE_PROLOGUE;
   const bool fast = (vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB) ||
                     (dwords && dlds &&
                      (tail_ok(P.transA, P.transB, P.K, CH) || b.batch > 1 || (P.ws && P.ws_bytes > 0)));
@@ -703,7 +718,7 @@ int run(const Problem& P, hipStream_t stream) {
   const bool whole = P.M % 32 == 0 && P.N % 32 == 0;
   const bool fast_epi = plan.splits == 1 && !P.ep.bias && !P.ep.residual && cvec &&
                         b.causal != MI_CAUSAL_OUT_LOWER && (whole || (P.N % 4 == 0 && !P.ep.row_scale));
-  const int64_t kstep = P.dtype_in != MI_BF16 ? 32 : plan.cfg == CFG_W || plan.cfg == CFG_V ? MI_W_BK : 64;
+  const int64_t kstep = P.dtype_in != MI_BF16 ? 32 : plan.cfg == CFG_W || plan.cfg == CFG_V || plan.cfg == CFG_DUAL_W ? MI_W_BK : 64;
   // with a row scale the direct epilogue has a variant of its own (A K-contiguous on the
   // 256x256, 256x192 and 128x128 tiles); elsewhere the general epilogue applies it
   int epi_kind = !fast_epi ? 0 : whole ? 1 : 3;
@@ -1637,7 +1652,7 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   // whole dwords
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
-  const bool dlds = dtype_in == MI_BF16 ? mode != MODE_PROLOGUE : mode == MODE_PLAIN;
+  const bool dlds = mode != MODE_PROLOGUE;
   const int64_t dw = dtype_in == MI_BF16 ? 2 : 1;
   const bool dwords = a_contig % dw == 0 && b_contig % dw == 0;
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) ||

@@ -81,8 +81,8 @@ __device__ __forceinline__ int mc_unswz(int kr, int p) {
 // 256-byte bank window.  Self-inverse.
 __device__ __forceinline__ int mc_swz32(int kr, int q) { return q ^ (((kr >> 2) & 1) << 3); }
 
-// Row-contiguous tiles whose row is not a power of two (192 columns) are stored
-// in 128-byte granules, column block by column block: granule G holds k-row
+// Row-contiguous tiles whose row is not a power of two (192 columns), or is a single
+// granule (64 columns of bf16), are stored in 128-byte granules, column block by column block: granule G holds k-row
 // G % BK of the 64-column block G / BK, so consecutive k-rows of one column block
 // are 128 bytes apart and any four of them cover both halves of a 256-byte bank
 // window; the two 64-byte halves of a granule swap on k-rows 2 and 3 (mod 4), so
@@ -128,7 +128,7 @@ struct DldsOperand {
   static constexpr int EPC = 16 / ES;                 // elements per 16-byte chunk
   static constexpr int NCH = BK / EPC;                // KC: 16-byte chunks per row
   static constexpr int CPR = R / EPC;                 // !KC: 16-byte chunks per k-row
-  static constexpr bool GRAN = !KC && (CPR & (CPR - 1)) != 0;  // 128-byte granule layout
+  static constexpr bool GRAN = !KC && ((CPR & (CPR - 1)) != 0 || CPR < 16);  // 128-byte granule layout
   static constexpr int KRB = GRAN ? 128 : R * ES;     // !KC: LDS bytes between k-rows
   static_assert(!GRAN || R % 64 == 0, "granule layout needs 64-column blocks");
   static_assert(ES == 2 || (!GRAN && (KC || CPR >= 16)), "fp32 k-rows: 2^n >= 16 chunks");
@@ -326,10 +326,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   constexpr int NSUB = NSUBT / KG;        // K substeps one wave computes per stage
   static_assert(MODE != MODE_PROLOGUE, "the SiLU-gate prologue needs register staging");
   static_assert(KG == 1 || KG == 2, "one or two K groups");
-  static_assert(KG == 1 || (MODE == MODE_PLAIN && TM == 2), "split-K groups: plain mode, two row blocks");
+  static_assert(KG == 1 || TM == 2, "split-K groups: two row blocks");
   static_assert(NSUB == 2 || NSUB == 4, "each wave computes 2 or 4 substeps per stage");
   static_assert(STAGES >= 2 && STAGES <= 4, "2..4 stages");
-  static_assert(ES == 2 || (ES == 4 && !DUAL), "bf16, or fp32 without the dual B");
+  static_assert(ES == 2 || ES == 4, "bf16 or fp32");
   // TRR: fragments of a row-contiguous bf16 operand come from transpose reads issued
   // as inline asm, whose completion the code waits for itself
   constexpr bool TRR = ES == 2 && (!AK || !BKC);
@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   ob.init_dma(p.ldb, p.N, n0, p.K);
   oa.init_lds(lds0 + A_REG, wm * WTM, wave_u, kg * NSUB);
   ob.init_lds(lds0 + B_REG, wn * WTN, wave_u, kg * NSUB);
-  if constexpr (DUAL) ob2.init_lds(lds0 + B2_REG, wn * WTN, wave_u);
+  if constexpr (DUAL) ob2.init_lds(lds0 + B2_REG, wn * WTN, wave_u, kg * NSUB);
 
   // Tile stream of the DMA.  Descriptors start at the tile (base + K offset,
   // extent reduced by the same amount) and step by one K tile; crossing into
@@ -717,10 +717,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     // group) through LDS, in slots [sender group][wave][j][quad][lane] of 16
     // bytes; the epilogue below then stores only row block kg.
     __syncthreads();  // every wave is past its last fragment read
-    static_assert(2 * NWG * TN * 4 * 64 * 16 <= LDS_BYTES, "exchange fits the ring");
+    static_assert(2 * NWG * NB * 4 * 64 * 16 <= LDS_BYTES, "exchange fits the ring");
     f32x4_t* xb = reinterpret_cast<f32x4_t*>(smem);
     auto slot = [&](int g, int j, int q) __attribute__((always_inline)) {
-      return (((g * NWG + wq) * TN + j) * 4 + q) * 64 + lane;
+      return (((g * NWG + wq) * NB + j) * 4 + q) * 64 + lane;
     };
     auto quad = [](const f32x16_t& a, int q) __attribute__((always_inline)) {
       return f32x4_t{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
@@ -728,12 +728,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     auto exchange = [&](auto KEEP_c) __attribute__((always_inline)) {
       constexpr int KEEP = decltype(KEEP_c)::value, SEND = 1 - KEEP;
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) xb[slot(KEEP, j, q)] = quad(acc[SEND][j], q);
       __syncthreads();
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const f32x4_t r = xb[slot(SEND, j, q)];

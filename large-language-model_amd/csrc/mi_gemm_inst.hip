@@ -19,7 +19,7 @@ typedef float elem_t;
 #endif
 // ktail: the K extent of a segment is not a multiple of 64 (bf16 direct-to-LDS
 // kernels then mask K-contiguous chunks past the end); fast_epi: the problem
-// qualifies for the direct epilogue.  Both are ignored for fp32.
+// qualifies for the direct epilogue.
 
 #ifndef MI_DLDS_BK
 #define MI_DLDS_BK 64
@@ -66,8 +66,8 @@ typedef float elem_t;
 
 #if MI_DT_BF16
 // bf16 direct-to-LDS kernels of one variant (K tile and LDS ring depth:
-// MI_DLDS_BK / MI_DLDS_STAGES for 256x256, MI_S_BK / MI_S_STAGES of the A layout for 128x128,
-// 32 / 4 for the dual-B 256x128).  256x256 runs 8 waves (2 x 4, wave tiles 128x64): two
+// MI_DLDS_BK / MI_DLDS_STAGES for 256x256, MI_S_BK / MI_S_STAGES of the A layout for 128x128;
+// the dual-B tiles are the plain ones with B's columns shared by the two matrices).  256x256 runs 8 waves (2 x 4, wave tiles 128x64): two
 // waves per SIMD, so one wave's MFMAs issue while the other waits on LDS or DMA issue
 // (8192x2048x5632 NT: 147 vs 161 us with 4 waves of 128x128; 8192x5632x2048 NN 157 vs
 // 166; 2048x5632x8192 TN 170 vs 180; bit-identical results).
@@ -92,7 +92,12 @@ KernelFn dlds_kernel(int cfg) {
     case CFG_L:
       return gemm_dlds_kernel<256, 256, MI_L_BK(AK, BK), MI_L_STAGES(AK, BK), AK, BK, MODE_PLAIN, V, 2, 4, 1>;
     case CFG_S: return gemm_dlds_kernel<128, 128, MI_S_BK(AK), MI_S_STAGES(AK), AK, BK, MODE_PLAIN, V>;
-    case CFG_DUAL: return gemm_dlds_kernel<256, 128, 32, 4, AK, BK, MODE_DUAL, V>;
+    case CFG_DUAL:
+      return gemm_dlds_kernel<256, 128, MI_L_BK(AK, BK), MI_L_STAGES(AK, BK), AK, BK, MODE_DUAL, V, 2, 4, 1>;
+    case CFG_DUAL_M:
+      return gemm_dlds_kernel<192, 128, MI_L_BK(AK, BK), MI_L_STAGES(AK, BK), AK, BK, MODE_DUAL, V, 2, 4, 1>;
+    case CFG_DUAL_S: return gemm_dlds_kernel<128, 64, MI_S_BK(AK), MI_S_STAGES(AK), AK, BK, MODE_DUAL, V>;
+    case CFG_DUAL_W: return gemm_dlds_kernel<128, 64, MI_W_BK, MI_W_STAGES, AK, BK, MODE_DUAL, V, 2, 2, 2>;
     case CFG_W:
       return gemm_dlds_kernel<128, 128, MI_W_BK, MI_W_STAGES, AK, BK, MODE_PLAIN, V, 2, 2, 2>;
     case CFG_M:
@@ -115,6 +120,7 @@ KernelFn dlds32_kernel(int cfg) {
   switch (cfg) {
     case CFG_V: return gemm_dlds_kernel<64, 128, 32, 2, AK, BK, MODE_PLAIN, V, 2, 2, 1, 4>;
     case CFG_M: return gemm_dlds_kernel<64, 64, 32, 2, AK, BK, MODE_PLAIN, V, 2, 2, 1, 4>;
+    case CFG_DUAL_S: return gemm_dlds_kernel<64, 64, 32, 2, AK, BK, MODE_DUAL, V, 2, 2, 1, 4>;
     default: return nullptr;
   }
 }
@@ -124,45 +130,31 @@ KernelFn MI_PICK_NAME(MI_DTN, MI_TA, MI_TB)(int cfg, bool fast, bool ktail, int 
   constexpr bool AK = (MI_TA == 0);  // A is K-contiguous when not transposed
   constexpr bool BK = (MI_TB == 1);  // B is K-contiguous when transposed
 #if MI_DT_BF16
-  constexpr int LM = 256, LN = 256, SM = 128, SN = 128, DM = 256, DN = 128, PM = 256, PN = 256;
+  constexpr int SM = 128, SN = 128, DM = 256, DN = 128, PM = 256, PN = 256;
 #else
-  constexpr int LM = 128, LN = 128, SM = 128, SN = 128, DM = 128, DN = 64, PM = 128, PN = 128;
+  constexpr int SM = 128, SN = 128, DM = 128, DN = 64, PM = 128, PN = 128;
 #endif
   if (fast) {
+    if (cfg == CFG_PRO) {
+      if constexpr (AK) return gemm_kernel<elem_t, PM, PN, 2, 2, AK, BK, MODE_PROLOGUE, true>;
+      return nullptr;
+    }
 #if MI_DT_BF16
-    if (cfg != CFG_PRO) {
-      // K-tail variants exist only where an operand is K-contiguous; a K tail
-      // takes the general epilogue.
-      if constexpr (AK || BK) {
-        if (ktail) return dlds_kernel<AK, BK, DLDS_KTAIL>(cfg);
-      }
-      if (fast_epi == 2) return dlds_kernel<AK, BK, DLDS_FAST_EPI | DLDS_ROWSCALE>(cfg);
-      if (fast_epi == 3) return dlds_kernel<AK, BK, DLDS_FAST_EPI | DLDS_EDGE>(cfg);
-      return fast_epi ? dlds_kernel<AK, BK, DLDS_FAST_EPI>(cfg) : dlds_kernel<AK, BK, 0>(cfg);
-    }
-    switch (cfg) {
-      case CFG_PRO:
-        if constexpr (AK) return gemm_kernel<elem_t, PM, PN, 2, 2, AK, BK, MODE_PROLOGUE, true>;
-        return nullptr;
-    }
+#define MI_DLDS(V) dlds_kernel<AK, BK, V>(cfg)
+#else
+#define MI_DLDS(V) dlds32_kernel<AK, BK, V>(cfg)
 #endif
-#if !MI_DT_BF16
-    if (cfg == CFG_V || cfg == CFG_M) {
-      if constexpr (AK || BK) {
-        if (ktail) return dlds32_kernel<AK, BK, DLDS_KTAIL>(cfg);
-      }
-      if (fast_epi == 3) return dlds32_kernel<AK, BK, DLDS_FAST_EPI | DLDS_EDGE>(cfg);
-      return fast_epi ? dlds32_kernel<AK, BK, DLDS_FAST_EPI>(cfg) : dlds32_kernel<AK, BK, 0>(cfg);
+    // K-tail variants exist only where an operand is K-contiguous; a K tail
+    // takes the general epilogue.
+    if constexpr (AK || BK) {
+      if (ktail) return MI_DLDS(DLDS_KTAIL);
     }
+#if MI_DT_BF16
+    if (fast_epi == 2) return MI_DLDS(DLDS_FAST_EPI | DLDS_ROWSCALE);
 #endif
-    switch (cfg) {
-      case CFG_L: return gemm_kernel<elem_t, LM, LN, 2, 2, AK, BK, MODE_PLAIN, true>;
-      case CFG_S: return gemm_kernel<elem_t, SM, SN, 2, 2, AK, BK, MODE_PLAIN, true>;
-      case CFG_DUAL: return gemm_kernel<elem_t, DM, DN, 2, 2, AK, BK, MODE_DUAL, true>;
-      case CFG_PRO:
-        if constexpr (AK) return gemm_kernel<elem_t, PM, PN, 2, 2, AK, BK, MODE_PROLOGUE, true>;
-        return nullptr;
-    }
+    if (fast_epi == 3) return MI_DLDS(DLDS_FAST_EPI | DLDS_EDGE);
+    return fast_epi ? MI_DLDS(DLDS_FAST_EPI) : MI_DLDS(0);
+#undef MI_DLDS
   } else {
     switch (cfg) {
       case CFG_S: return gemm_kernel<elem_t, SM, SN, 2, 2, AK, BK, MODE_PLAIN, false>;

@@ -787,3 +787,28 @@ def test_cut_blocks(mi, dev, bf16, M, N, K, want, tA, tB):
             want_c = (ref + 3.0 * beta).to(cdt)
             assert torch.equal(C, want_c), (cdt, beta, (C.double() - want_c.double()).abs().max().item())
             assert buf[M].isnan().all() and buf[:M, N:].isnan().all()
+
+
+@pytest.mark.parametrize("tB", [0, 1], ids=["NN", "NT"])
+@pytest.mark.parametrize("bf16,M,N,K,want", [
+    (True, 1000, 5632, 256, "256x128"), (True, 2048, 5632, 128, "192x128"), (True, 1345, 3076, 328, "192x128"),
+    (True, 500, 5632, 192, "128x64"), (True, 130, 2052, 520, "dlds-kg2"), (False, 155, 772, 100, "dlds f32 64x64"),
+    (False, 700, 1024, 64, "dlds f32 64x64"), (False, 70, 66, 37, "")])
+def test_dual_tiles(mi, dev, bf16, M, N, K, want, tB):
+    """C = SiLU(A Bg) (.) (A Bu) on every dual tile, whole and cut, with a K tail, in the direct
+    and the general epilogue (bias + residual), against float64."""
+    import torch
+
+    dt = torch.bfloat16 if bf16 else torch.float32
+    assert want in mi.describe(0, tB, M, N, K, mi.MI_BF16 if bf16 else mi.MI_F32, epi_mode=1)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    mk = lambda *s, std=1.0: (torch.randn(*s, generator=g, device=dev) * std).to(dt)  # noqa: E731
+    A, Bg, Bu = mk(M, K), mk(K, N, std=K ** -0.5), mk(K, N, std=K ** -0.5)
+    bias, R = mk(N), mk(M, N)
+    ref = torch.nn.functional.silu(A.double() @ Bg.double()) * (A.double() @ Bu.double())
+    st = (lambda b: b.T.contiguous()) if tB else (lambda b: b)
+    C = torch.full((M, N), float("nan"), dtype=dt, device=dev)
+    mi.gemm(A, st(Bg), C, M, N, K, transB=bool(tB), B2=st(Bu))
+    check(host(C), host(ref), _tol(bf16), f"dual {M}x{N}x{K}")
+    mi.gemm(A, st(Bg), C, M, N, K, transB=bool(tB), B2=st(Bu), bias=bias, residual=R)
+    check(host(C), host(ref + bias.double() + R.double()), _tol(bf16), f"dual {M}x{N}x{K} bias residual")
