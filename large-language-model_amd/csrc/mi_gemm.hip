@@ -245,7 +245,7 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
     const double cS = 1.8 * (double)full2 + (rem > cus ? 1.8 : rem > 0 ? 1.1 : 0.0);
     const double cM = 2.08 * (double)cdiv(cdiv(M, 192) * cdiv(N, 128) * batch, cus);
     if (cM < cL && cM <= cW && cM <= cS) return plan_for(CFG_DUAL_M, 1);
-    if (cL <= cW && cL <= cS) return plan_for(CFG_DUAL, 1);
+    if (cL <= cW && cL <= cS) return plan_for(CFG_DUAL_L, 1);
     return plan_for(cW < cS ? CFG_DUAL_W : CFG_DUAL_S, 1);
   }
   if (mode == MODE_PROLOGUE) return plan_for(CFG_PRO, 1);

@@ -92,7 +92,7 @@ KernelFn dlds_kernel(int cfg) {
     case CFG_L:
       return gemm_dlds_kernel<256, 256, MI_L_BK(AK, BK), MI_L_STAGES(AK, BK), AK, BK, MODE_PLAIN, V, 2, 4, 1>;
     case CFG_S: return gemm_dlds_kernel<128, 128, MI_S_BK(AK), MI_S_STAGES(AK), AK, BK, MODE_PLAIN, V>;
-    case CFG_DUAL:
+    case CFG_DUAL_L:
       return gemm_dlds_kernel<256, 128, MI_L_BK(AK, BK), MI_L_STAGES(AK, BK), AK, BK, MODE_DUAL, V, 2, 4, 1>;
     case CFG_DUAL_M:
       return gemm_dlds_kernel<192, 128, MI_L_BK(AK, BK), MI_L_STAGES(AK, BK), AK, BK, MODE_DUAL, V, 2, 4, 1>;

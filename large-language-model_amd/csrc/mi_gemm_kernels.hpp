@@ -10,10 +10,10 @@ typedef void (*KernelFn)(Params);
 
 // Tile configurations.  Output tile (BM x BN) per configuration and dtype:
 //   bf16: L 256x256 (8 waves of 128x64, two per SIMD), S 128x128 (4 waves of 64x64),
-//         DUAL 256x128 of each B (L's waves and LDS with two B tiles of half the width),
+//         DUAL_L 256x128 of each B (L's waves and LDS with two B tiles of half the width),
 //         DUAL_M 192x128 of each (8 waves of 96x32 of each), DUAL_S and DUAL_W 128x64 of
-//         each (S and W likewise), PRO 256x256 with the SiLU-gate A prologue,
-//         W 128x128 with wave-level split-K (8 waves: two groups of 4 waves of
+//         each (S and W likewise), DUAL 256x128 of each register-staged, PRO 256x256 with
+//         the SiLU-gate A prologue, W 128x128 with wave-level split-K (8 waves: two groups of 4 waves of
 //         64x64, each over half of every K tile, summed through LDS),
 //         M 256x192 (8 waves of 64x96), V 128x192 with wave-level split-K (two
 //         groups of 4 waves of 64x96).
@@ -21,7 +21,7 @@ typedef void (*KernelFn)(Params);
 //   fp32: V 64x128, M 64x64 and DUAL_S 64x64 of each B direct-to-LDS (four waves);
 //         register-staged L = S = W 128x128, DUAL 128x64, PRO 128x128.
 enum Cfg { CFG_L = 0, CFG_S = 1, CFG_DUAL = 2, CFG_PRO = 3, CFG_W = 4, CFG_M = 5, CFG_V = 6, CFG_SKINNY = 7, CFG_DUAL_S = 8,
-           CFG_DUAL_W = 9, CFG_DUAL_M = 10 };
+           CFG_DUAL_W = 9, CFG_DUAL_M = 10, CFG_DUAL_L = 11 };
 
 struct CfgShape {
   int bm, bn;
@@ -41,7 +41,8 @@ inline CfgShape cfg_shape(bool bf16, int cfg) {
          : cfg == CFG_W ? CfgShape{128, 128, 512}
          : cfg == CFG_M ? CfgShape{256, 192, 512}
          : cfg == CFG_V ? CfgShape{128, 192, 512}
-         : cfg == CFG_DUAL ? CfgShape{256, 128, 512}
+         : cfg == CFG_DUAL ? CfgShape{256, 128}
+         : cfg == CFG_DUAL_L ? CfgShape{256, 128, 512}
          : cfg == CFG_DUAL_M ? CfgShape{192, 128, 512}
          : cfg == CFG_DUAL_S ? CfgShape{128, 64}
          : cfg == CFG_DUAL_W ? CfgShape{128, 64, 512}

@@ -793,7 +793,7 @@ def test_cut_blocks(mi, dev, bf16, M, N, K, want, tA, tB):
 @pytest.mark.parametrize("bf16,M,N,K,want", [
     (True, 1000, 5632, 256, "256x128"), (True, 2048, 5632, 128, "192x128"), (True, 1345, 3076, 328, "192x128"),
     (True, 500, 5632, 192, "128x64"), (True, 130, 2052, 520, "dlds-kg2"), (False, 155, 772, 100, "dlds f32 64x64"),
-    (False, 700, 1024, 64, "dlds f32 64x64"), (False, 70, 66, 37, "")])
+    (False, 700, 1024, 64, "dlds f32 64x64"), (False, 70, 66, 37, ""), (True, 257, 259, 65, "regstage")])
 def test_dual_tiles(mi, dev, bf16, M, N, K, want, tB):
     """C = SiLU(A Bg) (.) (A Bu) on every dual tile, whole and cut, with a K tail, in the direct
     and the general epilogue (bias + residual), against float64."""
