@@ -226,7 +226,8 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 //     split below 5/8 of a wave (element-granular loader); the rules at the fp32
 //     branch.
 // Every split fits the workspace: splits * M * N * batch <= ws_limit_elems.
-Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, int mode,
+// nt: B is K-contiguous and A too (transB without transA).
+Plan make_plan(int dtype_in, bool nt, int64_t M, int64_t N, int64_t Ktot, int64_t batch, int mode,
                bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
   auto plan_for = [&](int cfg, int sp) {
     const CfgShape s = shape_of(dtype_in, cfg);
@@ -334,15 +335,23 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
   // qkv dW 768x2304x2048 64x64 113 vs 64x128 102; o forward 2048x768x768 64x128 93 vs
   // 64x64 87; gate forward 2048x2048x768 64x128 127 vs 64x64 122.  The rule picks the
   // best plan of every one of the 12, or one within 2 %.
+  // The score of an NN or TN plan is its time in us: the busiest CU's MFMAs at 2.1 GHz, and
+  // split 4 us for the second launch and the partials at 3 TB/s, which the share alone
+  // leaves out (768 x 768 x 512 TN: 64x64 12.4, 64x128 split 3 17.9; 512 x 768 x 768 NN: 15.9,
+  // 64x128 split 5 18.5; 200 x 2304 x 768 NN: 16.9, 64x128 split 3 19.0).  NT keeps the
+  // share: its small plans are in the pinned planner table.
+  // Batched products (the attention's, short K or causally cut) take 64x64 tiles:
+  // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304.
   // The element-granular loader (any alignment) runs 128x128 tiles (S): below 5/8
   // of a wave, K is split by the same score with units at most two per CU and each
   // split keeping >= 8 K tiles of 32, or >= 4 when the units fit one per CU (96
   // tiles at K = 2048: splits 1..8 ran 43 71 59 74 83 66 69 76 TFLOP/s; 108 tiles:
   // 47 78 67 83 65 73 76 71; 36 tiles: 16 28 37 44 49 52 54 41).
   if (fast) {
-    int best_cfg = CFG_V, best_sp = 1;
+    int best_cfg = CFG_M, best_sp = 1;
     double best_score = 1e300;
     for (int cfg : {CFG_V, CFG_M}) {
+      if (cfg == CFG_V && batch > 1) continue;
       const CfgShape t = shape_of(dtype_in, cfg);
       const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
       for (int sp = 1; sp <= (allow_split ? 8 : 1); ++sp) {
@@ -351,7 +360,11 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
           if (units > 3 * (int64_t)cus || (int64_t)sp * M * N * batch > ws_limit_elems) continue;
           if (Ktot < (units > cus ? 512 : 128) * (int64_t)sp) continue;
         }
-        const double score = (double)cdiv(units, cus) * t.bm * t.bn / sp;
+        double score = (double)cdiv(units, cus) * t.bm * t.bn / sp;
+        if (!nt) {
+          score *= (double)Ktot / (128 * 2100.0);
+          if (sp > 1) score += 4.0 + 8.0 * (double)(sp * M * N * batch) / 3e6;
+        }
         const bool wins = score < best_score ||
                           (score == best_score &&
                            (sp < best_sp || (sp == best_sp && cfg == (Ktot < 1024 ? CFG_V : CFG_M))));
@@ -377,12 +390,14 @@ Plan make_plan(int dtype_in, int64_t M, int64_t N, int64_t Ktot, int64_t batch, 
 // Products of few rows with op(A) not transposed, in whole 16-byte chunks of K: the kernels
 // of mi_skinny.hip, which read B once at the rate HBM gives (a layer's products on 8 rows:
 // 128-row tiles split along K spent 99 us of which 45 in the dual product's 44 workgroups).
-bool skinny_fits(int transA, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t segs, int causal, int mode,
-                 int64_t ch) {
-  return !transA && M <= SKINNY_MAX_M && (M <= 32 || N * K * (16 / ch) <= SKINNY_WIDE_BYTES) && K % ch == 0 &&
-         batch == 1 && segs == 1 && causal == MI_CAUSAL_NONE && mode != MODE_PROLOGUE;
+bool skinny_fits(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t segs, int causal,
+                 int mode, int64_t ch) {
+  if (transA || K % ch != 0 || batch != 1 || segs != 1 || causal != MI_CAUSAL_NONE || mode == MODE_PROLOGUE) return false;
+  if (M <= 32) return true;
+  if (M <= SKINNY_MAX_M) return N * K * (16 / ch) <= SKINNY_WIDE_BYTES;
+  return skinny_blocks_fit(ch == 8, transB != 0, mode == MODE_DUAL, M, N, K);
 }
-Plan skinny_as_plan(const SkinnyPlan& sk) { return Plan{CFG_SKINNY, sk.splits, 1, sk.strips}; }
+Plan skinny_as_plan(const SkinnyPlan& sk) { return Plan{CFG_SKINNY, sk.splits, sk.blocks, sk.strips}; }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -391,7 +406,7 @@ void describe_plan(char* buf, size_t len, int dtype_in, bool fast, const Plan& p
                    int transB, int64_t batch) {
   if (pl.cfg == CFG_SKINNY) {
     std::snprintf(buf, len, "skinny %s N%s split%d strips%d", dtype_in == MI_BF16 ? "bf16" : "f32",
-                  transB ? "T" : "N", pl.splits, pl.tiles_n);
+                  transB ? "T" : "N", pl.splits, pl.tiles_m * pl.tiles_n);
     return;
   }
   const CfgShape sh = shape_of(dtype_in, pl.cfg);
@@ -657,7 +672,7 @@ int run(const Problem& P, hipStream_t stream) {
   const bool fast = (vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB) ||
                     (dwords && dlds &&
                      (tail_ok(P.transA, P.transB, P.K, CH) || b.batch > 1 || (P.ws && P.ws_bytes > 0)));
-  const bool skinny = dwords && skinny_fits(P.transA, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode, CH);
+  const bool skinny = dwords && skinny_fits(P.transA, P.transB, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode, CH);
 
   // SiLU-gate prologue as its own pass when the workspace holds SiLU(A) * A2 (bf16,
   // one matrix, 16-byte rows): the activation is written once and the GEMM runs
@@ -699,7 +714,7 @@ int run(const Problem& P, hipStream_t stream) {
   const SkinnyPlan sk = skinny_plan(P.dtype_in == MI_BF16, P.transB != 0, mode == MODE_DUAL, P.M, P.N, P.K,
                                     allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0);
   Plan plan = skinny ? skinny_as_plan(sk)
-                     : make_plan(P.dtype_in, P.M, P.N, Ktot, b.batch, mode, allow_split || P.noalloc,
+                     : make_plan(P.dtype_in, !P.transA && P.transB, P.M, P.N, Ktot, b.batch, mode, allow_split || P.noalloc,
                                  P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
   if (P.noalloc && plan.splits > 1 && (int64_t)plan.splits * P.M * P.N * b.batch > ws_elems)
     return fail(MI_ERR_WORKSPACE,
@@ -713,15 +728,16 @@ int run(const Problem& P, hipStream_t stream) {
     return fail(MI_ERR_WORKSPACE, "split-K by %d needs %lld floats of workspace, %lld given",
                 plan.splits, (long long)plan.splits * P.M * P.N * b.batch, (long long)ws_elems);
   const CfgShape ts = shape_of(P.dtype_in, plan.cfg);
-  // the direct epilogue: whole 32x32 blocks (those past M, N skipped), or cut ones in
-  // quads of columns (epi_kind 3)
+  // the direct epilogue: whole 32x32 blocks (those past M, N skipped), or cut or causally
+  // masked ones in quads of columns (epi_kind 3)
   const bool whole = P.M % 32 == 0 && P.N % 32 == 0;
+  const bool masked = b.causal == MI_CAUSAL_OUT_LOWER;
   const bool fast_epi = plan.splits == 1 && !P.ep.bias && !P.ep.residual && cvec &&
-                        b.causal != MI_CAUSAL_OUT_LOWER && (whole || (P.N % 4 == 0 && !P.ep.row_scale));
+                        ((whole && !masked) || (P.N % 4 == 0 && !P.ep.row_scale));
   const int64_t kstep = P.dtype_in != MI_BF16 ? 32 : plan.cfg == CFG_W || plan.cfg == CFG_V || plan.cfg == CFG_DUAL_W ? MI_W_BK : 64;
   // with a row scale the direct epilogue has a variant of its own (A K-contiguous on the
   // 256x256, 256x192 and 128x128 tiles); elsewhere the general epilogue applies it
-  int epi_kind = !fast_epi ? 0 : whole ? 1 : 3;
+  int epi_kind = !fast_epi ? 0 : whole && !masked ? 1 : 3;
   if (P.ep.row_scale && fast_epi)
     epi_kind = (P.dtype_in == MI_BF16 && fast && !P.transA && P.K % kstep == 0 &&
                 (plan.cfg == CFG_L || plan.cfg == CFG_M || plan.cfg == CFG_S)) ? 2 : 0;
@@ -876,7 +892,105 @@ __device__ __forceinline__ float block_reduce(float v, bool is_max, float* red) 
   return r;
 }
 
-// One workgroup per row; row r is query position q = r % T.
+// Softmax rows of up to 64 * EV * NV scores (EV per 16 bytes) on one wave each, held in
+// registers: every score is read once, at the elements' own alignment, and its exponential
+// computed once.  Bound by the scores' bytes; a workgroup per row with two-pass 4-byte
+// accesses took 32 us for 24576 rows of 512 fp32 (forward) and 28 (backward), 15 and 22 here.
+template <bool BF, int NV>
+struct SoftRow {
+  static constexpr int EV = BF ? 8 : 4;
+  // v[i][e]: element (lane + 64 i) * EV + e of the row at base, the first n of it (others 0)
+  __device__ static __forceinline__ void load(const void* p, int64_t base, int n, int lane, float (&v)[NV][EV]) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int k = (lane + 64 * i) * EV;
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
+      if (k + EV <= n) __builtin_memcpy(w, (const char*)p + (base + k) * (BF ? 2 : 4), 16);
+#pragma unroll
+      for (int e = 0; e < EV; ++e)
+        v[i][e] = BF ? bf16_bits_to_f32((w[e / 2] >> (16 * (e & 1))) & 0xffffu) : __uint_as_float(w[e & 3]);
+      if (k < n && k + EV > n)
+#pragma unroll
+        for (int e = 0; e < EV; ++e)
+          if (k + e < n) v[i][e] = ldv<BF>(p, base + k + e);
+    }
+  }
+  __device__ static __forceinline__ void store(void* p, int64_t base, int n, int lane, const float (&v)[NV][EV]) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int k = (lane + 64 * i) * EV;
+      if (k + EV <= n) {
+        uint32_t w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = BF ? pack_bf16x2(v[i][(2 * q) % EV], v[i][(2 * q + 1) % EV]) : __float_as_uint(v[i][q]);
+        __builtin_memcpy((char*)p + (base + k) * (BF ? 2 : 4), w, 16);
+      } else {
+#pragma unroll
+        for (int e = 0; e < EV; ++e)
+          if (k + e < n) stv<BF>(p, base + k + e, v[i][e]);
+      }
+    }
+  }
+};
+
+template <bool BF, int NV>
+__global__ void __launch_bounds__(256) softmax_causal_wave(void* S, int64_t rows, int T, int64_t ld) {
+  using Row = SoftRow<BF, NV>;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int n = (int)(row % T) + 1;  // keys 0 .. q
+  float v[NV][Row::EV];
+  Row::load(S, row * ld, n, lane, v);
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < Row::EV; ++e)
+      if ((lane + 64 * i) * Row::EV + e < n) mx = fmaxf(mx, v[i][e]);
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < Row::EV; ++e) {
+      v[i][e] = (lane + 64 * i) * Row::EV + e < n ? __expf(v[i][e] - mx) : 0.0f;
+      sum += v[i][e];
+    }
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  const float inv = 1.0f / sum;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < Row::EV; ++e)
+      if ((lane + 64 * i) * Row::EV + e < n) v[i][e] *= inv;  // zeros past q stay zeros
+  Row::store(S, row * ld, T, lane, v);
+}
+
+template <bool BF, int NV>
+__global__ void __launch_bounds__(256) softmax_bwd_wave(const void* P, void* dP, int64_t rows, int T, int64_t ld,
+                                                        float scale) {
+  using Row = SoftRow<BF, NV>;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  float p[NV][Row::EV], d[NV][Row::EV];
+  Row::load(P, row * ld, T, lane, p);
+  Row::load(dP, row * ld, T, lane, d);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < Row::EV; ++e) s += p[i][e] * d[i][e];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < Row::EV; ++e) d[i][e] = p[i][e] * (d[i][e] - s) * scale;
+  Row::store(dP, row * ld, T, lane, d);
+}
+
+// Longer rows: one workgroup per row; row r is query position q = r % T.
 template <bool BF>
 __global__ void __launch_bounds__(256) softmax_causal_kernel(void* S, int64_t T, int64_t ld) {
   __shared__ float red[4];
@@ -909,6 +1023,37 @@ __global__ void __launch_bounds__(256) softmax_bwd_kernel(const void* P, void* d
   }
 }
 
+// Launch `wave` (a functor taking the vectors per lane as a constant) where a row fits a wave's
+// registers; false where it does not.
+template <bool BF, typename F>
+bool launch_soft_wave(int64_t T, F&& wave) {
+  const int64_t per = 64 * (BF ? 8 : 4);
+  if (T <= per) wave(std::integral_constant<int, 1>{});
+  else if (T <= 2 * per) wave(std::integral_constant<int, 2>{});
+  else if (T <= 4 * per) wave(std::integral_constant<int, 4>{});
+  else if (T <= 8 * per) wave(std::integral_constant<int, 8>{});
+  else return false;
+  return true;
+}
+
+template <bool BF>
+void launch_softmax(void* S, int64_t rows, int64_t T, int64_t ld, hipStream_t st) {
+  if (!launch_soft_wave<BF>(T, [&](auto nv) {
+        hipLaunchKernelGGL((softmax_causal_wave<BF, decltype(nv)::value>), dim3((unsigned)cdiv(rows, 4)), dim3(256), 0,
+                           st, S, rows, (int)T, ld);
+      }))
+    hipLaunchKernelGGL(softmax_causal_kernel<BF>, dim3((unsigned)rows), dim3(256), 0, st, S, T, ld);
+}
+
+template <bool BF>
+void launch_softmax_bwd(const void* P, void* dP, int64_t rows, int64_t T, int64_t ld, float scale, hipStream_t st) {
+  if (!launch_soft_wave<BF>(T, [&](auto nv) {
+        hipLaunchKernelGGL((softmax_bwd_wave<BF, decltype(nv)::value>), dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, st,
+                           P, dP, rows, (int)T, ld, scale);
+      }))
+    hipLaunchKernelGGL(softmax_bwd_kernel<BF>, dim3((unsigned)rows), dim3(256), 0, st, P, dP, T, ld, scale);
+}
+
 }  // namespace
 
 // ---- C ABI -------------------------------------------------------------------------
@@ -932,10 +1077,10 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
   int cus = 256;
   if (init_devices() == MI_OK) cus = current_cus();
-  const Plan pl = make_plan(dtype_in, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, true);
+  const Plan pl = make_plan(dtype_in, !transA && transB, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, true);
   size_t need = pl.splits > 1 ? (size_t)pl.splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float) : 0;
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
-  if (skinny_fits(transA, M, N, K, batch, 1, MI_CAUSAL_NONE, MODE_PLAIN, ch)) {
+  if (skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, MODE_PLAIN, ch)) {
     // operands that rule the skinny kernels out take the tile plan, so room for either
     const SkinnyPlan sk = skinny_plan(dtype_in == MI_BF16, transB != 0, false, M, N, K, INT64_MAX / 8);
     if (sk.splits > 1) need = std::max(need, (size_t)sk.splits * (size_t)M * (size_t)N * sizeof(float));
@@ -1040,12 +1185,8 @@ int mi_softmax_causal(void* stream, void* S, int64_t rows, int64_t T, int64_t ld
   if (dtype != MI_F32 && dtype != MI_BF16) return fail(MI_ERR_DTYPE, "dtype %d", dtype);
   int st = init_devices();
   if (st != MI_OK) return st;
-  if (dtype == MI_BF16)
-    hipLaunchKernelGGL(softmax_causal_kernel<true>, dim3((unsigned)rows), dim3(256), 0,
-                       (hipStream_t)stream, S, T, ld);
-  else
-    hipLaunchKernelGGL(softmax_causal_kernel<false>, dim3((unsigned)rows), dim3(256), 0,
-                       (hipStream_t)stream, S, T, ld);
+  if (dtype == MI_BF16) launch_softmax<true>(S, rows, T, ld, (hipStream_t)stream);
+  else launch_softmax<false>(S, rows, T, ld, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? MI_OK : fail(MI_ERR_HIP, "softmax: %s", hipGetErrorString(e));
 }
@@ -1060,12 +1201,8 @@ int mi_softmax_bwd(void* stream, const void* P, void* dP, int64_t rows, int64_t 
   if (dtype != MI_F32 && dtype != MI_BF16) return fail(MI_ERR_DTYPE, "dtype %d", dtype);
   int st = init_devices();
   if (st != MI_OK) return st;
-  if (dtype == MI_BF16)
-    hipLaunchKernelGGL(softmax_bwd_kernel<true>, dim3((unsigned)rows), dim3(256), 0,
-                       (hipStream_t)stream, P, dP, T, ld, scale);
-  else
-    hipLaunchKernelGGL(softmax_bwd_kernel<false>, dim3((unsigned)rows), dim3(256), 0,
-                       (hipStream_t)stream, P, dP, T, ld, scale);
+  if (dtype == MI_BF16) launch_softmax_bwd<true>(P, dP, rows, T, ld, scale, (hipStream_t)stream);
+  else launch_softmax_bwd<false>(P, dP, rows, T, ld, scale, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? MI_OK : fail(MI_ERR_HIP, "softmax_bwd: %s", hipGetErrorString(e));
 }
@@ -1190,7 +1327,7 @@ int mi_flash_attn_bwd_scaled(void* stream, const void* Q, const void* K, const v
     // Causal skipping in the dQ GEMM works on whole K tiles up to the end of a
     // 128-row output tile; the dK/dV kernel writes dS^T (zeros included) for every
     // key below that bound, and not beyond it, so taller tiles take the dQ kernel.
-    const Plan pl = make_plan(MI_BF16, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN, false, 0,
+    const Plan pl = make_plan(MI_BF16, false, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN, false, 0,
                               current_cus(), true);
     if (shape_of(MI_BF16, pl.cfg).bm != 128) p.dsT = nullptr;
   }
@@ -1657,9 +1794,9 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   const bool dwords = a_contig % dw == 0 && b_contig % dw == 0;
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) ||
                     (dwords && dlds && (tail_ok(transA, transB, K, ch) || batch > 1 || ws > 0));
-  const Plan pl = (K == 0 || dwords) && skinny_fits(transA, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
+  const Plan pl = (K == 0 || dwords) && skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
                       ? skinny_as_plan(skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws))
-                      : make_plan(dtype_in, M, N, K, batch, mode, ws > 0, ws, cus, fast);
+                      : make_plan(dtype_in, !transA && transB, M, N, K, batch, mode, ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

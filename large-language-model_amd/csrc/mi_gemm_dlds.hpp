@@ -312,8 +312,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   // a variant of its own, so that the plain GEMMs carry no row-scale code (+0.45 % on the
   // configuration-3 set, one box)
   constexpr bool ROWSCALE = (VAR & DLDS_ROWSCALE) != 0;
-  // EDGE: M or N is not whole 32x32 blocks, so the direct epilogue guards its rows and quads
-  // of columns; a variant of its own, since the guards cost the whole-block GEMMs 1 %
+  // EDGE: M or N is not whole 32x32 blocks, or the causal mask is written: the direct epilogue
+  // guards its rows and quads of columns and masks them; a variant of its own, since the guards cost the whole-block GEMMs 1 %
   // (configuration-3 set 1903 -> 1924 us)
   constexpr bool EDGE = (VAR & DLDS_EDGE) != 0;
   constexpr int NWG = WGM * WGN;          // waves of one K group
@@ -367,6 +367,18 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
 
   if (p.causal == CAUSAL_OUT_LOWER && n0 > m0 + BM - 1) {
     if (p.splits > 1) return;  // the reduction kernel writes the mask
+    if (p.cvec && (p.N & 3) == 0) {  // in quads of columns
+      const uint32_t h = pack_bf16x2(p.mask_value, p.mask_value);
+      const f32x4_t f = {p.mask_value, p.mask_value, p.mask_value, p.mask_value};
+      for (int idx = threadIdx.x; idx < BM * BN / 4; idx += 64 * NWAVE) {
+        const int m = m0 + idx / (BN / 4), n = n0 + idx % (BN / 4) * 4;
+        if (m >= p.M || n >= p.N) continue;
+        const int64_t ci = (int64_t)m * p.ldc + n;
+        if (p.c_bf16) __builtin_nontemporal_store(u32x2_t{h, h}, (u32x2_t*)((uint16_t*)Cz + ci));
+        else __builtin_nontemporal_store(f, (f32x4_t*)((float*)Cz + ci));
+      }
+      return;
+    }
     for (int idx = threadIdx.x; idx < BM * BN; idx += 64 * NWAVE) {
       const int m = m0 + idx / BN, n = n0 + idx % BN;
       if (m < p.M && n < p.N) {
@@ -779,6 +791,14 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     const float beta = p.beta;
     // whether the quad of columns col of a row is inside a cut block
     auto in = [&](int row, int col) __attribute__((always_inline)) { return !EDGE || (row < p.M && col < p.N); };
+    auto mask = [&](f32x4_t& v, int row, int col) __attribute__((always_inline)) {
+      if constexpr (EDGE) {
+        if (p.causal == CAUSAL_OUT_LOWER)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = col + e > row ? p.mask_value : v[e];
+      }
+      (void)v; (void)row; (void)col;
+    };
     const int r_in = lane & 31, h_in = lane >> 5;
     const int r_out = lane >> 3, c_out = (lane & 7) * 4;  // + 8 rows per step
     // BF: bf16 C; BETA: beta*C is added.  Both uniform, hoisted out of the tile.
@@ -849,8 +869,9 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
             const int64_t roww = m0 + wm * WTM + i * 32 + rw_out;
 #pragma unroll
             for (int st = 0; st < 8; ++st) {
-              const f32x4_t v = *reinterpret_cast<const f32x4_t*>(patchw + (rw_out + 4 * st) * PPW + cw_out);
+              f32x4_t v = *reinterpret_cast<const f32x4_t*>(patchw + (rw_out + 4 * st) * PPW + cw_out);
               const int64_t ci = (roww + 4 * st) * p.ldc + colw;
+              mask(v, (int)roww + 4 * st, colw);
               if (ok && in((int)roww + 4 * st, colw))
                 __builtin_nontemporal_store(u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])},
                                             (u32x2_t*)((uint16_t*)Cz + ci));
@@ -884,6 +905,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
                 v[2] += beta * bf16_bits_to_f32(o[1] & 0xffffu);
                 v[3] += beta * bf16_bits_to_f32(o[1] >> 16);
               }
+              mask(v, (int)row0 + 8 * st, col);
               // non-temporal: C streams out instead of filling the XCD's L2 with dirty lines
               // (configuration-3 set 1133-1134 -> 1141-1144 TFLOP/s, down forward +4 %, one box)
               __builtin_nontemporal_store(u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])},
@@ -894,6 +916,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
                 v[0] += beta * o[0]; v[1] += beta * o[1];
                 v[2] += beta * o[2]; v[3] += beta * o[3];
               }
+              mask(v, (int)row0 + 8 * st, col);
               __builtin_nontemporal_store(v, (f32x4_t*)((float*)Cz + ci));
             }
           }

@@ -1,5 +1,6 @@
 // mi_skinny.hip -- GEMM of a few rows (token generation, short batches): C[M, N] with
-// M <= 64 and op(A) not transposed, bf16 or fp32, optionally with the dual-B SiLU gate.
+// M <= 64 and op(A) not transposed, bf16 or fp32, optionally with the dual-B SiLU gate; and
+// small fp32 products in blocks of 64 rows (skinny_blocks_fit).
 //
 // Bound: the weights B are read once from HBM and everything else is small, so a call
 // takes the time of streaming K x N elements plus a memory latency per launch.  What that
@@ -101,7 +102,9 @@ __global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))
   const int strips = (p.N + STRIP - 1) / STRIP;
   const int strip = uniform(item % strips), rest = uniform(item / strips);
   const int parts = dual_parts ? 2 : 1;
-  const int which = uniform(rest % parts), split = uniform(rest / parts);
+  const int which = uniform(rest % parts), outer = uniform(rest / parts);
+  // the K part, or of an unsplit product the block of rows
+  const int split = PART ? outer : 0, m0 = PART ? 0 : outer * (16 * MB);
   const int n0 = strip * STRIP;
 
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A, p.extA);
@@ -112,7 +115,7 @@ __global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))
   // byte offsets at k = 0; rows of A past M lie past its extent
   uint32_t ao[MB], bo[BKC ? CB : 1];
 #pragma unroll
-  for (int i = 0; i < MB; ++i) ao[i] = (uint32_t)((16 * i + cr) * lda + gr * 16);
+  for (int i = 0; i < MB; ++i) ao[i] = (uint32_t)((m0 + 16 * i + cr) * lda + gr * 16);
   if constexpr (BKC) {
 #pragma unroll
     for (int j = 0; j < CB; ++j) bo[j] = n0 + 16 * j + cr < p.N ? (uint32_t)((n0 + 16 * j + cr) * ldb + gr * 16) : kBufOOB;
@@ -206,7 +209,7 @@ __global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))
     compute(st);
   }
 
-  // acc[d][i][j][e]: row 16i + c, column n0 + CB * (4g + e) + j (K-contiguous B: 16j + 4g + e)
+  // acc[d][i][j][e]: row m0 + 16i + c, column n0 + CB * (4g + e) + j (K-contiguous B: 16j + 4g + e)
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -226,7 +229,7 @@ __global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))
     }
   __syncthreads();
   constexpr int QPR = STRIP / 4;  // 4-column groups per row
-  const int rows = p.M < MB * 16 ? p.M : MB * 16;
+  const int rows = p.M - m0 < MB * 16 ? p.M - m0 : MB * 16;
   const bool partial = p.splits > 1 || dual_parts;
   for (int t = threadIdx.x; t < rows * QPR; t += 64 * NW) {
     const int m = t / QPR, nq = (t - m * QPR) * 4, n = n0 + nq;
@@ -252,7 +255,7 @@ __global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       v[e] = ND == 2 ? silu_f(p.alpha * sum[0][e]) * (p.alpha * sum[ND - 1][e]) : p.alpha * sum[0][e];
-    epilogue4(p, p.C, p.R, m, n, v);
+    epilogue4(p, p.C, p.R, m0 + m, n, v);
   }
 }
 
@@ -304,7 +307,7 @@ __global__ void __launch_bounds__(64) skinny_reduce_kernel(Params p) {
 
 template <typename T, bool BKC, int MB, int ND, bool PART>
 void launch_one(const Params& p, const SkinnyPlan& pl, hipStream_t st) {
-  const dim3 grid((unsigned)(pl.strips * pl.splits * (pl.dual_parts ? 2 : 1)));
+  const dim3 grid((unsigned)(pl.strips * pl.splits * pl.blocks * (pl.dual_parts ? 2 : 1)));
   const dim3 block((unsigned)(64 * (PART ? PART_WAVES : whole_waves(MB, ND))));
   hipLaunchKernelGGL((skinny_kernel<T, BKC, MB, ND, PART>), grid, block, 0, st, p, (int)pl.dual_parts);
 }
@@ -323,6 +326,11 @@ void launch_rows(const Params& p, const SkinnyPlan& pl, bool both, hipStream_t s
 }
 
 }  // namespace
+
+bool skinny_blocks_fit(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K) {
+  const int64_t blocks = ((M + 63) / 64) * ((N + 31) / 32);
+  return !bf16 && !transB && !dual && K <= 1024 && blocks >= 128 && blocks <= 256;
+}
 
 SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems) {
   SkinnyPlan pl{};
@@ -348,7 +356,8 @@ SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, 
   const double t_whole = 1.0 + std::max(whole / 24e3 * (double)((strips_of(false) + 255) / 256), bytes / 2.3e6);
   const double t_part = bytes / 3.5e6 * std::max(1.0, 160.0 / (double)(groups * std::max<int64_t>(sp, 1))) +
                         (sp > 1 || dual ? 3.5 + 8.0 * (double)(sp * nd * M * N) / 3.5e6 : 0.0);
-  pl.part = sp >= 1 && t_part < t_whole;
+  pl.blocks = (int)((M + 63) / 64);
+  pl.part = sp >= 1 && t_part < t_whole && pl.blocks == 1;
   pl.splits = pl.part ? (int)sp : 1;
   pl.dual_parts = pl.part && dual;
   pl.cols = cols_of(pl.part);

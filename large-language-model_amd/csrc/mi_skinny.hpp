@@ -12,8 +12,15 @@ namespace mig {
 constexpr int SKINNY_MAX_M = 64;
 constexpr int64_t SKINNY_WIDE_BYTES = (int64_t)24 << 20;
 
+// Taller fp32 NN products whose 64-row x 32-column blocks fill at least half of the CUs and at
+// most all of them, K up to 1024: each on a workgroup of 8 waves that share K.  A tile kernel leaves them the choice
+// between idle CUs and a second launch (512 x 768 x 768 with bias: 64x128 tiles split 5 16.0
+// us, 64x64 tiles 16.9, here 12.1).  The NT form would read A again for every 16 columns.
+bool skinny_blocks_fit(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K);
+
 struct SkinnyPlan {
-  int mb;      // blocks of 16 rows: 1, 2 or 4
+  int mb;      // blocks of 16 rows of a workgroup: 1, 2 or 4
+  int blocks;  // workgroups along M: 1 up to 64 rows
   int cols;    // output columns of a workgroup's strip
   int strips;
   int splits;  // workgroups along K

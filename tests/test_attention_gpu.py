@@ -344,3 +344,29 @@ def test_flash_backward_graph_replays(mi, dev):
         eager = mi.flash_attn_bwd(Q, K, V, O, dO, lse, workspace=ws)
         for got, want in zip(eager, ref):
             assert torch.equal(got, want), i
+
+
+@pytest.mark.parametrize("bf16", [True, False], ids=["bf16", "f32"])
+@pytest.mark.parametrize("T", [1, 2, 7, 255, 256, 257, 511, 1023, 1029, 2048, 2052, 4095, 4100])
+def test_softmax_rows(mi, dev, bf16, T):
+    """Causal row softmax and its backward at the edges of a wave's registers (and past them), odd
+    rows off 16-byte alignment, keys past the query infinite or NaN: they are not read."""
+    import torch
+
+    dt = torch.bfloat16 if bf16 else torch.float32
+    g = torch.Generator(device=dev).manual_seed(T)
+    n = 2 if T < 3000 else 1
+    S = (4 * torch.randn(n, T, T, generator=g, device=dev)).to(dt)
+    up = torch.ones(T, T, dtype=torch.bool, device=dev).triu_(1)
+    ref = torch.softmax(S.double().masked_fill(up, -float("inf")), -1)
+    P = S.clone()
+    P[0].masked_fill_(up, float("inf"))
+    P[n - 1].masked_fill_(up, float("nan"))
+    mi.softmax_causal_(P, T)
+    tol = 2.0 ** -8 if bf16 else 1e-5  # one bf16 rounding; fp32 exp and sum
+    assert (P.double() - ref).abs().max().item() <= tol
+    assert (P.masked_select(up) == 0).all()
+    dP = torch.randn(n, T, T, generator=g, device=dev).to(dt)
+    want = P.double() * (dP.double() - (P.double() * dP.double()).sum(-1, keepdim=True)) * 0.125
+    mi.softmax_bwd_(P, dP, T, 0.125)
+    assert (dP.double() - want).abs().max().item() <= tol * max(1e-3, want.abs().max().item())

@@ -812,3 +812,34 @@ def test_dual_tiles(mi, dev, bf16, M, N, K, want, tB):
     check(host(C), host(ref), _tol(bf16), f"dual {M}x{N}x{K}")
     mi.gemm(A, st(Bg), C, M, N, K, transB=bool(tB), B2=st(Bu), bias=bias, residual=R)
     check(host(C), host(ref + bias.double() + R.double()), _tol(bf16), f"dual {M}x{N}x{K} bias residual")
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 4096, 4), (512, 768, 768), (200, 1026, 1024), (1025, 480, 52), (4096, 65, 36)])
+def test_small_fp32_blocks(mi, dev, oracle, M, N, K):
+    """fp32 NN products in 64-row x 32-column blocks (mi_skinny.hip), whole and cut, with the
+    epilogues."""
+    assert mi.describe(0, 0, M, N, K, mi.MI_F32).startswith("skinny f32")
+    for kw in (dict(bias=True), dict(beta=0.5, residual=True, pad=(4, 0, 4))):
+        got, ref = _run(mi, dev, oracle, M, N, K, 0, 0, False, seed=500 + M, **kw)
+        check(got, ref, TOL_F32, f"small fp32 {M}x{N}x{K} {kw}")
+
+
+@pytest.mark.parametrize("bf16", [True, False], ids=["bf16", "f32"])
+@pytest.mark.parametrize("T,N", [(128, 128), (300, 300), (132, 260), (260, 130), (67, 67), (520, 516)])
+def test_causal_output_mask(mi, dev, bf16, T, N):
+    """MI_CAUSAL_OUT_LOWER on whole, cut and wholly masked tiles, C = 2 on entry with beta = 1, the
+    mask written over everything above the diagonal; integers, bit for bit in fp32."""
+    import torch
+
+    dt = torch.bfloat16 if bf16 else torch.float32
+    g = torch.Generator(device=dev).manual_seed(T + N)
+    a = torch.randint(-2, 3, (3, T, 40), generator=g, device=dev)
+    b = torch.randint(-2, 3, (3, 40, N), generator=g, device=dev)
+    for beta in (0.0, 1.0):
+        C = torch.full((3, T, N), 2.0, dtype=dt, device=dev)
+        bt = mi.make_batch(3, 1, a=(T * 40, 0, 1), b=(40 * N, 0, 1), c=(T * N, 0, 1),
+                           causal=mi.MI_CAUSAL_OUT_LOWER, mask_value=-7.0)
+        mi.gemm_batched(a.to(dt), b.to(dt), C, T, N, 40, bt, beta=beta)
+        ref = (a.double() @ b.double() + 2.0 * beta)
+        ref.masked_fill_(torch.ones(T, N, dtype=torch.bool, device=dev).triu_(1), -7.0)
+        assert torch.equal(C, ref.to(dt)), (T, N, beta)
