@@ -217,7 +217,14 @@ def _ptr(t):
 
 
 def _stream():
-    return ctypes.c_void_p(_torch().cuda.current_stream().cuda_stream)
+    """The handle of torch's current stream. Once CUDA is initialised it is read without the
+    Stream object that torch.cuda.current_stream() builds: 0.4 instead of 3-4 us, a third of the
+    host time of a small call."""
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(raw(torch.cuda.current_device()))
 
 
 _scope_depth = 0
