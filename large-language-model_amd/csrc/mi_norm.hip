@@ -21,14 +21,16 @@
 // weight gradient of its own columns in registers; the waves of a workgroup add
 // their partials in wave order through LDS into one workspace row, and a second
 // kernel sums the workspace rows in order: dw is bit-identical across launches.
-// Generic path (rows that are not whole aligned 16-byte vectors, or longer): one
-// 256-thread workgroup per row, strided passes over global memory.  xhat is formed as
+// Rows that are not whole aligned 16-byte vectors, or longer (up to 16384 bf16 / 8192 fp32
+// values): a workgroup per row, the row in registers too (norm_fwd_row, norm_bwd_row); past
+// that, or under 16 bytes, strided passes over global memory.  xhat is formed as
 // x * (1/rms): one reciprocal per row instead of a division per element (the divide
 // sequence made the backward VALU-bound).
 #include <hip/hip_runtime.h>
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "mi_gemm_device.hpp"
 #include "mi_norm.hpp"
@@ -167,6 +169,127 @@ __global__ void __launch_bounds__(256) norm_fwd_vec(NormParams p) {
       for (int e = 0; e < EV; ++e) o[e] = v[i][e] * rs * wv[e];
       store_act<BF16>(yr, j * EV, o);
     }
+  }
+}
+
+// Rows that the wave kernels do not take (more than 8 vectors a lane, or off 16-byte
+// alignment): one workgroup per row, the row in registers in runs of EV elements (16 bytes,
+// loaded and stored at the elements' own alignment), NV runs per thread.  The run that the
+// row's end would cut is moved back to end there, and the elements it then shares with the
+// run before it count and are stored there only: every load is one unconditional 16-byte
+// access, which keeps the backward's next row in flight (with the cut run read element by
+// element each row waited for memory: 132 us instead of 42 for 13361 x 1487 bf16).  The
+// strided kernels read a row two or three times in 2- or 4-byte accesses; forward + backward
+// against them, us: 13361 x 1487 bf16 331 -> 77, 8192 x 8192 bf16 1102 -> 165,
+// 4000 x 4097 fp32 299 -> 94, 40 x 6001 bf16 71 -> 24.
+template <int EV>
+struct RunSpan {
+  int k, skip;  // first element; elements of the run that belong to the run before (EV: all)
+  __device__ __forceinline__ RunSpan(int run, int n) {
+    const int64_t at = (int64_t)run * EV, last = n - EV;  // n >= EV
+    k = (int)(at < last ? at : last);
+    skip = at - k < EV ? (int)(at - k) : EV;
+  }
+};
+template <bool BF>
+struct NormRun {
+  uint32_t w[4];
+  __device__ __forceinline__ void load(const void* base, int k) {
+    __builtin_memcpy(w, (const char*)base + (int64_t)k * (BF ? 2 : 4), 16);
+  }
+  __device__ __forceinline__ float at(int e) const {
+    if constexpr (BF) return __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16);
+    else return __uint_as_float(w[e]);
+  }
+};
+// EV weights from element k on (EV: the run of the rows, the weights' own type may differ).
+template <bool WBF, int EV>
+__device__ __forceinline__ void load_weights(const void* w, int k, float* v) {
+#pragma unroll
+  for (int e = 0; e < EV; ++e) v[e] = ld_elem<WBF>(w, k + e);
+}
+template <bool BF, int EV>
+__device__ __forceinline__ void store_run(void* base, int k, int skip, const float* v) {
+  if (skip == 0) {
+#pragma unroll
+    for (int h = 0; h < EV; h += BF ? 8 : 4) {
+      uint32_t w[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if constexpr (BF) w[q] = pack_bf16x2(v[2 * q], v[2 * q + 1]);
+        else w[q] = __float_as_uint(v[h + q]);
+      }
+      __builtin_memcpy((char*)base + (int64_t)(k + h) * (BF ? 2 : 4), w, 16);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < EV; ++e)
+      if (e >= skip) st_elem<BF>(base, k + e, v[e]);
+  }
+}
+// Sum of the waves' partials, pairwise.
+template <int N>
+__device__ __forceinline__ float sum_waves(const float* v) {
+  if constexpr (N == 1) return v[0];
+  else return sum_waves<N / 2>(v) + sum_waves<N / 2>(v + N / 2);
+}
+
+template <bool BF16, bool W_BF16, int NV, int TH>
+__global__ void __launch_bounds__(TH) norm_fwd_row(NormParams p) {
+  constexpr int EV = BF16 ? 8 : 4, ES = BF16 ? 2 : 4;
+  __shared__ float red[TH / 64];
+  const int row = blockIdx.x, n = p.dims;
+  char* xr = (char*)p.x + (int64_t)row * p.ld * ES;
+  float v[NV][EV];
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    NormRun<BF16> xv;
+    xv.load(xr, RunSpan<EV>(threadIdx.x + TH * i, n).k);
+#pragma unroll
+    for (int e = 0; e < EV; ++e) v[i][e] = xv.at(e);
+  }
+  if (p.r) {
+    const char* rr = (const char*)p.r + (int64_t)row * p.ld * ES;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const RunSpan<EV> at(threadIdx.x + TH * i, n);
+      NormRun<BF16> rv;
+      rv.load(rr, at.k);
+#pragma unroll
+      for (int e = 0; e < EV; ++e) v[i][e] += rv.at(e);
+      store_run<BF16, EV>(xr, at.k, at.skip, v[i]);
+      if constexpr (BF16) {
+#pragma unroll
+        for (int e = 0; e < EV; ++e) v[i][e] = bf16_round(v[i][e]);  // the value stored
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const RunSpan<EV> at(threadIdx.x + TH * i, n);
+#pragma unroll
+    for (int e = 0; e < EV; ++e) {
+      const float x = e >= at.skip ? v[i][e] : 0.0f;
+      ss = __builtin_fmaf(x, x, ss);
+    }
+  }
+  ss = nwave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = sum_waves<TH / 64>(red);
+  const float rs = 1.0f / sqrtf(ss / (float)n + p.eps);
+  if (p.rstd && threadIdx.x == 0) p.rstd[row] = rs;
+  if (!p.y) return;  // statistic only (the norm folded into a GEMM)
+  char* yr = (char*)p.y + (int64_t)row * p.ld * ES;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const RunSpan<EV> at(threadIdx.x + TH * i, n);
+    float wv[EV];
+    load_weights<W_BF16, EV>(p.w, at.k, wv);
+#pragma unroll
+    for (int e = 0; e < EV; ++e) v[i][e] = v[i][e] * rs * wv[e];
+    store_run<BF16, EV>(yr, at.k, at.skip, v[i]);
   }
 }
 
@@ -338,6 +461,93 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NV <= 
   }
 }
 
+// Backward of norm_fwd_row's rows: each workgroup walks its rows with the next row's runs in
+// flight, its columns' weight and weight gradient in registers.  Rows of more than 512 runs
+// take more threads, not more runs each: 8 runs of 256 threads need every register a wave can
+// have, and one wave a SIMD left 8192 x 8192 bf16 at 359 us instead of 165.
+template <bool BF16, bool W_BF16, int NV, int TH>
+__global__ void __launch_bounds__(TH) norm_bwd_row(NormParams p) {
+  constexpr int EV = BF16 ? 8 : 4, ES = BF16 ? 2 : 4;
+  constexpr bool AHEAD = TH < 1024;  // 1024 threads have 128 registers each
+  __shared__ float red[2][2][TH / 64];
+  const int n = p.dims;
+  float acc[NV][EV], wr[NV][EV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const RunSpan<EV> at(threadIdx.x + TH * i, n);
+    load_weights<W_BF16, EV>(p.w, at.k, wr[i]);
+#pragma unroll
+    for (int e = 0; e < EV; ++e) {
+      wr[i][e] = e >= at.skip ? wr[i][e] : 0.0f;  // not the other run's infinity times zero
+      acc[i][e] = 0.0f;
+    }
+  }
+  struct Row {
+    NormRun<BF16> x[NV], g[NV], r[NV];
+  };
+  auto load_row = [&](int row, Row& d) __attribute__((always_inline)) {
+    const int64_t off = (int64_t)row * p.ld * ES;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int k = RunSpan<EV>(threadIdx.x + TH * i, n).k;
+      d.x[i].load((const char*)p.x + off, k);
+      d.g[i].load((const char*)p.dy + off, k);
+      if (p.r) d.r[i].load((const char*)p.r + off, k);
+      else d.r[i] = NormRun<BF16>{};
+    }
+  };
+  Row cur;
+  int row = blockIdx.x, par = 0;
+  if (row < p.rows) load_row(row, cur);
+  for (; row < p.rows; row += gridDim.x, par ^= 1) {
+    Row nxt;
+    if (AHEAD && row + (int)gridDim.x < p.rows) load_row(row + gridDim.x, nxt);
+    float ss = 0.0f, t = 0.0f;  // sum x^2, sum dy*w*x
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const RunSpan<EV> at(threadIdx.x + TH * i, n);
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        const float x = e >= at.skip ? cur.x[i].at(e) : 0.0f, g = e >= at.skip ? cur.g[i].at(e) : 0.0f;
+        ss = __builtin_fmaf(x, x, ss);
+        t = __builtin_fmaf(g * wr[i][e], x, t);
+      }
+    }
+    nwave_sum2(ss, t);
+    if ((threadIdx.x & 63) == 0) {
+      red[par][0][threadIdx.x >> 6] = ss;
+      red[par][1][threadIdx.x >> 6] = t;
+    }
+    __syncthreads();  // the other half of red is not read again before the next row's barrier
+    ss = sum_waves<TH / 64>(red[par][0]);
+    t = sum_waves<TH / 64>(red[par][1]);
+    const float rinv = 1.0f / sqrtf(ss / (float)n + p.eps);
+    const float cx = rinv * rinv * rinv * (t / (float)n);
+    char* dxr = (char*)p.dx + (int64_t)row * p.ld * ES;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float o[EV];
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        o[e] = __builtin_fmaf(rinv, cur.g[i].at(e) * wr[i][e], __builtin_fmaf(-cx, cur.x[i].at(e), cur.r[i].at(e)));
+        acc[i][e] = __builtin_fmaf(cur.g[i].at(e) * rinv, cur.x[i].at(e), acc[i][e]);
+      }
+      const RunSpan<EV> at(threadIdx.x + TH * i, n);
+      store_run<BF16, EV>(dxr, at.k, at.skip, o);
+    }
+    if (AHEAD) cur = nxt;
+    else if (row + (int)gridDim.x < p.rows) load_row(row + gridDim.x, cur);
+  }
+  if (p.dw) {
+    float* wsr = p.ws + (int64_t)blockIdx.x * n;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const RunSpan<EV> at(threadIdx.x + TH * i, n);
+      store_run<false, EV>(wsr, at.k, at.skip, acc[i]);
+    }
+  }
+}
+
 template <bool BF16, bool W_BF16>
 __global__ void __launch_bounds__(256) norm_bwd_gen(NormParams p) {
   constexpr int ES = BF16 ? 2 : 4;
@@ -434,6 +644,14 @@ __global__ void __launch_bounds__(256) norm_fold_weight_kernel(const void* w, co
   }
 }
 
+// Runs of 16 bytes per thread of a 256-thread workgroup that holds a row: 1, 2, 4, 8, or 9
+// where the row kernels do not apply (more, or less than one run).
+int runs_per_thread(int dims, bool bf16) {
+  if (dims < (bf16 ? 8 : 4)) return 9;
+  const int64_t per = ((int64_t)dims + (bf16 ? 2048 : 1024) - 1) / (bf16 ? 2048 : 1024);
+  return per <= 2 ? (int)per : per <= 4 ? 4 : per <= 8 ? 8 : 9;
+}
+
 int vec_per_lane(int dims, bool bf16) {
   const int per = (dims / (bf16 ? 8 : 4) + 63) / 64;
   return per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : 8;
@@ -441,6 +659,17 @@ int vec_per_lane(int dims, bool bf16) {
 
 template <bool BF16, bool W_BF16>
 hipError_t fwd_one(const NormParams& p, bool vector_path, hipStream_t st) {
+  const int runs = runs_per_thread(p.dims, BF16);
+  const dim3 rows((unsigned)p.rows);
+  if (!vector_path && runs <= 8) {
+    switch (runs) {
+      case 1: hipLaunchKernelGGL((norm_fwd_row<BF16, W_BF16, 1, 256>), rows, dim3(256), 0, st, p); break;
+      case 2: hipLaunchKernelGGL((norm_fwd_row<BF16, W_BF16, 2, 256>), rows, dim3(256), 0, st, p); break;
+      case 4: hipLaunchKernelGGL((norm_fwd_row<BF16, W_BF16, 2, 512>), rows, dim3(512), 0, st, p); break;
+      default: hipLaunchKernelGGL((norm_fwd_row<BF16, W_BF16, 2, 1024>), rows, dim3(1024), 0, st, p); break;
+    }
+    return hipGetLastError();
+  }
   if (!vector_path) {
     hipLaunchKernelGGL((norm_fwd_gen<BF16, W_BF16>), dim3((unsigned)p.rows), dim3(256), 0, st, p);
     return hipGetLastError();
@@ -458,7 +687,16 @@ hipError_t fwd_one(const NormParams& p, bool vector_path, hipStream_t st) {
 template <bool BF16, bool W_BF16>
 hipError_t bwd_one(const NormParams& p, bool vector_path, hipStream_t st) {
   const int G = norm_bwd_grid(p.rows);
-  if (!vector_path) {
+  const int runs = runs_per_thread(p.dims, BF16);
+  const dim3 groups((unsigned)G);
+  if (!vector_path && runs <= 8) {
+    switch (runs) {
+      case 1: hipLaunchKernelGGL((norm_bwd_row<BF16, W_BF16, 1, 256>), groups, dim3(256), 0, st, p); break;
+      case 2: hipLaunchKernelGGL((norm_bwd_row<BF16, W_BF16, 2, 256>), groups, dim3(256), 0, st, p); break;
+      case 4: hipLaunchKernelGGL((norm_bwd_row<BF16, W_BF16, 2, 512>), groups, dim3(512), 0, st, p); break;
+      default: hipLaunchKernelGGL((norm_bwd_row<BF16, W_BF16, 2, 1024>), groups, dim3(1024), 0, st, p); break;
+    }
+  } else if (!vector_path) {
     hipLaunchKernelGGL((norm_bwd_gen<BF16, W_BF16>), dim3((unsigned)G), dim3(256), 0, st, p);
   } else {
     const dim3 grid((unsigned)G), block(256);

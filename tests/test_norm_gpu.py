@@ -101,6 +101,49 @@ def test_in_place_and_determinism(mi, dev, dt_x, dims):
     assert torch.equal(dx4, dx5)
 
 
+@pytest.mark.parametrize("dt_x,dt_w", [("bf16", "bf16"), ("bf16", "f32"), ("f32", "bf16")])
+@pytest.mark.parametrize("runs,off", [(1, -1), (1, 0), (1, 1), (2, -1), (255, 3), (256, 1), (512, 1), (1023, 1),
+                                      (1024, 1), (2047, 1), (2048, 0), (2048, 1)])
+def test_rows_off_alignment(mi, dev, oracle, runs, off, dt_x, dt_w):
+    """Rows of `runs` 16-byte runs and `off` elements, at odd addresses and pitches: the last run
+    moved back into the row, every workgroup size and run count, the strided kernels past them
+    and under one run; weights that are infinite or NaN stay in their own columns.  Bounds: each
+    sum of n fp32 products in any order errs by at most n * 2^-24 of its terms' magnitudes
+    (n <= 16385: 1e-3), here ~ sqrt(n) * 2^-24 < 1e-5 (TOL_F32 1e-4); bf16 stores 2^-9."""
+    import torch
+
+    dt = torch.bfloat16 if dt_x == "bf16" else torch.float32
+    wdt = torch.bfloat16 if dt_w == "bf16" else torch.float32
+    dims, rows, eps = runs * (8 if dt_x == "bf16" else 4) + off, 9, 1e-5
+    ld = dims + 3
+    rng = np.random.default_rng(dims)
+    flat = [torch.full((rows * ld + 1,), 7.0, dtype=dt, device=dev) for _ in range(5)]
+    x, r, g, y, dx = [f[1:].view(rows, ld)[:, :dims] for f in flat]
+    for t in (x, r, g):
+        t.copy_(torch.from_numpy(rng.normal(0, 1, (rows, dims)).astype(np.float32)).to(dev, dt))
+    w = torch.full((dims + 1,), 1.0, dtype=wdt, device=dev)[1:]
+    w.copy_(torch.from_numpy(rng.normal(1, 0.2, dims).astype(np.float32)).to(dev, wdt))
+    xv, rv, gv, wv = _np(x), _np(r), _np(g), _np(w)
+    tol = TOL_F32 if dt_x == "f32" else TOL_BF16
+    dx_ref, dw_ref = oracle.rmsnorm_bwd(gv, xv, wv, eps, residual_grad=rv, dw0=np.zeros(dims))
+    mi.rms_norm_backward(g, x, w, eps, residual_grad=r, dx=dx)
+    check(host(dx), dx_ref, tol, "dx")
+    dx2, dw = mi.rms_norm_backward(g, x, w, eps, residual_grad=r)
+    assert torch.equal(dx2, dx)
+    check(host(dw), dw_ref, TOL_F32 if dt_x == "f32" else 2e-3, "dw")
+    y_ref, _, x_after = oracle.rmsnorm_fwd(xv, wv, eps, residual=rv, round_bf16=dt_x == "bf16")
+    mi.rms_norm_forward(x, w, eps, residual=r, out=y)
+    assert np.array_equal(_np(x), x_after)
+    check(host(y), y_ref, tol, "y")
+    for f in flat:      # nothing before the first row or between rows
+        pad = f[1:].view(rows, ld)[:, dims:]
+        assert float(f[0]) == 7.0 and bool((pad == 7.0).all())
+    w[0], w[-1] = float("inf"), float("nan")
+    bad = host(mi.rms_norm_forward(x, w, eps)).reshape(rows, dims)
+    ok = np.isfinite(bad).all(0)
+    assert ok[1:-1].all() and np.isnan(bad[:, -1]).all()
+
+
 def test_bf16_weight_gradient_and_mirror(mi, dev, oracle):
     import torch
 
