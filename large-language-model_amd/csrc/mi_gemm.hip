@@ -668,8 +668,9 @@ int run(const Problem& P, hipStream_t stream) {
   };
   const bool spanA = extA < lim && span_ok(!P.transA, a_rows, P.lda);
   const bool spanB = extB < lim && span_ok(P.transB != 0, b_rows, P.ldb);
-  // The skinny and the direct-to-LDS kernels (every mode but the prologue) need no more than 4-byte alignment: a buffer load's address and its bounds check work in
-  // dwords.  A row-contiguous chunk that straddles the matrix edge feeds outputs that are
+  // The skinny and the direct-to-LDS kernels (every mode but the prologue) need no more than
+  // 4-byte alignment: a buffer load's address and its bounds check work in dwords.  A
+  // row-contiguous chunk that straddles the matrix edge feeds outputs that are
   // not stored; a K-contiguous one is zeroed past K in LDS (tail_ok).
   auto dw = [&](const void* q, int64_t ld, int64_t o, int64_t i, int64_t sg) {
     return ((uintptr_t)q & 3u) == 0 && (esz == 4 || (ld % 2 == 0 && o % 2 == 0 && i % 2 == 0 && sg % 2 == 0));
@@ -742,7 +743,8 @@ int run(const Problem& P, hipStream_t stream) {
   const bool masked = b.causal == MI_CAUSAL_OUT_LOWER;
   const bool fast_epi = plan.splits == 1 && !P.ep.bias && !P.ep.residual && cvec &&
                         ((whole && !masked) || (P.N % 4 == 0 && !P.ep.row_scale));
-  const int64_t kstep = P.dtype_in != MI_BF16 ? 32 : plan.cfg == CFG_W || plan.cfg == CFG_V || plan.cfg == CFG_DUAL_W ? MI_W_BK : 64;
+  const bool groups = plan.cfg == CFG_W || plan.cfg == CFG_V || plan.cfg == CFG_DUAL_W;
+  const int64_t kstep = P.dtype_in != MI_BF16 ? 32 : groups ? MI_W_BK : 64;
   // with a row scale the direct epilogue has a variant of its own (A K-contiguous on the
   // 256x256, 256x192 and 128x128 tiles); elsewhere the general epilogue applies it
   int epi_kind = !fast_epi ? 0 : whole && !masked ? 1 : 3;

@@ -313,8 +313,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   // configuration-3 set, one box)
   constexpr bool ROWSCALE = (VAR & DLDS_ROWSCALE) != 0;
   // EDGE: M or N is not whole 32x32 blocks, or the causal mask is written: the direct epilogue
-  // guards its rows and quads of columns and masks them; a variant of its own, since the guards cost the whole-block GEMMs 1 %
-  // (configuration-3 set 1903 -> 1924 us)
+  // guards its rows and quads of columns and masks them; a variant of its own, since the guards
+  // cost the whole-block GEMMs 1 % (configuration-3 set 1903 -> 1924 us)
   constexpr bool EDGE = (VAR & DLDS_EDGE) != 0;
   constexpr int NWG = WGM * WGN;          // waves of one K group
   constexpr int NWAVE = NWG * KG;         // waves of the workgroup
@@ -413,6 +413,19 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  // fp32: every other MFMA of a fragment pair sums into accumulators of its own, joined at
+  // the end: each rounding chain is half as long, as if K were split in two, which keeps the
+  // products that the planner no longer splits as close to their 64-bit values as before.
+  // The registers are there: LDS bounds the workgroups per CU (5 of 64x64, 3 of 64x128).
+  // Error against 64 bits: training block on 2048 tokens 8.1e-7 -> 5.7e-7, the materialised
+  // attention 5.6e-7 -> 4.0e-7; their times 771 -> 779 us, and 162 -> 162-164.
+  f32x16_t acc_odd[ES == 4 ? TM : 1][ES == 4 ? NB : 1];
+  if constexpr (ES == 4) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc_odd[i][j] = acc[i][j];
+  }
 
   OpA oa;
   OpB ob;
@@ -532,8 +545,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
       // (lanes 32-63), the two k of one 32x32x2 MFMA
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[set][j][t]),
-                                                         __uint_as_float(fa[set][i][t]), acc[i][j], 0, 0, 0);
+        (t & 1 ? acc_odd : acc)[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            __uint_as_float(fb[set][j][t]), __uint_as_float(fa[set][i][t]), (t & 1 ? acc_odd : acc)[i][j], 0, 0, 0);
     }
   };
 
@@ -720,6 +733,14 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     }
   }
   wait_vmcnt<0>();  // DMAs of the all-zero tiles past it1
+  if constexpr (ES == 4) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] += acc_odd[i][j][e];
+  }
 
   // acc[i][j][4q + e] holds C[m][n + e] with
   //   m = m0 + wm*WTM + i*32 + (lane & 31),  n = n0 + wn*WTN + j*32 + 8q + 4*(lane >> 5).
