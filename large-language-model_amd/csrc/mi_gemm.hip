@@ -111,7 +111,7 @@ int current_cus() {
 
 // ---- kernel table ------------------------------------------------------------
 
-KernelFn pick_kernel(int dtype_in, int transA, int transB, int cfg, bool fast, bool ktail,
+KernelFn pick_kernel(int dtype_in, int transA, int transB, int cfg, bool fast, int ktail,
                      int fast_epi) {
   const int lay = (transA ? 2 : 0) | (transB ? 1 : 0);
   if (dtype_in == MI_BF16) {
@@ -751,8 +751,10 @@ int run(const Problem& P, hipStream_t stream) {
   if (P.ep.row_scale && fast_epi)
     epi_kind = (P.dtype_in == MI_BF16 && fast && !P.transA && P.K % kstep == 0 &&
                 (plan.cfg == CFG_L || plan.cfg == CFG_M || plan.cfg == CFG_S)) ? 2 : 0;
+  const bool straddle = (!P.transA && !mult(a_ext)) || (P.transB && !mult(b_ext));
+  const int ktail = P.K % kstep == 0 ? 0 : straddle ? 2 : 1;
   KernelFn fn = skinny ? nullptr
-                       : pick_kernel(P.dtype_in, P.transA, P.transB, plan.cfg, fast, P.K % kstep != 0, epi_kind);
+                       : pick_kernel(P.dtype_in, P.transA, P.transB, plan.cfg, fast, ktail, epi_kind);
   if (!fn && !skinny) return fail(MI_ERR_UNSUPPORTED, "no kernel for this layout / mode");
 
   Params p;

@@ -288,11 +288,12 @@ struct DldsOperand {
 };
 
 // Kernel variants (VAR bits): the K segment length is not a multiple of BK
-// (K-contiguous operands then mask the chunks past the segment end, and zero the rest
-// of a chunk that straddles it in LDS), and the problem takes the direct epilogue (every tile full, epilogue alpha / SiLU
+// (K-contiguous operands then mask the chunks past the segment end), nor of a 16-byte chunk
+// (STRADDLE, with KTAIL: the rest of the chunk that straddles the end is zeroed in LDS), and
+// the problem takes the direct epilogue (every tile full, epilogue alpha / SiLU
 // gate, beta*C and the output conversion only, no split-K).  One kernel holding
 // both epilogues would need the accumulators in two places at once.
-enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4, DLDS_EDGE = 8 };
+enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4, DLDS_EDGE = 8, DLDS_STRADDLE = 16 };
 
 // GEMM of WGM x WGN waves, wave tile (BM/WGM) x (BN/WGN) of 32x32 MFMA blocks: bf16
 // (ES = 2, one 32x32x16 MFMA per block and substep) or fp32 (ES = 4, four 32x32x2).
@@ -307,6 +308,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     __attribute__((amdgpu_waves_per_eu(WGM * WGN * KG / 4)))
     gemm_dlds_kernel(Params p) {
   constexpr bool KTAIL = (VAR & DLDS_KTAIL) != 0;
+  // STRADDLE: a variant of its own, since following the K tiles cost a K tail of whole chunks
+  // up to a tenth of its time (us without / with: bf16 NN 624 x 256 x 4176 25.5 / 27.6, NT
+  // 968 x 160 x 1320 14.1 / 14.9; fp32 NT 65 x 3209 x 2520 45.3 / 50.1)
+  constexpr bool STRADDLE = (VAR & DLDS_STRADDLE) != 0;
   constexpr bool FAST_EPI = (VAR & DLDS_FAST_EPI) != 0;
   // ROWSCALE: the direct epilogue multiplies row m by p.row_scale[m] (a folded RMSNorm);
   // a variant of its own, so that the plain GEMMs carry no row-scale code (+0.45 % on the
@@ -506,7 +511,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
   const int tail_kt = tail_nv ? kt_seg - 1 - klo : -1;
   auto zero_tail = [&](auto J_c) __attribute__((always_inline)) {
     constexpr int J = decltype(J_c)::value;
-    if constexpr (KTAIL) {
+    if constexpr (STRADDLE) {
       if (c_kt == tail_kt) {
         const int c = (p.K - (kt_seg - 1) * BK) / EPC;
         if constexpr (AK) oa.template zero_tail<J>(lds0 + A_REG, c, tail_nv);

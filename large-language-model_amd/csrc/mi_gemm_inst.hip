@@ -17,9 +17,9 @@ typedef __bf16 elem_t;
 typedef float elem_t;
 #define MI_DTN f32
 #endif
-// ktail: the K extent of a segment is not a multiple of 64 (bf16 direct-to-LDS
-// kernels then mask K-contiguous chunks past the end); fast_epi: the problem
-// qualifies for the direct epilogue.
+// ktail: the K extent of a segment is not whole K tiles (direct-to-LDS kernels then mask
+// K-contiguous chunks past the end; 2: and zero the rest of a straddling chunk);
+// fast_epi: the problem qualifies for the direct epilogue.
 
 #ifndef MI_DLDS_BK
 #define MI_DLDS_BK 64
@@ -126,7 +126,7 @@ KernelFn dlds32_kernel(int cfg) {
 }
 #endif
 
-KernelFn MI_PICK_NAME(MI_DTN, MI_TA, MI_TB)(int cfg, bool fast, bool ktail, int fast_epi) {
+KernelFn MI_PICK_NAME(MI_DTN, MI_TA, MI_TB)(int cfg, bool fast, int ktail, int fast_epi) {
   constexpr bool AK = (MI_TA == 0);  // A is K-contiguous when not transposed
   constexpr bool BK = (MI_TB == 1);  // B is K-contiguous when transposed
 #if MI_DT_BF16
@@ -147,6 +147,7 @@ KernelFn MI_PICK_NAME(MI_DTN, MI_TA, MI_TB)(int cfg, bool fast, bool ktail, int 
     // K-tail variants exist only where an operand is K-contiguous; a K tail
     // takes the general epilogue.
     if constexpr (AK || BK) {
+      if (ktail == 2) return MI_DLDS(DLDS_KTAIL | DLDS_STRADDLE);
       if (ktail) return MI_DLDS(DLDS_KTAIL);
     }
 #if MI_DT_BF16

@@ -59,11 +59,11 @@ inline CfgShape cfg_shape(bool bf16, int cfg) {
 // the fast (buffer-load) or the element-granular loader, or nullptr when the
 // combination does not exist (prologue with transA = 1).  The element-granular
 // variant of the plain configurations exists only for CFG_S.  ktail: the K
-// extent is not a multiple of 64; fast_epi: the epilogue is alpha (SiLU
+// extent is not whole K tiles (2: nor whole 16-byte chunks of a K-contiguous operand); fast_epi: the epilogue is alpha (SiLU
 // gate), beta*C and the output conversion only, with no split-K (1: on whole 32x32
 // blocks, 2: and the row scale, 3: with blocks cut by the matrix edge).
 #define MI_DECL_PICK(dt, ta, tb) \
-  KernelFn pick_##dt##_##ta##tb(int cfg, bool fast, bool ktail, int fast_epi);
+  KernelFn pick_##dt##_##ta##tb(int cfg, bool fast, int ktail, int fast_epi);
 MI_DECL_PICK(bf16, 0, 0)
 MI_DECL_PICK(bf16, 0, 1)
 MI_DECL_PICK(bf16, 1, 0)

@@ -6,6 +6,8 @@ max|y - ref| / max|ref|). Small integers give bit-exact expectations. Full-size
 benchmark configurations are checked on sampled rows against the oracle and on
 every element through row/column checksums.
 """
+import itertools
+
 import numpy as np
 import pytest
 
@@ -843,3 +845,38 @@ def test_causal_output_mask(mi, dev, bf16, T, N):
         ref = (a.double() @ b.double() + 2.0 * beta)
         ref.masked_fill_(torch.ones(T, N, dtype=torch.bool, device=dev).triu_(1), -7.0)
         assert torch.equal(C, ref.to(dt)), (T, N, beta)
+
+
+@pytest.mark.parametrize("tB", [0, 1], ids=["NN", "NT+TT"])
+@pytest.mark.parametrize("bf16,dual,M,N", [
+    (True, 0, 300, 264), (True, 0, 2047, 2052), (True, 0, 4095, 4092), (True, 1, 130, 2052), (True, 1, 1000, 2816),
+    (False, 0, 300, 260), (False, 0, 2047, 1540), (False, 1, 155, 772)])
+def test_k_tails(mi, dev, bf16, dual, M, N, tB):
+    """K ends inside a K tile, on a 16-byte chunk and inside one (the direct-to-LDS kernels' two
+    tail variants), plain and dual, with NaN in the gap after each operand row. Plain: integer
+    products, bit for bit."""
+    import torch
+
+    dt = torch.bfloat16 if bf16 else torch.float32
+    g = torch.Generator(device=dev).manual_seed(M + N + tB)
+    ws = torch.full((8 << 20,), float("nan"), dtype=torch.float32, device=dev)
+
+    def place(m, trans):  # rows `gap` elements apart, NaN between them
+        m = m.T if trans else m
+        buf = torch.full((m.shape[0], m.shape[1] + 2 + m.shape[1] % 2), float("nan"), dtype=dt, device=dev)
+        buf[:, :m.shape[1]] = m
+        return buf, buf.shape[1]
+
+    for K, tA in itertools.product((328, 330, 70) if bf16 else (108, 110, 333), (0, 1) if tB and not dual else (0,)):
+        a = torch.randint(-2, 3, (M, K), generator=g, device=dev)
+        bs = [torch.randint(-2, 3, (K, N), generator=g, device=dev) for _ in range(1 + dual)]
+        (A, lda), B = place(a, tA), [place(b, tB) for b in bs]
+        C = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+        s = 1.0 / 64 if dual else 1.0
+        mi.gemm(A, B[0][0], C, M, N, K, transA=bool(tA), transB=bool(tB), lda=lda, ldb=B[0][1], alpha=s,
+                B2=B[1][0] if dual else None, workspace=ws)
+        ref = [s * (a.double() @ b.double()) for b in bs]
+        if dual:
+            check(host(C), host(torch.nn.functional.silu(ref[0]) * ref[1]), _tol(bf16), f"dual {M}x{N}x{K}")
+        else:
+            assert torch.equal(C, ref[0].float()), (K, tA)
