@@ -302,10 +302,13 @@ enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4, DLDS_EDGE = 8, DLDS
 // groups share the stage's DMA), so a workgroup keeps two waves per SIMD on one
 // output tile; the groups' accumulators are summed through LDS before the
 // epilogue, each group then storing half of the tile.
+// waves_per_eu of fp32: with 3 or more waves a SIMD a wave has at most 168 registers, and the
+// compiler keeps the accumulators in VGPRs, where their sum and the epilogue read them
+// (no kernel needs more than 144; accumulation registers have to be copied out first).
 template <int BM, int BN, int BK, int STAGES, bool AK, bool BKC, int MODE, int VAR, int WGM = 2,
           int WGN = 2, int KG = 1, int ES = 2>
 __global__ void __launch_bounds__(64 * WGM * WGN * KG)
-    __attribute__((amdgpu_waves_per_eu(WGM * WGN * KG / 4)))
+    __attribute__((amdgpu_waves_per_eu(ES == 4 ? 3 : WGM * WGN * KG / 4)))
     gemm_dlds_kernel(Params p) {
   constexpr bool KTAIL = (VAR & DLDS_KTAIL) != 0;
   // STRADDLE: a variant of its own, since following the K tiles cost a K tail of whole chunks
@@ -420,10 +423,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
   // fp32: every other MFMA of a fragment pair sums into accumulators of its own, joined at
   // the end: each rounding chain is half as long, as if K were split in two, which keeps the
-  // products that the planner no longer splits as close to their 64-bit values as before.
-  // The registers are there: LDS bounds the workgroups per CU (5 of 64x64, 3 of 64x128).
-  // Error against 64 bits: training block on 2048 tokens 8.1e-7 -> 5.7e-7, the materialised
-  // attention 5.6e-7 -> 4.0e-7; their times 771 -> 779 us, and 162 -> 162-164.
+  // products that the planner splits less than it could as close to their 64-bit values as
+  // the split would.  LDS bounds the workgroups per CU (5 of 64x64, 3 of 64x128), so the
+  // registers are there; held in VGPRs (waves_per_eu above) they cost no time, where moving
+  // both sets out of accumulation registers at a tile's end cost 1.5 % (training block on 2048
+  // tokens 771-779 us; here 776, one set 776).  Error against 64 bits: that block 8.1e-7 ->
+  // 5.7e-7, the materialised attention 5.6e-7 -> 4.0e-7.
   f32x16_t acc_odd[ES == 4 ? TM : 1][ES == 4 ? NB : 1];
   if constexpr (ES == 4) {
 #pragma unroll
