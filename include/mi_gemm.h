@@ -104,9 +104,7 @@ const char* mi_last_error(void);
 const char* mi_version(void);
 
 /* Workspace bytes mi_gemm / mi_gemm_batched would use for split-K on this
- * problem when given unlimited workspace.  Without a split it is 0, or 256 where a
- * single problem's K is not whole 16-byte chunks of a K-contiguous operand: any
- * workspace then selects the direct-to-LDS kernels (no byte of it is written). */
+ * problem when given unlimited workspace (0 if it would not split). */
 size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int64_t K,
                               int32_t dtype_in, int32_t dtype_c, int64_t batch);
 
@@ -409,7 +407,6 @@ int mi_convert_matrices(void* stream, const mi_convert_job* jobs, int64_t n);
  * Describe the kernel mi_gemm_batched would launch for this problem (tile,
  * loader, split-K factor) as text into buf (always NUL-terminated), for packed
  * operands (leading dimension = contiguous extent) at 16-byte-aligned addresses.
- * workspace_bytes > 0 also counts as "a workspace is given" for the loader choice.
  * For measurement and logging; no reference counterpart.  epi_mode: 0 plain,
  * 1 dual-B, 2 SiLU-gate prologue.
  */

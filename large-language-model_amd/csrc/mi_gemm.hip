@@ -468,15 +468,6 @@ bool rows_overlap(const void* a, const void* b, int64_t bytes) {
   return a0 < b0 + (uintptr_t)bytes && b0 < a0 + (uintptr_t)bytes;
 }
 
-// Whether the direct-to-LDS kernels take this K without a workspace: a K-contiguous
-// operand whose K is not whole 16-byte chunks has a straddling chunk to zero.  Without a
-// workspace such a single problem keeps the register-staged kernel, the plan that
-// mi_gemm_describe reports for it; with one, and in a batch, it takes the direct-to-LDS
-// kernels (fp32 forward, dX and dW of 1500 x 1343 x 811 in us: 282 -> 141; 77 x 1343 x
-// 811: 92 -> 44; bf16 2000 x 3144 x 942, rows of whole dwords: 721 -> 87).
-constexpr size_t kTailWorkspace = 256;  // what mi_gemm_workspace_size asks for then, without a split
-bool tail_ok(int transA, int transB, int64_t K, int64_t ch) { return (transA && !transB) || K % ch == 0; }
-
 struct Problem {
   int transA, transB;
   int64_t M, N, K;
@@ -671,16 +662,17 @@ int run(const Problem& P, hipStream_t stream) {
   // The skinny and the direct-to-LDS kernels (every mode but the prologue) need no more than
   // 4-byte alignment: a buffer load's address and its bounds check work in dwords.  A
   // row-contiguous chunk that straddles the matrix edge feeds outputs that are
-  // not stored; a K-contiguous one is zeroed past K in LDS (tail_ok).
+  // not stored; a K-contiguous one is zeroed past K in LDS.  The register-staged kernels
+  // are left with odd bf16 rows, offsets past 31 bits and the prologue (forward, dX and dW
+  // of 1500 x 1343 x 811 fp32 in us: 282 there, 141 here; without a workspace 1146 x 112 x
+  // 2226 NT: 192, 43; bf16 2000 x 3144 x 942, rows of whole dwords: 721, 87).
   auto dw = [&](const void* q, int64_t ld, int64_t o, int64_t i, int64_t sg) {
     return ((uintptr_t)q & 3u) == 0 && (esz == 4 || (ld % 2 == 0 && o % 2 == 0 && i % 2 == 0 && sg % 2 == 0));
   };
   const bool dwords = spanA && spanB && dw(P.A, P.lda, b.a_outer, b.a_inner, b.seg_a) &&
                       dw(P.B, P.ldb, b.b_outer, b.b_inner, b.seg_b) && (!P.ep.B2 || ((uintptr_t)P.ep.B2 & 3u) == 0);
-  const bool dlds = mode != MODE_PROLOGUE;
   const bool fast = (vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB) ||
-                    (dwords && dlds &&
-                     (tail_ok(P.transA, P.transB, P.K, CH) || b.batch > 1 || (P.ws && P.ws_bytes > 0)));
+                    (dwords && mode != MODE_PROLOGUE);
   const bool skinny = dwords && skinny_fits(P.transA, P.transB, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode, CH);
 
   // SiLU-gate prologue as its own pass when the workspace holds SiLU(A) * A2 (bf16,
@@ -1097,8 +1089,7 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
     const SkinnyPlan sk = skinny_plan(dtype_in == MI_BF16, transB != 0, false, M, N, K, INT64_MAX / 8);
     if (sk.splits > 1) need = std::max(need, (size_t)sk.splits * (size_t)M * (size_t)N * sizeof(float));
   }
-  if (need) return need;
-  return batch == 1 && !tail_ok(transA, transB, K, ch) ? kTailWorkspace : 0;
+  return need;
 }
 
 int mi_gemm(void* stream, int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
@@ -1801,11 +1792,9 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   // whole dwords
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
-  const bool dlds = mode != MODE_PROLOGUE;
   const int64_t dw = dtype_in == MI_BF16 ? 2 : 1;
   const bool dwords = a_contig % dw == 0 && b_contig % dw == 0;
-  const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) ||
-                    (dwords && dlds && (tail_ok(transA, transB, K, ch) || batch > 1 || ws > 0));
+  const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) || (dwords && mode != MODE_PROLOGUE);
   const Plan pl = (K == 0 || dwords) && skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
                       ? skinny_as_plan(skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws))
                       : make_plan(dtype_in, !transA && transB, M, N, K, batch, mode, ws > 0, ws, cus, fast);

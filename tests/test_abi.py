@@ -288,8 +288,24 @@ def test_block_plans(mi):
     }
     for (M, N, K, tA, tB), w in want2.items():
         assert mi.describe(tA, tB, M, N, K, mi.MI_F32, workspace_bytes=ws).startswith(w), (M, N, K, tA, tB)
-    # unaligned fp32 operands (odd K) take the register-staged 128x128 tiles
-    assert mi.describe(0, 0, 1000, 600, 333, mi.MI_F32).startswith("regstage f32 128x128")
+    # odd bf16 rows (not whole dwords) take the register-staged 128x128 tiles
+    assert mi.describe(0, 0, 1000, 600, 333, mi.MI_BF16).startswith("regstage bf16 128x128")
+
+
+@pytest.mark.parametrize("dt,M,N,K", [("f32", 1000, 600, 333), ("f32", 584, 475, 2137), ("f32", 1848, 490, 950),
+                                      ("bf16", 2000, 3144, 942)])
+def test_loader_follows_alignment(mi, dt, M, N, K):
+    """The loader follows the operands' alignment and never whether a workspace is given: rows of
+    whole dwords take the direct-to-LDS kernels, also where the end of K cuts a 16-byte chunk
+    (fp32 without a workspace, register-staged and so: 1146 x 112 x 2226 NT 192 and 43 us, 10 x
+    766 x 1606 NN 153 and 30, 60 x 2594 x 1435 NN 141 and 28)."""
+    dti = mi.MI_F32 if dt == "f32" else mi.MI_BF16
+    for tB in (0, 1):
+        for ws in (0, 64 << 20):
+            assert mi.describe(0, tB, M, N, K, dti, workspace_bytes=ws).startswith("dlds"), (tB, ws)
+        assert mi.describe(0, tB, M, N, K, dti, epi_mode=1).startswith("dlds")
+        need = mi.workspace_size(0, tB, M, N, K, dti, dti)
+        assert need == 0 or need >= 4 * M * N * 2  # partials or nothing
 
 
 def test_cross_entropy_validation(mi):
