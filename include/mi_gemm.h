@@ -104,7 +104,10 @@ const char* mi_last_error(void);
 const char* mi_version(void);
 
 /* Workspace bytes mi_gemm / mi_gemm_batched would use for split-K on this
- * problem when given unlimited workspace (0 if it would not split). */
+ * problem when given unlimited workspace, for packed operands (0 if it would not
+ * split).  bf16 operands whose leading dimensions or addresses are not whole dwords where
+ * their packed rows would be run another kernel, which may split more than this holds: it
+ * then splits as far as the workspace goes. */
 size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int64_t K,
                               int32_t dtype_in, int32_t dtype_c, int64_t batch);
 

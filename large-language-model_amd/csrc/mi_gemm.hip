@@ -226,9 +226,9 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 //     split below 5/8 of a wave (element-granular loader); the rules at the fp32
 //     branch.
 // Every split fits the workspace: splits * M * N * batch <= ws_limit_elems.
-// nt: B is K-contiguous and A too (transB without transA).
-Plan make_plan(int dtype_in, bool nt, int64_t M, int64_t N, int64_t Ktot, int64_t batch, int mode,
-               bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
+Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64_t Ktot, int64_t batch,
+               int mode, bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
+  const bool nt = !transA && transB, tn = transA && !transB;
   auto plan_for = [&](int cfg, int sp) {
     const CfgShape s = shape_of(dtype_in, cfg);
     return Plan{cfg, sp, (int)cdiv(M, s.bm), (int)cdiv(N, s.bn)};
@@ -320,7 +320,15 @@ Plan make_plan(int dtype_in, bool nt, int64_t M, int64_t N, int64_t Ktot, int64_
       }
       return plan_for(CFG_S, 1);
     }
-    return plan_for(CFG_S, split_of(tilesS, 32));
+    // The register-staged loader takes 1.5 us a K tile of 64, a split 5 us and its partials at
+    // 3 TB/s: NN and NT split where that is less (213 x 1368 x 1775 NN 61.8 us whole, split 7
+    // 39.9; 1694 x 1081 x 1213 NT 37.0, split 2 41.5).  TN always does: a weight gradient in
+    // fp32 keeps the shorter rounding chains (1304 x 479 x 1351: error against 64 bits 1.6e-7
+    // whole, 7.5e-8 split 5).
+    int sp = split_of(tilesS, 32);
+    const double kt = (double)cdiv(Ktot, 64);
+    if (!tn && 1.5 * kt <= 1.5 * kt / sp + 5.0 + 8.0 * (double)(sp * M * N * batch) / 3e6) sp = 1;
+    return plan_for(CFG_S, sp);
   }
   // fp32 with the direct-to-LDS kernel: 64x128 tiles (V; four waves of 32x64) or 64x64
   // tiles (M; four waves of 32x32), several workgroups per CU.  Score of a plan: the
@@ -400,6 +408,12 @@ bool skinny_fits(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_
 Plan skinny_as_plan(const SkinnyPlan& sk) { return Plan{CFG_SKINNY, sk.splits, sk.blocks, sk.strips}; }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+// Whether packed rows (leading dimension = contiguous extent) are whole dwords, as the
+// direct-to-LDS and the few-row kernels want them.
+bool packed_dwords(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64_t K) {
+  return dtype_in != MI_BF16 || ((transA ? M : K) % 2 == 0 && (transB ? K : N) % 2 == 0);
+}
 
 // Text of a plan, as mi_gemm_describe and the profiler records show it.
 void describe_plan(char* buf, size_t len, int dtype_in, bool fast, const Plan& pl, int transA,
@@ -715,8 +729,8 @@ int run(const Problem& P, hipStream_t stream) {
   const SkinnyPlan sk = skinny_plan(P.dtype_in == MI_BF16, P.transB != 0, mode == MODE_DUAL, P.M, P.N, P.K,
                                     allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0);
   Plan plan = skinny ? skinny_as_plan(sk)
-                     : make_plan(P.dtype_in, !P.transA && P.transB, P.M, P.N, Ktot, b.batch, mode, allow_split || P.noalloc,
-                                 P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
+                     : make_plan(P.dtype_in, P.transA, P.transB, P.M, P.N, Ktot, b.batch, mode,
+                                 allow_split || P.noalloc, P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
   if (P.noalloc && plan.splits > 1 && (int64_t)plan.splits * P.M * P.N * b.batch > ws_elems)
     return fail(MI_ERR_WORKSPACE,
                 "mi_gemm_noalloc: split-K by %d needs %lld bytes of scratch, above its %lld-byte "
@@ -1081,13 +1095,22 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
   int cus = 256;
   if (init_devices() == MI_OK) cus = current_cus();
-  const Plan pl = make_plan(dtype_in, !transA && transB, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, true);
-  size_t need = pl.splits > 1 ? (size_t)pl.splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float) : 0;
+  size_t need = 0;
+  auto cover = [&](int splits) {
+    if (splits > 1) need = std::max(need, (size_t)splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float));
+  };
+  auto tile_splits = [&](bool fast) {
+    return make_plan(dtype_in, transA, transB, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, fast).splits;
+  };
+  cover(tile_splits(true));
+  // odd bf16 rows: the register-staged kernel's plan, whose splits matter more (us without room
+  // for them and with it: TN 1263 x 528 x 1710 93 and 42, 121 x 2036 x 1362 71 and 36; NN
+  // 337 x 1593 x 1659 69 and 39)
+  if (!packed_dwords(dtype_in, transA, transB, M, N, K)) cover(tile_splits(false));
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
   if (skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, MODE_PLAIN, ch)) {
     // operands that rule the skinny kernels out take the tile plan, so room for either
-    const SkinnyPlan sk = skinny_plan(dtype_in == MI_BF16, transB != 0, false, M, N, K, INT64_MAX / 8);
-    if (sk.splits > 1) need = std::max(need, (size_t)sk.splits * (size_t)M * (size_t)N * sizeof(float));
+    cover(skinny_plan(dtype_in == MI_BF16, transB != 0, false, M, N, K, INT64_MAX / 8).splits);
   }
   return need;
 }
@@ -1330,7 +1353,7 @@ int mi_flash_attn_bwd_scaled(void* stream, const void* Q, const void* K, const v
     // Causal skipping in the dQ GEMM works on whole K tiles up to the end of a
     // 128-row output tile; the dK/dV kernel writes dS^T (zeros included) for every
     // key below that bound, and not beyond it, so taller tiles take the dQ kernel.
-    const Plan pl = make_plan(MI_BF16, false, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN, false, 0,
+    const Plan pl = make_plan(MI_BF16, 1, 0, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN, false, 0,
                               current_cus(), true);
     if (shape_of(MI_BF16, pl.cfg).bm != 128) p.dsT = nullptr;
   }
@@ -1792,12 +1815,11 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   // whole dwords
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
-  const int64_t dw = dtype_in == MI_BF16 ? 2 : 1;
-  const bool dwords = a_contig % dw == 0 && b_contig % dw == 0;
+  const bool dwords = packed_dwords(dtype_in, transA, transB, M, N, K);
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) || (dwords && mode != MODE_PROLOGUE);
   const Plan pl = (K == 0 || dwords) && skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
                       ? skinny_as_plan(skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws))
-                      : make_plan(dtype_in, !transA && transB, M, N, K, batch, mode, ws > 0, ws, cus, fast);
+                      : make_plan(dtype_in, transA, transB, M, N, K, batch, mode, ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

@@ -308,6 +308,21 @@ def test_loader_follows_alignment(mi, dt, M, N, K):
         assert need == 0 or need >= 4 * M * N * 2  # partials or nothing
 
 
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)], ids=["NN", "NT", "TN", "TT"])
+def test_workspace_covers_odd_rows(mi, tA, tB):
+    """mi_gemm_workspace_size holds the partials of the plan that packed odd bf16 rows get (the
+    register-staged kernel's, not the direct-to-LDS kernels'), so that they split with it as
+    with more."""
+    split = 0
+    for M, N, K in [(500, 941, 1023), (213, 1367, 1775), (779, 753, 1677), (63, 129, 831), (28, 1217, 1127),
+                    (501, 940, 1024), (1, 1, 100001)]:
+        full = mi.workspace_size(tA, tB, M, N, K, mi.MI_BF16, mi.MI_F32)
+        plan = mi.describe(tA, tB, M, N, K, mi.MI_BF16, workspace_bytes=1 << 34)
+        assert mi.describe(tA, tB, M, N, K, mi.MI_BF16, workspace_bytes=full) == plan, (M, N, K, plan)
+        split = max(split, _planned_split(mi, tA, tB, M, N, K, mi.MI_BF16, 1, 0, full))
+    assert split >= 4
+
+
 def test_cross_entropy_validation(mi):
     # mi_cross_entropy rejects bad arguments before any device work.
     lib = mi.load_library()
