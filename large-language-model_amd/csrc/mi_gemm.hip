@@ -228,7 +228,7 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Every split fits the workspace: splits * M * N * batch <= ws_limit_elems.
 Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64_t Ktot, int64_t batch,
                int mode, bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
-  const bool nt = !transA && transB, tn = transA && !transB;
+  const bool tn = transA && !transB;
   auto plan_for = [&](int cfg, int sp) {
     const CfgShape s = shape_of(dtype_in, cfg);
     return Plan{cfg, sp, (int)cdiv(M, s.bm), (int)cdiv(N, s.bn)};
@@ -343,11 +343,14 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
   // qkv dW 768x2304x2048 64x64 113 vs 64x128 102; o forward 2048x768x768 64x128 93 vs
   // 64x64 87; gate forward 2048x2048x768 64x128 127 vs 64x64 122.  The rule picks the
   // best plan of every one of the 12, or one within 2 %.
-  // The score of an NN or TN plan is its time in us: the busiest CU's MFMAs at 2.1 GHz, and
-  // split 4 us for the second launch and the partials at 3 TB/s, which the share alone
-  // leaves out (768 x 768 x 512 TN: 64x64 12.4, 64x128 split 3 17.9; 512 x 768 x 768 NN: 15.9,
-  // 64x128 split 5 18.5; 200 x 2304 x 768 NN: 16.9, 64x128 split 3 19.0).  NT keeps the
-  // share: its small plans are in the pinned planner table.
+  // That share decides how many rounding chains K is summed in, and leaves out what a split
+  // costs: among the plans with as many chains (two in a workgroup, see gemm_dlds_kernel, so at
+  // least half of its splits) the one with the least time runs, in us the busiest CU's MFMAs at
+  // 2.1 GHz, and split 2.5 for the second launch and the partials at 3 TB/s.  2061 products of
+  // 40-2048 rows: 0.9 % faster than the share's plan and never more than 5 % slower, error
+  // against 64 bits no larger; without the bound on the chains 1.2 %, but up to 9 % slower and
+  // an error up to 2.2 times as large (256 x 3180 x 4288 NN: 64x128 split 5 64.6 us, 3.7e-7;
+  // 64x64 whole 72, 5.8e-7).
   // Batched products (the attention's, short K or causally cut) take 64x64 tiles:
   // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304.
   // The element-granular loader (any alignment) runs 128x128 tiles (S): below 5/8
@@ -356,28 +359,31 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
   // tiles at K = 2048: splits 1..8 ran 43 71 59 74 83 66 69 76 TFLOP/s; 108 tiles:
   // 47 78 67 83 65 73 76 71; 36 tiles: 16 28 37 44 49 52 54 41).
   if (fast) {
-    int best_cfg = CFG_M, best_sp = 1;
-    double best_score = 1e300;
-    for (int cfg : {CFG_V, CFG_M}) {
-      if (cfg == CFG_V && batch > 1) continue;
-      const CfgShape t = shape_of(dtype_in, cfg);
-      const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
-      for (int sp = 1; sp <= (allow_split ? 8 : 1); ++sp) {
-        const int64_t units = tiles * sp;
-        if (sp > 1) {
-          if (units > 3 * (int64_t)cus || (int64_t)sp * M * N * batch > ws_limit_elems) continue;
-          if (Ktot < (units > cus ? 512 : 128) * (int64_t)sp) continue;
+    int best_cfg = CFG_M, best_sp = 1, least_sp = 1;
+    for (const bool timed : {false, true}) {
+      double best_score = 1e300;
+      for (int cfg : {CFG_V, CFG_M}) {
+        if (cfg == CFG_V && batch > 1) continue;
+        const CfgShape t = shape_of(dtype_in, cfg);
+        const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
+        for (int sp = least_sp; sp <= (allow_split ? 8 : 1); ++sp) {
+          const int64_t units = tiles * sp;
+          if (sp > 1) {
+            if (units > 3 * (int64_t)cus || (int64_t)sp * M * N * batch > ws_limit_elems) continue;
+            if (Ktot < (units > cus ? 512 : 128) * (int64_t)sp) continue;
+          }
+          double score = (double)cdiv(units, cus) * t.bm * t.bn / sp;
+          if (timed) {
+            score *= (double)Ktot / (128 * 2100.0);
+            if (sp > 1) score += 2.5 + 8.0 * (double)(sp * M * N * batch) / 3e6;
+          }
+          const bool wins = score < best_score ||
+                            (score == best_score &&
+                             (sp < best_sp || (sp == best_sp && cfg == (Ktot < 1024 ? CFG_V : CFG_M))));
+          if (wins) best_cfg = cfg, best_sp = sp, best_score = score;
         }
-        double score = (double)cdiv(units, cus) * t.bm * t.bn / sp;
-        if (!nt) {
-          score *= (double)Ktot / (128 * 2100.0);
-          if (sp > 1) score += 4.0 + 8.0 * (double)(sp * M * N * batch) / 3e6;
-        }
-        const bool wins = score < best_score ||
-                          (score == best_score &&
-                           (sp < best_sp || (sp == best_sp && cfg == (Ktot < 1024 ? CFG_V : CFG_M))));
-        if (wins) best_cfg = cfg, best_sp = sp, best_score = score;
       }
+      least_sp = (best_sp + 1) / 2;
     }
     return plan_for(best_cfg, best_sp);
   }

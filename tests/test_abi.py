@@ -2,10 +2,12 @@
 and validates arguments (status codes and messages) without touching a GPU.
 Also the host-side shape rules of the Tensor::matmul mirror (Tensor.cpp:174-209)."""
 import ctypes
+import math
 import os
 import re
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -306,6 +308,38 @@ def test_loader_follows_alignment(mi, dt, M, N, K):
         assert mi.describe(0, tB, M, N, K, dti, epi_mode=1).startswith("dlds")
         need = mi.workspace_size(0, tB, M, N, K, dti, dti)
         assert need == 0 or need >= 4 * M * N * 2  # partials or nothing
+
+
+def test_fp32_plans_keep_their_chains(mi):
+    """The fp32 planner sums K in as many rounding chains (splits x the two of a workgroup) as the
+    plan that shares the work most evenly among the CUs splits it into, so that a quicker plan is
+    never a less accurate one; and it plans NN, NT and TN alike."""
+    cus, deeper = 256, 0
+
+    def even_split(M, N, K):
+        best = (math.inf, 0, 0, 0)
+        for bm, bn in ((64, 128), (64, 64)):
+            tiles = -(-M // bm) * -(-N // bn)
+            for sp in range(1, 9):
+                units = tiles * sp
+                if sp > 1 and (units > 3 * cus or K < (512 if units > cus else 128) * sp):
+                    continue
+                tie = (bn == 64) if K < 1024 else (bn == 128)
+                best = min(best, (-(-units // cus) * bm * bn / sp, sp, tie, bn))
+        return best[1]
+
+    rng = np.random.default_rng(11)
+    shapes = [(256, 3180, 4288), (448, 64, 384), (1664, 392, 2184), (512, 768, 768), (1134, 83, 419)]
+    shapes += [tuple(int(x) for x in np.exp(rng.uniform(np.log(65), np.log(4096), 3))) for _ in range(300)]
+    for M, N, K in shapes:
+        texts = [mi.describe(tA, tB, M, N, K, mi.MI_F32, workspace_bytes=1 << 34) for tA, tB in ((0, 0), (0, 1), (1, 0))]
+        assert texts[1].replace("NT", "TN") == texts[2], (M, N, K, texts)
+        if not texts[0].startswith("skinny"):
+            assert texts[0].replace("NN", "TN") == texts[2], (M, N, K, texts)
+        need = even_split(M, N, K)
+        assert 2 * int(re.search(r"split(\d+)", texts[2]).group(1)) >= need, (M, N, K, texts[2], need)
+        deeper += need > 2
+    assert deeper > 50
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)], ids=["NN", "NT", "TN", "TT"])
