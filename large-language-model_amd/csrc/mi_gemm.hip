@@ -359,17 +359,19 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
   // tiles at K = 2048: splits 1..8 ran 43 71 59 74 83 66 69 76 TFLOP/s; 108 tiles:
   // 47 78 67 83 65 73 76 71; 36 tiles: 16 28 37 44 49 52 54 41).
   if (fast) {
-    int best_cfg = CFG_M, best_sp = 1, least_sp = 1;
-    for (const bool timed : {false, true}) {
+    int best_cfg = CFG_M, best_sp = 1;
+    // the best plan of at least `least` splits by its time, else by its share; false if the
+    // workspace (of the timed pass) holds none
+    auto search = [&](bool timed, int least) {
       double best_score = 1e300;
       for (int cfg : {CFG_V, CFG_M}) {
         if (cfg == CFG_V && batch > 1) continue;
         const CfgShape t = shape_of(dtype_in, cfg);
         const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
-        for (int sp = least_sp; sp <= (allow_split ? 8 : 1); ++sp) {
+        for (int sp = least; sp <= (allow_split ? 8 : 1); ++sp) {
           const int64_t units = tiles * sp;
           if (sp > 1) {
-            if (units > 3 * (int64_t)cus || (int64_t)sp * M * N * batch > ws_limit_elems) continue;
+            if (units > 3 * (int64_t)cus || (timed && (int64_t)sp * M * N * batch > ws_limit_elems)) continue;
             if (Ktot < (units > cus ? 512 : 128) * (int64_t)sp) continue;
           }
           double score = (double)cdiv(units, cus) * t.bm * t.bn / sp;
@@ -383,8 +385,10 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
           if (wins) best_cfg = cfg, best_sp = sp, best_score = score;
         }
       }
-      least_sp = (best_sp + 1) / 2;
-    }
+      return best_score < 1e300;
+    };
+    search(false, 1);
+    for (int least = (best_sp + 1) / 2; !search(true, least); --least) {}
     return plan_for(best_cfg, best_sp);
   }
   if (tilesS * 8 >= (int64_t)cus * 5 || !allow_split) return plan_for(CFG_S, 1);

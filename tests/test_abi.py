@@ -329,7 +329,8 @@ def test_fp32_plans_keep_their_chains(mi):
         return best[1]
 
     rng = np.random.default_rng(11)
-    shapes = [(256, 3180, 4288), (448, 64, 384), (1664, 392, 2184), (512, 768, 768), (1134, 83, 419)]
+    shapes = [(256, 3180, 4288), (448, 64, 384), (1664, 392, 2184), (512, 768, 768), (1134, 83, 419),
+              (250, 1134, 941), (127, 3176, 640), (2169, 114, 907)]
     shapes += [tuple(int(x) for x in np.exp(rng.uniform(np.log(65), np.log(4096), 3))) for _ in range(300)]
     for M, N, K in shapes:
         texts = [mi.describe(tA, tB, M, N, K, mi.MI_F32, workspace_bytes=1 << 34) for tA, tB in ((0, 0), (0, 1), (1, 0))]
@@ -338,6 +339,8 @@ def test_fp32_plans_keep_their_chains(mi):
             assert texts[0].replace("NN", "TN") == texts[2], (M, N, K, texts)
         need = even_split(M, N, K)
         assert 2 * int(re.search(r"split(\d+)", texts[2]).group(1)) >= need, (M, N, K, texts[2], need)
+        own = mi.workspace_size(1, 0, M, N, K, mi.MI_F32, mi.MI_F32)  # no room beyond the plan's own partials
+        assert mi.describe(1, 0, M, N, K, mi.MI_F32, workspace_bytes=own) == texts[2], (M, N, K, own)
         deeper += need > 2
     assert deeper > 50
 
