@@ -409,7 +409,8 @@ int mi_convert_matrices(void* stream, const mi_convert_job* jobs, int64_t n);
 /*
  * Describe the kernel mi_gemm_batched would launch for this problem (tile,
  * loader, split-K factor) as text into buf (always NUL-terminated), for packed
- * operands (leading dimension = contiguous extent) at 16-byte-aligned addresses.
+ * operands (leading dimension = contiguous extent) at 16-byte-aligned addresses, no
+ * bias or residual, and C of the input type, or fp32 where only A is transposed.
  * For measurement and logging; no reference counterpart.  epi_mode: 0 plain,
  * 1 dual-B, 2 SiLU-gate prologue.
  */

@@ -203,6 +203,14 @@ struct Plan {
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Epilogue of an unsplit product: 1 direct on whole 32x32 blocks, 3 direct with cut or causally
+// masked blocks in quads of columns, 0 general.  plain_c: no bias or residual, C in aligned
+// quads; K-contiguous operands with a K tail have the general epilogue only.
+int direct_kind(int transA, int transB, int64_t M, int64_t N, int64_t K, bool plain_c, bool masked) {
+  if (!plain_c || ((!transA || transB) && K % 64 != 0)) return 0;
+  return M % 32 == 0 && N % 32 == 0 && !masked ? 1 : N % 4 == 0 ? 3 : 0;
+}
+
 // Tile and split choice.  Rules fitted to forced-plan sweeps of the decoder-block
 // and LM-head shapes on MI355X (TFLOP/s of bf16 256x256 "L" vs 128x128 "S" tiles,
 // split-K factor after the letter):
@@ -226,8 +234,9 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 //     split below 5/8 of a wave (element-granular loader); the rules at the fp32
 //     branch.
 // Every split fits the workspace: splits * M * N * batch <= ws_limit_elems.
-Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64_t Ktot, int64_t batch,
-               int mode, bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
+// direct: direct_kind of the problem.
+Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int64_t N, int64_t Ktot, int64_t batch,
+               int mode, int direct, bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
   const bool tn = transA && !transB;
   auto plan_for = [&](int cfg, int sp) {
     const CfgShape s = shape_of(dtype_in, cfg);
@@ -256,10 +265,11 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
   const double fillL = (double)(M * N * batch) / ((double)tilesL * L.bm * L.bn);
   const double fillS = (double)(M * N * batch) / ((double)tilesS * S.bm * S.bn);
   // split K until the units cover the CUs once; each split keeps >= 8 K tiles
-  // of 32 and its partials fit the workspace
-  auto split_of = [&](int64_t tiles, int kt) {
-    int sp = (int)std::min<int64_t>(cus / std::max<int64_t>(tiles, 1), 8);
-    while (sp > 1 && (cdiv(Ktot, kt) < 8 * sp || (int64_t)sp * M * N * batch > ws_limit_elems)) --sp;
+  // of 32 and (within) its partials fit the workspace
+  auto fits = [&](int sp) { return sp == 1 || (allow_split && (int64_t)sp * M * N * batch <= ws_limit_elems); };
+  auto split_of = [&](int64_t tiles, int kt, bool within) {
+    int sp = (int)std::max<int64_t>(1, std::min<int64_t>(cus / std::max<int64_t>(tiles, 1), 8));
+    while (sp > 1 && (cdiv(Ktot, kt) < 8 * sp || (within && !fits(sp)))) --sp;
     return sp;
   };
   if (dtype_in == MI_BF16) {
@@ -274,20 +284,29 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
       if (frac > 0.0 && frac <= 0.5 && tilesS >= cus) return plan_for(CFG_S, 1);
       return plan_for(CFG_L, 1);
     }
-    // Grids of S tiles that leave half the CUs idle (a quarter at short K): W tiles, whose two wave groups keep a
-    // lone workgroup's CU busy, split along K only where the shorter loop pays for the
-    // second launch and the partials.  Time in us of a plan: 7.5 + 0.36 per K tile of 64, and
-    // split 4.5 + the partials at 3 TB/s (500 x 768 x 2304 NT: W split 1 / 2 / 3 / 4 17.9 /
-    // 17.0 / 15.8 / 16.8, S split 8 18.9; 2000 x 768 x 2304: W 18.4, W split 2 22.9, S split 2
-    // 26.0; 768 x 2304 x 500 TN: W 11.5, S 11.5, S split 2 20.7; 500 x 2304 x 768: W 11.1, S
-    // split 3 19.4; 1000 x 2304 x 768, 144 tiles: W 11.7, S 13.0).
+    // Grids of S tiles that leave half the CUs idle (a quarter at short K).  W tiles, whose two
+    // wave groups keep a lone workgroup's CU busy and halve its epilogue, split along K only
+    // where the shorter loop pays for the second launch and the partials: time in us 0.42 per K
+    // tile of 64, and split 4 + the partials at 3 TB/s (500 x 768 x 2304 NT: W split 1 / 2 / 3 /
+    // 4 17.9 / 17.0 / 15.8 / 16.8, S split 8 18.9; 2000 x 768 x 2304: W 18.4, W split 2 22.9).
+    // A short K with the direct epilogue has neither to gain and runs S tiles, whose prologue
+    // is shorter.  Time of S over W by K under 128 tiles, inputs in the caches and rotating
+    // through HBM: whole blocks 0.82 and 0.81 at 64, 0.92 and 0.90 at 320, 0.93 and 1.00 at
+    // 640, 0.97 and 1.01 at 896, 1.06 and 1.08 at 1024 to 1216; cut blocks 0.91 up to 128, 1.02
+    // at 192; general epilogue 1.1 at 64.
+    // fp32 C: as many rounding chains (two in a W tile) as S tiles split to fill the CUs once.
     if (fast && (tilesS * 2 < cus || (Ktot < 1024 && tilesS * 4 <= 3 * cus))) {
+      const int even = tilesS * 2 < cus ? split_of(tilesS, 32, false) : 1;
+      const bool short_k = direct == 1 ? Ktot < 1024 : direct == 3 && Ktot <= 128;
+      if (short_k && (even == 1 || dtype_c != MI_F32)) return plan_for(CFG_S, 1);
+      int least = dtype_c == MI_F32 ? (even + 1) / 2 : 1;
+      while (!fits(least)) --least;
       const double kt = (double)cdiv(Ktot, 64);
-      int best = 1;
-      double best_t = 0.36 * kt;
-      for (int sp = 2; allow_split && sp <= std::min<int64_t>(8, cus / tilesS); ++sp) {
-        if (Ktot < 256 * (int64_t)sp || (int64_t)sp * M * N * batch > ws_limit_elems) continue;
-        const double t = 0.36 * kt / sp + 4.5 + 8.0 * (double)(sp * M * N * batch) / 3e6;
+      int best = least;
+      double best_t = 1e300;
+      for (int sp = least; sp <= std::min<int64_t>(8, cus / tilesS) && fits(sp); ++sp) {
+        if (Ktot < 256 * (int64_t)sp && sp > 1) break;
+        const double t = 0.42 * kt / sp + (sp > 1 ? 4.0 + 8.0 * (double)(sp * M * N * batch) / 3e6 : 0.0);
         if (t < best_t) best = sp, best_t = t;
       }
       return plan_for(CFG_W, best);
@@ -325,7 +344,7 @@ Plan make_plan(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64
     // 39.9; 1694 x 1081 x 1213 NT 37.0, split 2 41.5).  TN always does: a weight gradient in
     // fp32 keeps the shorter rounding chains (1304 x 479 x 1351: error against 64 bits 1.6e-7
     // whole, 7.5e-8 split 5).
-    int sp = split_of(tilesS, 32);
+    int sp = split_of(tilesS, 32, true);
     const double kt = (double)cdiv(Ktot, 64);
     if (!tn && 1.5 * kt <= 1.5 * kt / sp + 5.0 + 8.0 * (double)(sp * M * N * batch) / 3e6) sp = 1;
     return plan_for(CFG_S, sp);
@@ -738,8 +757,10 @@ int run(const Problem& P, hipStream_t stream) {
   // mi_gemm_noalloc runs it as mi_gemm does without a workspace
   const SkinnyPlan sk = skinny_plan(P.dtype_in == MI_BF16, P.transB != 0, mode == MODE_DUAL, P.M, P.N, P.K,
                                     allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0);
+  const bool masked = b.causal == MI_CAUSAL_OUT_LOWER;
+  const int direct = direct_kind(P.transA, P.transB, P.M, P.N, P.K, !P.ep.bias && !P.ep.residual && cvec, masked);
   Plan plan = skinny ? skinny_as_plan(sk)
-                     : make_plan(P.dtype_in, P.transA, P.transB, P.M, P.N, Ktot, b.batch, mode,
+                     : make_plan(P.dtype_in, P.dtype_c, P.transA, P.transB, P.M, P.N, Ktot, b.batch, mode, direct,
                                  allow_split || P.noalloc, P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
   if (P.noalloc && plan.splits > 1 && (int64_t)plan.splits * P.M * P.N * b.batch > ws_elems)
     return fail(MI_ERR_WORKSPACE,
@@ -756,7 +777,6 @@ int run(const Problem& P, hipStream_t stream) {
   // the direct epilogue: whole 32x32 blocks (those past M, N skipped), or cut or causally
   // masked ones in quads of columns (epi_kind 3)
   const bool whole = P.M % 32 == 0 && P.N % 32 == 0;
-  const bool masked = b.causal == MI_CAUSAL_OUT_LOWER;
   const bool fast_epi = plan.splits == 1 && !P.ep.bias && !P.ep.residual && cvec &&
                         ((whole && !masked) || (P.N % 4 == 0 && !P.ep.row_scale));
   const bool groups = plan.cfg == CFG_W || plan.cfg == CFG_V || plan.cfg == CFG_DUAL_W;
@@ -1101,7 +1121,6 @@ const char* mi_version(void) { return "mi_gemm 0.1 (gfx950)"; }
 
 size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int64_t K,
                               int32_t dtype_in, int32_t dtype_c, int64_t batch) {
-  (void)dtype_c;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return 0;
   int cus = 256;
   if (init_devices() == MI_OK) cus = current_cus();
@@ -1110,7 +1129,8 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
     if (splits > 1) need = std::max(need, (size_t)splits * (size_t)M * (size_t)N * (size_t)batch * sizeof(float));
   };
   auto tile_splits = [&](bool fast) {
-    return make_plan(dtype_in, transA, transB, M, N, K, batch, MODE_PLAIN, true, INT64_MAX / 8, cus, fast).splits;
+    return make_plan(dtype_in, dtype_c, transA, transB, M, N, K, batch, MODE_PLAIN,
+                     direct_kind(transA, transB, M, N, K, true, false), true, INT64_MAX / 8, cus, fast).splits;
   };
   cover(tile_splits(true));
   // odd bf16 rows: the register-staged kernel's plan, whose splits matter more (us without room
@@ -1363,8 +1383,8 @@ int mi_flash_attn_bwd_scaled(void* stream, const void* Q, const void* K, const v
     // Causal skipping in the dQ GEMM works on whole K tiles up to the end of a
     // 128-row output tile; the dK/dV kernel writes dS^T (zeros included) for every
     // key below that bound, and not beyond it, so taller tiles take the dQ kernel.
-    const Plan pl = make_plan(MI_BF16, 1, 0, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN, false, 0,
-                              current_cus(), true);
+    const Plan pl = make_plan(MI_BF16, MI_BF16, 1, 0, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN,
+                              direct_kind(1, 0, seq_len, head_dim, seq_len, true, false), false, 0, current_cus(), true);
     if (shape_of(MI_BF16, pl.cfg).bm != 128) p.dsT = nullptr;
   }
   hipError_t e = launch_flash_bwd(p, (int)head_dim, (hipStream_t)stream);
@@ -1829,7 +1849,8 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) || (dwords && mode != MODE_PROLOGUE);
   const Plan pl = (K == 0 || dwords) && skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
                       ? skinny_as_plan(skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws))
-                      : make_plan(dtype_in, transA, transB, M, N, K, batch, mode, ws > 0, ws, cus, fast);
+                      : make_plan(dtype_in, transA && !transB ? MI_F32 : dtype_in, transA, transB, M, N, K, batch, mode,
+                                  direct_kind(transA, transB, M, N, K, true, false), ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

@@ -345,6 +345,36 @@ def test_fp32_plans_keep_their_chains(mi):
     assert deeper > 50
 
 
+def test_bf16_plans_of_small_grids(mi):
+    """Under 128 tiles of 128x128: four-wave tiles at a short K with the direct epilogue, eight-wave
+    ones (kg2) past it; and weight gradients (TN, fp32) summed in as many chains (two in an
+    eight-wave tile) as tiles split to fill the CUs."""
+    for tA, tB, M, N, K, eight in [(0, 0, 128, 256, 64, 0), (0, 0, 576, 1856, 384, 0), (0, 1, 1504, 448, 128, 0),
+                                   (0, 0, 576, 1856, 1024, 1), (0, 0, 128, 896, 640, 0), (1, 0, 64, 4096, 128, 0), (1, 0, 320, 4672, 320, 0),
+                                   (1, 0, 320, 4672, 1024, 1), (1, 0, 100, 1216, 110, 0), (1, 0, 100, 1216, 192, 1),
+                                   (0, 0, 99, 1216, 192, 1), (0, 0, 128, 256, 72, 1)]:
+        text = mi.describe(tA, tB, M, N, K, mi.MI_BF16, workspace_bytes=1 << 34)
+        assert text.startswith("dlds-kg2 bf16 128x128" if eight else "dlds bf16 128x128"), (M, N, K, text)
+    rng = np.random.default_rng(12)
+    deeper = 0
+    shapes = [(32, 192, 640), (192, 768, 640), (64, 2368, 512)]
+    shapes += [[2 * int(x / 2) for x in np.exp(rng.uniform(np.log(65), np.log(4096), 3))] for _ in range(300)]
+    for M, N, K in shapes:
+        tiles = -(-M // 128) * -(-N // 128)
+        if tiles >= 128:
+            continue
+        even = max(1, min(256 // tiles, 8))
+        while even > 1 and -(-K // 32) < 8 * even:
+            even -= 1
+        text = mi.describe(1, 0, M, N, K, mi.MI_BF16, workspace_bytes=1 << 34)
+        chains = int(re.search(r"split(\d+)", text).group(1)) * (2 if text.startswith("dlds-kg2") else 1)
+        assert chains >= even, (M, N, K, text, even)
+        own = mi.workspace_size(1, 0, M, N, K, mi.MI_BF16, mi.MI_F32)
+        assert mi.describe(1, 0, M, N, K, mi.MI_BF16, workspace_bytes=own) == text, (M, N, K, own)
+        deeper += even > 2
+    assert deeper > 50
+
+
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)], ids=["NN", "NT", "TN", "TT"])
 def test_workspace_covers_odd_rows(mi, tA, tB):
     """mi_gemm_workspace_size holds the partials of the plan that packed odd bf16 rows get (the
