@@ -820,6 +820,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     static_assert(NWAVE * 32 * PP * 4 <= LDS_BYTES, "epilogue patches fit the ring");
     float* patch = reinterpret_cast<float*>(smem) + wave * (32 * PP);
     const float beta = p.beta;
+    // fp32 rows off 64-byte lines: a store fills lines in part, and the L2 has to merge them with
+    // the next block's, so it is not non-temporal (us, before / after: TN 3192 x 3544 x 4096
+    // 93.6 / 83.2, 4100 x 4100 x 512 with beta 75.6 / 61.7; NT 1771 x 4388 x 256 19.5 / 13.7)
+    const bool cut_lines = EDGE && (p.ldc & 15) != 0;
     // whether the quad of columns col of a row is inside a cut block
     auto in = [&](int row, int col) __attribute__((always_inline)) { return !EDGE || (row < p.M && col < p.N); };
     auto mask = [&](f32x4_t& v, int row, int col) __attribute__((always_inline)) {
@@ -948,7 +952,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
                 v[2] += beta * o[2]; v[3] += beta * o[3];
               }
               mask(v, (int)row0 + 8 * st, col);
-              __builtin_nontemporal_store(v, (f32x4_t*)((float*)Cz + ci));
+              if (cut_lines) *(f32x4_t*)((float*)Cz + ci) = v;
+              else __builtin_nontemporal_store(v, (f32x4_t*)((float*)Cz + ci));
             }
           }
           __builtin_amdgcn_sched_barrier(0);
