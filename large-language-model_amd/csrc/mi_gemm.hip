@@ -427,12 +427,13 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
 // Products of few rows with op(A) not transposed, in whole 16-byte chunks of K: the kernels
 // of mi_skinny.hip, which read B once at the rate HBM gives (a layer's products on 8 rows:
 // 128-row tiles split along K spent 99 us of which 45 in the dual product's 44 workgroups).
-bool skinny_fits(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t segs, int causal,
-                 int mode, int64_t ch) {
-  if (transA || K % ch != 0 || batch != 1 || segs != 1 || causal != MI_CAUSAL_NONE || mode == MODE_PROLOGUE) return false;
-  if (M <= 32) return true;
-  if (M <= SKINNY_MAX_M) return N * K * (16 / ch) <= SKINNY_WIDE_BYTES;
-  return skinny_blocks_fit(ch == 8, transB != 0, mode == MODE_DUAL, M, N, K);
+// dwords: the operands' rows are whole dwords.  The plan says whether to take them (.take).
+SkinnyPlan plan_skinny(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch,
+                       int64_t segs, int causal, int mode, bool dwords, int64_t ws_elems, int cus) {
+  const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
+  if (transA || K % ch != 0 || batch != 1 || segs != 1 || causal != MI_CAUSAL_NONE || mode == MODE_PROLOGUE || !dwords)
+    return SkinnyPlan{};
+  return skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws_elems, cus);
 }
 Plan skinny_as_plan(const SkinnyPlan& sk) { return Plan{CFG_SKINNY, sk.splits, sk.blocks, sk.strips}; }
 
@@ -716,7 +717,6 @@ int run(const Problem& P, hipStream_t stream) {
                       dw(P.B, P.ldb, b.b_outer, b.b_inner, b.seg_b) && (!P.ep.B2 || ((uintptr_t)P.ep.B2 & 3u) == 0);
   const bool fast = (vecA && vecB && mult(a_ext) && mult(b_ext) && spanA && spanB) ||
                     (dwords && mode != MODE_PROLOGUE);
-  const bool skinny = dwords && skinny_fits(P.transA, P.transB, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode, CH);
 
   // SiLU-gate prologue as its own pass when the workspace holds SiLU(A) * A2 (bf16,
   // one matrix, 16-byte rows): the activation is written once and the GEMM runs
@@ -755,8 +755,9 @@ int run(const Problem& P, hipStream_t stream) {
   // kernels on the same problem)
   // a dual product's partials are no part of what mi_gemm_workspace_size promises, so
   // mi_gemm_noalloc runs it as mi_gemm does without a workspace
-  const SkinnyPlan sk = skinny_plan(P.dtype_in == MI_BF16, P.transB != 0, mode == MODE_DUAL, P.M, P.N, P.K,
-                                    allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0);
+  const SkinnyPlan sk = plan_skinny(P.dtype_in, P.transA, P.transB, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode,
+                                    dwords, allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0, current_cus());
+  const bool skinny = sk.take;
   const bool masked = b.causal == MI_CAUSAL_OUT_LOWER;
   const int direct = direct_kind(P.transA, P.transB, P.M, P.N, P.K, !P.ep.bias && !P.ep.residual && cvec, masked);
   Plan plan = skinny ? skinny_as_plan(sk)
@@ -1137,11 +1138,10 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
   // for them and with it: TN 1263 x 528 x 1710 93 and 42, 121 x 2036 x 1362 71 and 36; NN
   // 337 x 1593 x 1659 69 and 39)
   if (!packed_dwords(dtype_in, transA, transB, M, N, K)) cover(tile_splits(false));
-  const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
-  if (skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, MODE_PLAIN, ch)) {
-    // operands that rule the skinny kernels out take the tile plan, so room for either
-    cover(skinny_plan(dtype_in == MI_BF16, transB != 0, false, M, N, K, INT64_MAX / 8).splits);
-  }
+  // operands that rule the few-row kernels out take the tile plan, so room for either
+  const SkinnyPlan sk = plan_skinny(dtype_in, transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, MODE_PLAIN, true,
+                                    INT64_MAX / 8, cus);
+  if (sk.take) cover(sk.splits);
   return need;
 }
 
@@ -1847,10 +1847,10 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
   const bool dwords = packed_dwords(dtype_in, transA, transB, M, N, K);
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) || (dwords && mode != MODE_PROLOGUE);
-  const Plan pl = (K == 0 || dwords) && skinny_fits(transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, ch)
-                      ? skinny_as_plan(skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws))
-                      : make_plan(dtype_in, transA && !transB ? MI_F32 : dtype_in, transA, transB, M, N, K, batch, mode,
-                                  direct_kind(transA, transB, M, N, K, true, false), ws > 0, ws, cus, fast);
+  const SkinnyPlan sk = plan_skinny(dtype_in, transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, K == 0 || dwords, ws, cus);
+  const Plan pl = sk.take ? skinny_as_plan(sk)
+                          : make_plan(dtype_in, transA && !transB ? MI_F32 : dtype_in, transA, transB, M, N, K, batch, mode,
+                                      direct_kind(transA, transB, M, N, K, true, false), ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

@@ -17,9 +17,10 @@ typedef void (*KernelFn)(Params);
 //         64x64, each over half of every K tile, summed through LDS),
 //         M 256x192 (8 waves of 64x96), V 128x192 with wave-level split-K (two
 //         groups of 4 waves of 64x96).
-//   SKINNY (either type): at most 64 rows, mi_skinny.hip (the shape is in skinny_plan).
+//   SKINNY (either type): products of up to 64 rows and small fp32 ones in blocks of 64
+//         rows, mi_skinny.hip (the shape is in skinny_plan).
 //   fp32: V 64x128, M 64x64 and DUAL_S 64x64 of each B direct-to-LDS (four waves);
-//         register-staged L = S = W 128x128, DUAL 128x64, PRO 128x128.
+//         register-staged S 128x128, DUAL 128x64, PRO 128x128.
 enum Cfg { CFG_L = 0, CFG_S = 1, CFG_DUAL = 2, CFG_PRO = 3, CFG_W = 4, CFG_M = 5, CFG_V = 6, CFG_SKINNY = 7, CFG_DUAL_S = 8,
            CFG_DUAL_W = 9, CFG_DUAL_M = 10, CFG_DUAL_L = 11 };
 

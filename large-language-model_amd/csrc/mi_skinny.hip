@@ -1,6 +1,6 @@
 // mi_skinny.hip -- GEMM of a few rows (token generation, short batches): C[M, N] with
 // M <= 64 and op(A) not transposed, bf16 or fp32, optionally with the dual-B SiLU gate; and
-// small fp32 products in blocks of 64 rows (skinny_blocks_fit).
+// small fp32 products in blocks of 64 rows (mi_skinny.hpp).
 //
 // Bound: the weights B are read once from HBM and everything else is small, so a call
 // takes the time of streaming K x N elements plus a memory latency per launch.  What that
@@ -327,41 +327,53 @@ void launch_rows(const Params& p, const SkinnyPlan& pl, bool both, hipStream_t s
 
 }  // namespace
 
-bool skinny_blocks_fit(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K) {
-  const int64_t blocks = ((M + 63) / 64) * ((N + 31) / 32);
-  return !bf16 && !transB && !dual && K <= 1024 && blocks >= 128 && blocks <= 256;
-}
-
-SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems) {
+SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems, int cus) {
   SkinnyPlan pl{};
+  const int64_t es = bf16 ? 2 : 4, nd = dual ? 2 : 1;
+  pl.blocks = (int)((M + 63) / 64);
+  if (M > SKINNY_MAX_M) {
+    const int64_t blocks = pl.blocks * ((N + 31) / 32);
+    if (bf16 || transB || dual || K > 1024 || 2 * blocks < cus || blocks > cus) return pl;
+  } else if (M > 32 && N * K * es > SKINNY_WIDE_BYTES) {
+    return pl;
+  }
   pl.mb = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-  const int64_t es = bf16 ? 2 : 4, steps = std::max<int64_t>(1, (K * es + 63) / 64), nd = dual ? 2 : 1;
+  const int64_t steps = std::max<int64_t>(1, (K * es + 63) / 64);
   auto cols_of = [&](bool part) {
     const int dw = lane_dwords(part, transB, (int)es, pl.mb);
     return 16 * (transB ? dw : dw * 4 / (int)es);
   };
   auto strips_of = [&](bool part) { return (N + cols_of(part) - 1) / cols_of(part); };
-  // K parts: up to 512 workgroups, each wave at least one step, and the partials (written
+  // K parts: up to two workgroups a CU, each wave at least one step, and the partials (written
   // and read back) at most half the bytes of B
   const int64_t groups = strips_of(true) * nd;
-  const int64_t sp = std::min<int64_t>({512 / groups, steps / PART_WAVES, K * es / (16 * M),
+  const int64_t sp = std::min<int64_t>({2 * cus / groups, steps / PART_WAVES, K * es / (16 * M),
                                         ws_elems / std::max<int64_t>(1, nd * M * N), 64});
-  // Time of either form in us, fitted to the rates above and to whole decoder layers: a
-  // whole-K workgroup takes 1 us and 24 GB/s of its strip and half of A (which the L2 holds),
-  // at most 2.3 TB/s over the chip; K parts run at 3.5 TB/s from 160 workgroups on, and
-  // their second launch takes 3.5 us.  Layer of 8 rows, all whole / all parts: width 2048 68.5
-  // / 56.7 us, width 768 36.0 / 41.6.
+  // Time of either form in us, fitted to the rates above, to 4758 products with B cold and to whole
+  // decoder layers, whose weights the last-level cache holds: a whole-K workgroup takes 1 us
+  // and 24 GB/s of its strip and half of A (which the L2 holds), at most 2.3 TB/s over the
+  // chip; K parts run at 3.5 TB/s from 5 workgroups on 8 CUs on, and their second launch takes
+  // 4.5 us (cold products prefer 6.5, by 1 %: 16 x 768 x 768 fp32 parts 6.3 us, whole 5.9; a
+  // layer of 8 rows, all whole / all parts / by this rule: width 2048 68.5 / 56.7 / 57.0 us,
+  // with 6.5 59.7; width 768 all whole 36.0, all parts 41.6).
   const double bytes = (double)(nd * N * K * es);
   const double whole = (double)((nd * cols_of(false) + 8 * pl.mb) * K * es);
-  const double t_whole = 1.0 + std::max(whole / 24e3 * (double)((strips_of(false) + 255) / 256), bytes / 2.3e6);
-  const double t_part = bytes / 3.5e6 * std::max(1.0, 160.0 / (double)(groups * std::max<int64_t>(sp, 1))) +
-                        (sp > 1 || dual ? 3.5 + 8.0 * (double)(sp * nd * M * N) / 3.5e6 : 0.0);
-  pl.blocks = (int)((M + 63) / 64);
+  const double t_whole = 1.0 + std::max(whole / 24e3 * (double)((strips_of(false) + cus - 1) / cus), bytes / 2.3e6);
+  const double t_part = bytes / 3.5e6 * std::max(1.0, 0.625 * cus / (double)(groups * std::max<int64_t>(sp, 1))) +
+                        (sp > 1 || dual ? 4.5 + 8.0 * (double)(sp * nd * M * N) / 3.5e6 : 0.0);
   pl.part = sp >= 1 && t_part < t_whole && pl.blocks == 1;
   pl.splits = pl.part ? (int)sp : 1;
   pl.dual_parts = pl.part && dual;
   pl.cols = cols_of(pl.part);
   pl.strips = (int)strips_of(pl.part);
+  // Strips past two or three to a CU are short work for a workgroup each, and 128-row tiles
+  // leave no CU idle either: the tile kernels take them, but for a few rows only while K is
+  // short (us, skinny and tile: 2 x 32000 x 112 bf16 NT 11.5 and 6.6, 3 x 32000 x 1152 19.3
+  // and 17.1, 8 x 32000 x 2048 cold 0.8 of the tile's time, 7 x 32000 x 64 fp32 NT 13.1 and
+  // 7.1; 26 x 32000 x 2424 fp32 NT 119 and 84; 64 x 32000 x 192 bf16 dual 16.9 and 12.9).
+  const int64_t per_cu = M > 32 ? (dual ? 1 : 2) : M > 16 ? 3 : 2;
+  pl.take = pl.part || M > SKINNY_MAX_M || pl.strips <= per_cu * cus ||
+            (M <= 16 && K * es >= (pl.strips > 4 * cus ? 3072 : 1024));
   return pl;
 }
 

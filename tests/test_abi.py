@@ -345,6 +345,19 @@ def test_fp32_plans_keep_their_chains(mi):
     assert deeper > 50
 
 
+def test_few_row_routes(mi):
+    """Products of few rows leave their kernels where tiles fill the chip anyway: many strips of a
+    short K, more than 16 rows on very many strips, more than 32 rows of a large B."""
+    for dt, tB, M, N, K, dual, few in [
+            ("bf16", 1, 2, 32000, 112, 0, False), ("f32", 1, 7, 32000, 64, 0, False), ("bf16", 0, 7, 32000, 64, 0, False),
+            ("bf16", 1, 2, 32000, 2048, 0, True), ("f32", 1, 7, 32000, 1024, 0, True), ("bf16", 0, 8, 3072, 2048, 0, True),
+            ("f32", 1, 26, 32000, 2424, 0, False), ("bf16", 0, 32, 5632, 2048, 1, True), ("bf16", 0, 16, 768, 64, 0, True),
+            ("bf16", 0, 64, 32000, 192, 1, False), ("bf16", 0, 64, 2048, 2048, 0, True), ("f32", 0, 64, 2048, 5632, 0, False)]:
+        dti = mi.MI_F32 if dt == "f32" else mi.MI_BF16
+        text = mi.describe(0, tB, M, N, K, dti, epi_mode=dual)
+        assert text.startswith("skinny") == few, (dt, tB, M, N, K, dual, text)
+
+
 def test_bf16_plans_of_small_grids(mi):
     """Under 128 tiles of 128x128: four-wave tiles at a short K with the direct epilogue, eight-wave
     ones (kg2) past it; and weight gradients (TN, fp32) summed in as many chains (two in an
