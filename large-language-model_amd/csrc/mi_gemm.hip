@@ -234,9 +234,9 @@ int direct_kind(int transA, int transB, int64_t M, int64_t N, int64_t K, bool pl
 //     split below 5/8 of a wave (element-granular loader); the rules at the fp32
 //     branch.
 // Every split fits the workspace: splits * M * N * batch <= ws_limit_elems.
-// direct: direct_kind of the problem.
+// direct: direct_kind of the problem; cut: causally skipped or masked.
 Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int64_t N, int64_t Ktot, int64_t batch,
-               int mode, int direct, bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
+               int mode, int direct, bool cut, bool allow_split, int64_t ws_limit_elems, int cus, bool fast) {
   const bool tn = transA && !transB;
   auto plan_for = [&](int cfg, int sp) {
     const CfgShape s = shape_of(dtype_in, cfg);
@@ -370,8 +370,10 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
   // against 64 bits no larger; without the bound on the chains 1.2 %, but up to 9 % slower and
   // an error up to 2.2 times as large (256 x 3180 x 4288 NN: 64x128 split 5 64.6 us, 3.7e-7;
   // 64x64 whole 72, 5.8e-7).
-  // Batched products (the attention's, short K or causally cut) take 64x64 tiles:
-  // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304.
+  // Causally cut products (the attention's) take 64x64 tiles, which waste less on the diagonal:
+  // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304;
+  // uncut batches do not (47 of 1536 x 256 x 61 TN 64x64 34.5 us, 64x128 30.3; 48 of 1152 x
+  // 1024 x 48 NT 111, 99).
   // The element-granular loader (any alignment) runs 128x128 tiles (S): below 5/8
   // of a wave, K is split by the same score with units at most two per CU and each
   // split keeping >= 8 K tiles of 32, or >= 4 when the units fit one per CU (96
@@ -384,7 +386,7 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
     auto search = [&](bool timed, int least) {
       double best_score = 1e300;
       for (int cfg : {CFG_V, CFG_M}) {
-        if (cfg == CFG_V && batch > 1) continue;
+        if (cfg == CFG_V && cut) continue;
         const CfgShape t = shape_of(dtype_in, cfg);
         const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
         for (int sp = least; sp <= (allow_split ? 8 : 1); ++sp) {
@@ -762,7 +764,7 @@ int run(const Problem& P, hipStream_t stream) {
   const int direct = direct_kind(P.transA, P.transB, P.M, P.N, P.K, !P.ep.bias && !P.ep.residual && cvec, masked);
   Plan plan = skinny ? skinny_as_plan(sk)
                      : make_plan(P.dtype_in, P.dtype_c, P.transA, P.transB, P.M, P.N, Ktot, b.batch, mode, direct,
-                                 allow_split || P.noalloc, P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
+                                 b.causal != MI_CAUSAL_NONE, allow_split || P.noalloc, P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
   if (P.noalloc && plan.splits > 1 && (int64_t)plan.splits * P.M * P.N * b.batch > ws_elems)
     return fail(MI_ERR_WORKSPACE,
                 "mi_gemm_noalloc: split-K by %d needs %lld bytes of scratch, above its %lld-byte "
@@ -1131,7 +1133,7 @@ size_t mi_gemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int6
   };
   auto tile_splits = [&](bool fast) {
     return make_plan(dtype_in, dtype_c, transA, transB, M, N, K, batch, MODE_PLAIN,
-                     direct_kind(transA, transB, M, N, K, true, false), true, INT64_MAX / 8, cus, fast).splits;
+                     direct_kind(transA, transB, M, N, K, true, false), false, true, INT64_MAX / 8, cus, fast).splits;
   };
   cover(tile_splits(true));
   // odd bf16 rows: the register-staged kernel's plan, whose splits matter more (us without room
@@ -1384,7 +1386,8 @@ int mi_flash_attn_bwd_scaled(void* stream, const void* Q, const void* K, const v
     // 128-row output tile; the dK/dV kernel writes dS^T (zeros included) for every
     // key below that bound, and not beyond it, so taller tiles take the dQ kernel.
     const Plan pl = make_plan(MI_BF16, MI_BF16, 1, 0, seq_len, head_dim, seq_len, batch * n_heads, MODE_PLAIN,
-                              direct_kind(1, 0, seq_len, head_dim, seq_len, true, false), false, 0, current_cus(), true);
+                              direct_kind(1, 0, seq_len, head_dim, seq_len, true, false), causal != 0, false, 0,
+                              current_cus(), true);
     if (shape_of(MI_BF16, pl.cfg).bm != 128) p.dsT = nullptr;
   }
   hipError_t e = launch_flash_bwd(p, (int)head_dim, (hipStream_t)stream);
@@ -1850,7 +1853,7 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   const SkinnyPlan sk = plan_skinny(dtype_in, transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, K == 0 || dwords, ws, cus);
   const Plan pl = sk.take ? skinny_as_plan(sk)
                           : make_plan(dtype_in, transA && !transB ? MI_F32 : dtype_in, transA, transB, M, N, K, batch, mode,
-                                      direct_kind(transA, transB, M, N, K, true, false), ws > 0, ws, cus, fast);
+                                      direct_kind(transA, transB, M, N, K, true, false), false, ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

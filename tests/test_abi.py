@@ -345,6 +345,14 @@ def test_fp32_plans_keep_their_chains(mi):
     assert deeper > 50
 
 
+def test_fp32_batches_keep_wide_tiles(mi):
+    """Uncut fp32 batches choose between both tiles as single products do."""
+    for tA, tB, batch, M, N, K, tile in [(1, 0, 47, 1536, 256, 61, "64x128"), (0, 1, 48, 1152, 1024, 48, "64x128"),
+                                         (0, 0, 14, 1472, 1280, 128, "64x128"), (0, 1, 8, 256, 192, 512, "64x64")]:
+        text = mi.describe(tA, tB, M, N, K, mi.MI_F32, batch=batch)
+        assert text.startswith("dlds f32 " + tile), (batch, M, N, K, text)
+
+
 def test_few_row_routes(mi):
     """Products of few rows leave their kernels where tiles fill the chip anyway: many strips of a
     short K, more than 16 rows on very many strips, more than 32 rows of a large B."""
