@@ -23,7 +23,7 @@
 // kernel sums the workspace rows in order: dw is bit-identical across launches.
 // Rows that are not whole aligned 16-byte vectors, or longer (up to 16384 bf16 / 8192 fp32
 // values): a workgroup per row, the row in registers too (norm_fwd_row, norm_bwd_row); past
-// that, or under 16 bytes, strided passes over global memory.  xhat is formed as
+// that, under 16 bytes, or short in the forward, strided passes over global memory.  xhat is formed as
 // x * (1/rms): one reciprocal per row instead of a division per element (the divide
 // sequence made the backward VALU-bound).
 #include <hip/hip_runtime.h>
@@ -661,7 +661,11 @@ template <bool BF16, bool W_BF16>
 hipError_t fwd_one(const NormParams& p, bool vector_path, hipStream_t st) {
   const int runs = runs_per_thread(p.dims, BF16);
   const dim3 rows((unsigned)p.rows);
-  if (!vector_path && runs <= 8) {
+  // A row of up to 512 bf16 / 256 fp32 values is one or two elements a thread of the strided
+  // kernel, which the row kernel's few busy lanes cannot match (us, strided and row: 15451 x
+  // 116 bf16 10.7 and 14.7, 5744 x 38 bf16 5.0 and 6.9, 8818 x 42 fp32 6.5 and 7.6; 768 bf16
+  // columns 1.05 times as fast in registers, 384 fp32 1.02).  The backward gains at any size.
+  if (!vector_path && runs <= 8 && p.dims > (BF16 ? 512 : 256)) {
     switch (runs) {
       case 1: hipLaunchKernelGGL((norm_fwd_row<BF16, W_BF16, 1, 256>), rows, dim3(256), 0, st, p); break;
       case 2: hipLaunchKernelGGL((norm_fwd_row<BF16, W_BF16, 2, 256>), rows, dim3(256), 0, st, p); break;
