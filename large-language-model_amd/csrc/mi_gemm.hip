@@ -960,10 +960,16 @@ struct SoftRow {
 #pragma unroll
       for (int e = 0; e < EV; ++e)
         v[i][e] = BF ? bf16_bits_to_f32((w[e / 2] >> (16 * (e & 1))) & 0xffffu) : __uint_as_float(w[e & 3]);
-      if (k < n && k + EV > n)
+      if (k < n && k + EV > n) {
+        // every load at an address of the row, so that none waits for another's branch (bf16 rows
+        // of 37 to 119 values, backward: 3.9-4.2 us with a branch a value)
+        float t[EV];
+#pragma unroll
+        for (int e = 0; e < EV; ++e) t[e] = ldv<BF>(p, base + (k + e < n ? k + e : n - 1));
 #pragma unroll
         for (int e = 0; e < EV; ++e)
-          if (k + e < n) v[i][e] = ldv<BF>(p, base + k + e);
+          if (k + e < n) v[i][e] = t[e];
+      }
     }
   }
   __device__ static __forceinline__ void store(void* p, int64_t base, int n, int lane, const float (&v)[NV][EV]) {
@@ -1075,21 +1081,24 @@ __global__ void __launch_bounds__(256) softmax_bwd_kernel(const void* P, void* d
 }
 
 // Launch `wave` (a functor taking the vectors per lane as a constant) where a row fits a wave's
-// registers; false where it does not.
+// registers; false where it does not.  half8: whether 8 vectors a lane pay while the row fills
+// little more than half of them.
 template <bool BF, typename F>
-bool launch_soft_wave(int64_t T, F&& wave) {
+bool launch_soft_wave(int64_t T, bool half8, F&& wave) {
   const int64_t per = 64 * (BF ? 8 : 4);
   if (T <= per) wave(std::integral_constant<int, 1>{});
   else if (T <= 2 * per) wave(std::integral_constant<int, 2>{});
   else if (T <= 4 * per) wave(std::integral_constant<int, 4>{});
-  else if (T <= 8 * per) wave(std::integral_constant<int, 8>{});
+  else if (T <= 8 * per && (half8 || 2 * T > 11 * per)) wave(std::integral_constant<int, 8>{});
   else return false;
   return true;
 }
 
 template <bool BF>
 void launch_softmax(void* S, int64_t rows, int64_t T, int64_t ld, hipStream_t st) {
-  if (!launch_soft_wave<BF>(T, [&](auto nv) {
+  // The causal rows are half as long on average: bf16 rows of 2144 took 59.6 us in a workgroup
+  // each and 65.6 in a wave, 2392 11.2 and 12.2, 3072 1.02 times the wave's time, 4096 1.2.
+  if (!launch_soft_wave<BF>(T, !BF, [&](auto nv) {
         hipLaunchKernelGGL((softmax_causal_wave<BF, decltype(nv)::value>), dim3((unsigned)cdiv(rows, 4)), dim3(256), 0,
                            st, S, rows, (int)T, ld);
       }))
@@ -1098,7 +1107,11 @@ void launch_softmax(void* S, int64_t rows, int64_t T, int64_t ld, hipStream_t st
 
 template <bool BF>
 void launch_softmax_bwd(const void* P, void* dP, int64_t rows, int64_t T, int64_t ld, float scale, hipStream_t st) {
-  if (!launch_soft_wave<BF>(T, [&](auto nv) {
+  // bf16 rows that end inside a run cost a wave a second round of loads, which shows while all
+  // rows run at once, on a workgroup each (450 rows of 150 3.0 us so, 3.6 in waves; past 2048
+  // rows the waves lead, 1.2 times at 10000 rows of 200).
+  const bool few = BF && T % 8 != 0 && rows <= 8 * (int64_t)current_cus();
+  if (few || !launch_soft_wave<BF>(T, true, [&](auto nv) {
         hipLaunchKernelGGL((softmax_bwd_wave<BF, decltype(nv)::value>), dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, st,
                            P, dP, rows, (int)T, ld, scale);
       }))

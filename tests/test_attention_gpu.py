@@ -370,3 +370,22 @@ def test_softmax_rows(mi, dev, bf16, T):
     want = P.double() * (dP.double() - (P.double() * dP.double()).sum(-1, keepdim=True)) * 0.125
     mi.softmax_bwd_(P, dP, T, 0.125)
     assert (dP.double() - want).abs().max().item() <= tol * max(1e-3, want.abs().max().item())
+
+
+@pytest.mark.parametrize("T,n", [(3, 700), (67, 40), (255, 9), (257, 9), (1023, 3), (2100, 1), (2814, 1), (2817, 1)])
+def test_softmax_routes(mi, dev, T, n):
+    """bf16 rows on both sides of the lines between a wave and a workgroup a row: the backward of more
+    rows than run at once, ragged; the forward of rows just past half of eight vectors a lane."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(T)
+    S = (4 * torch.randn(n, T, T, generator=g, device=dev)).to(torch.bfloat16)
+    low = torch.ones(T, T, dtype=torch.bool, device=dev).tril_()
+    ref = torch.softmax(S.double().masked_fill(~low, -float("inf")), -1)
+    P = S.clone()
+    mi.softmax_causal_(P, T)
+    assert (P.double() - ref).abs().max().item() <= 2.0 ** -8  # one bf16 rounding of values up to 1
+    dP = torch.randn(n, T, T, generator=g, device=dev).to(torch.bfloat16)
+    want = P.double() * (dP.double() - (P.double() * dP.double()).sum(-1, keepdim=True)) * 0.125
+    mi.softmax_bwd_(P, dP, T, 0.125)
+    assert (dP.double() - want).abs().max().item() <= 2.0 ** -8 * max(1e-3, want.abs().max().item())
