@@ -848,13 +848,18 @@ def test_causal_output_mask(mi, dev, bf16, T, N):
 
 
 @pytest.mark.parametrize("tB", [0, 1], ids=["NN", "NT+TT"])
-@pytest.mark.parametrize("bf16,dual,M,N", [
-    (True, 0, 300, 264), (True, 0, 2047, 2052), (True, 0, 4095, 4092), (True, 1, 130, 2052), (True, 1, 1000, 2816),
-    (False, 0, 300, 260), (False, 0, 2047, 1540), (False, 1, 155, 772)])
-def test_k_tails(mi, dev, bf16, dual, M, N, tB):
+@pytest.mark.parametrize("bf16,dual,M,N,Ks,want", [
+    (True, 0, 300, 264, (328, 330, 70), "128x128"), (True, 0, 2047, 2052, (328, 330), "128x128"),
+    (True, 0, 4095, 4092, (328, 330), "256x256"), (True, 0, 2047, 5632, (328, 330), "256x192"),
+    (True, 0, 1000, 5632, (1032, 1034), "dlds-kg2 bf16 128x192"), (True, 0, 999, 2052, (1096, 1098), "dlds-kg2 bf16 128x128"),
+    (True, 1, 1000, 5632, (328, 330), "256x128"), (True, 1, 2048, 5632, (136, 138), "192x128"),
+    (True, 1, 500, 5632, (520, 522), "dlds bf16 128x64"), (True, 1, 130, 2052, (328, 330, 522), "dlds-kg2 bf16 128x64"),
+    (False, 0, 300, 260, (108, 110, 333), "64x64"), (False, 0, 2047, 772, (68, 70), "64x128"),
+    (False, 1, 155, 772, (108, 110, 333), "64x64")])
+def test_k_tails(mi, dev, bf16, dual, M, N, Ks, want, tB):
     """K ends inside a K tile, on a 16-byte chunk and inside one (the direct-to-LDS kernels' two
-    tail variants), plain and dual, with NaN in the gap after each operand row. Plain: integer
-    products, bit for bit."""
+    tail variants), on every tile, plain and dual, with NaN in the gap after each operand row.
+    Plain: integer products, bit for bit."""
     import torch
 
     dt = torch.bfloat16 if bf16 else torch.float32
@@ -867,7 +872,9 @@ def test_k_tails(mi, dev, bf16, dual, M, N, tB):
         buf[:, :m.shape[1]] = m
         return buf, buf.shape[1]
 
-    for K, tA in itertools.product((328, 330, 70) if bf16 else (108, 110, 333), (0, 1) if tB and not dual else (0,)):
+    for K, tA in itertools.product(Ks, (0, 1) if tB and not dual else (0,)):
+        plan = mi.describe(0, tB, M, N, K, mi.MI_BF16 if bf16 else mi.MI_F32, epi_mode=dual, workspace_bytes=32 << 20)
+        assert plan.startswith("dlds") and want in plan, plan
         a = torch.randint(-2, 3, (M, K), generator=g, device=dev)
         bs = [torch.randint(-2, 3, (K, N), generator=g, device=dev) for _ in range(1 + dual)]
         (A, lda), B = place(a, tA), [place(b, tB) for b in bs]
@@ -880,3 +887,86 @@ def test_k_tails(mi, dev, bf16, dual, M, N, tB):
             check(host(C), host(torch.nn.functional.silu(ref[0]) * ref[1]), _tol(bf16), f"dual {M}x{N}x{K}")
         else:
             assert torch.equal(C, ref[0].float()), (K, tA)
+
+
+@pytest.mark.parametrize("bf16", [True, False], ids=["bf16", "f32"])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 1)], ids=["NN", "NT", "TT"])
+def test_straddling_chunk_with_segments_splits_and_causal(mi, dev, bf16, tA, tB):
+    """K ends inside a 16-byte chunk of each of several K segments, split along K, and under causal
+    skipping of either side; NaN after each operand row. Integers, bit for bit."""
+    import torch
+
+    dt = torch.bfloat16 if bf16 else torch.float32
+    g = torch.Generator(device=dev).manual_seed(31 + 2 * tA + tB)
+    ws = torch.full((8 << 20,), float("nan"), dtype=torch.float32, device=dev)
+
+    def place(m, trans):  # [nb, segs, rows, K] or [nb, segs, K, cols], each row followed by NaN
+        m = m.transpose(-1, -2) if trans else m
+        pitch = m.shape[-1] + 2 + m.shape[-1] % 2
+        buf = torch.full((*m.shape[:-1], pitch), float("nan"), dtype=dt, device=dev)
+        buf[..., :m.shape[-1]] = m
+        return buf, pitch, m.shape[-2] * pitch
+
+    for nb, segs, M, N, K, causal in [(1, 3, 70, 66, 1034 if bf16 else 1033, 0), (2, 2, 66, 130, 330 if bf16 else 333, 0),
+                                      (1, 1, 130, 70, 2058 if bf16 else 1029, 0),
+                                      (2, 1, 330, 66, 330, mi.MI_CAUSAL_A_LOWER), (2, 1, 330, 70, 330, mi.MI_CAUSAL_A_UPPER)]:
+        a = torch.randint(-2, 3, (nb, segs, M, K), generator=g, device=dev)
+        if causal:
+            a = a.tril() if causal == mi.MI_CAUSAL_A_LOWER else a.triu()
+        b = torch.randint(-2, 3, (nb, segs, K, N), generator=g, device=dev)
+        (A, lda, sa), (B, ldb, sb) = place(a, tA), place(b, tB)
+        C = torch.full((nb, M, N), float("nan"), dtype=torch.float32, device=dev)
+        bt = mi.make_batch(nb, 1, a=(segs * sa, 0, 1), b=(segs * sb, 0, 1), c=(M * N, 0, 1), k_segments=segs, seg_a=sa,
+                           seg_b=sb, causal=causal)
+        mi.gemm_batched(A, B, C, M, N, K, bt, transA=bool(tA), transB=bool(tB), lda=lda, ldb=ldb,
+                        workspace=None if causal else ws)
+        ref = (a.double() @ b.double()).sum(1)
+        assert torch.equal(C, ref.float()), (nb, segs, M, N, K, causal)
+
+
+@pytest.mark.parametrize("bf16", [True, False], ids=["bf16", "f32"])
+def test_row_scale_on_few_rows(mi, dev, oracle, bf16):
+    """A factor per row of A B (a folded RMSNorm) on the few-row kernels, K whole and in parts, and on
+    fp32 64-row blocks, before the bias and the residual."""
+    import torch
+
+    ws = torch.full((4 << 20,), float("nan"), dtype=torch.float32, device=dev)
+    for M, N, K, parts in [(8, 768, 256, False), (7, 130, 136, False), (16, 1024, 4096, True), (33, 514, 4096, True)] + (
+            [] if bf16 else [(300, 1026, 768, False)]):
+        plan = mi.describe(0, 0, M, N, K, mi.MI_BF16 if bf16 else mi.MI_F32, workspace_bytes=16 << 20)
+        assert plan.startswith("skinny") and ("split1 " not in plan) == parts, plan
+        a, b = inputs(oracle, (M, K), 700 + M, 1.0, bf16), inputs(oracle, (K, N), 701 + M, 0.02, bf16)
+        bias, r = inputs(oracle, (N,), 702, 0.1, bf16), inputs(oracle, (M, N), 703, 0.5, bf16)
+        rs = np.random.default_rng(M).uniform(0.5, 2.0, M).astype(np.float32)
+        C = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+        mi.gemm(to_dev(a, dev, bf16), to_dev(b, dev, bf16), C, M, N, K, bias=to_dev(bias, dev, bf16),
+                residual=to_dev(r, dev, bf16), row_scale=to_dev(rs, dev, False), workspace=ws)
+        ref = (a.astype(np.float64) @ b.astype(np.float64)) * rs[:, None].astype(np.float64) + bias + r
+        check(host(C), ref, _tol(bf16), f"row scale {M}x{N}x{K} parts={parts}")
+
+
+@pytest.mark.parametrize("tB", [0, 1], ids=["TN", "TT"])
+@pytest.mark.parametrize("bf16,M,N,K,want", [
+    (True, 4094, 4092, 128, "256x256"), (True, 2046, 5636, 1024, "256x256"), (True, 2046, 5632, 1024, "256x192"),
+    (True, 1000, 5632, 1024, "128x192"), (True, 998, 2052, 1088, "dlds-kg2 bf16 128x128"),
+    (True, 2046, 2052, 256, "dlds bf16 128x128"), (False, 300, 260, 96, "64x64"), (False, 2046, 772, 64, "64x128")])
+def test_cut_blocks_of_transposed_a(mi, dev, bf16, M, N, K, want, tB):
+    """The direct epilogue's cut blocks behind a transposed A, on the tile named, C's rows on
+    64-byte lines and off them, with and without beta; the gap after each row stays."""
+    import torch
+
+    plan = mi.describe(1, tB, M, N, K, mi.MI_BF16 if bf16 else mi.MI_F32)
+    assert plan.startswith("dlds") and want in plan, plan
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    a = torch.randint(-2, 3, (M, K), generator=g, device=dev)
+    b = torch.randint(-2, 3, (K, N), generator=g, device=dev)
+    ref = a.double() @ b.double()
+    A, B = a.T.contiguous().to(dt), (b.T if tB else b).contiguous().to(dt)
+    for ldc, beta in ((N + 4, 0.0), ((N + 31) // 16 * 16, 0.0), (N + 4, 2.0), ((N + 31) // 16 * 16, 2.0)):
+        buf = torch.full((M, ldc), float("nan"), dtype=torch.float32, device=dev)
+        C = buf[:, :N]
+        C.fill_(3.0)
+        mi.gemm(A, B, C, M, N, K, transA=True, transB=bool(tB), beta=beta, ldc=ldc)
+        assert torch.equal(C, (ref + 3.0 * beta).float()), (ldc, beta)
+        assert buf[:, N:].isnan().all()
