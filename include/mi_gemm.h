@@ -142,8 +142,8 @@ int mi_gemm(void* stream, int transA, int transB, int64_t M, int64_t N, int64_t 
  * SiLU-gate prologue (epi->A2) it runs the plan mi_gemm makes given no workspace
  * (the activation applied while each A tile is loaded, no split): the two-pass
  * form mi_gemm takes when its workspace holds the M x K activation does not fit
- * the scratch.  A dual-B product (epi->B2) of few rows likewise runs unsplit.  Calls no allocating routine.  Every call on a
- * GPU shares that GPU's array: calls that overlap in time on one GPU (different
+ * the scratch.  A dual-B product (epi->B2) of few rows likewise runs unsplit.
+ * Calls no allocating routine.  Every call on a GPU shares that GPU's array: calls that overlap in time on one GPU (different
  * streams, or different host threads) race and must be serialised by the caller.
  * Not recorded by the profiler.
  */

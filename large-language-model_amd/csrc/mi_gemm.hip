@@ -433,7 +433,8 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
 SkinnyPlan plan_skinny(int dtype_in, int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch,
                        int64_t segs, int causal, int mode, bool dwords, int64_t ws_elems, int cus) {
   const int64_t ch = dtype_in == MI_BF16 ? 8 : 4;
-  if (transA || K % ch != 0 || batch != 1 || segs != 1 || causal != MI_CAUSAL_NONE || mode == MODE_PROLOGUE || !dwords)
+  if (transA || K % ch != 0 || batch != 1 || segs != 1 || causal != MI_CAUSAL_NONE ||
+      mode == MODE_PROLOGUE || !dwords)
     return SkinnyPlan{};
   return skinny_plan(dtype_in == MI_BF16, transB != 0, mode == MODE_DUAL, M, N, K, ws_elems, cus);
 }
@@ -757,14 +758,16 @@ int run(const Problem& P, hipStream_t stream) {
   // kernels on the same problem)
   // a dual product's partials are no part of what mi_gemm_workspace_size promises, so
   // mi_gemm_noalloc runs it as mi_gemm does without a workspace
-  const SkinnyPlan sk = plan_skinny(P.dtype_in, P.transA, P.transB, P.M, P.N, P.K, b.batch, b.k_segments, b.causal, mode,
-                                    dwords, allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0, current_cus());
+  const SkinnyPlan sk = plan_skinny(P.dtype_in, P.transA, P.transB, P.M, P.N, P.K, b.batch, b.k_segments,
+                                    b.causal, mode, dwords,
+                                    allow_split && !(P.noalloc && mode == MODE_DUAL) ? ws_elems : 0, current_cus());
   const bool skinny = sk.take;
   const bool masked = b.causal == MI_CAUSAL_OUT_LOWER;
   const int direct = direct_kind(P.transA, P.transB, P.M, P.N, P.K, !P.ep.bias && !P.ep.residual && cvec, masked);
   Plan plan = skinny ? skinny_as_plan(sk)
                      : make_plan(P.dtype_in, P.dtype_c, P.transA, P.transB, P.M, P.N, Ktot, b.batch, mode, direct,
-                                 b.causal != MI_CAUSAL_NONE, allow_split || P.noalloc, P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
+                                 b.causal != MI_CAUSAL_NONE, allow_split || P.noalloc,
+                                 P.noalloc ? INT64_MAX / 8 : ws_elems, current_cus(), fast);
   if (P.noalloc && plan.splits > 1 && (int64_t)plan.splits * P.M * P.N * b.batch > ws_elems)
     return fail(MI_ERR_WORKSPACE,
                 "mi_gemm_noalloc: split-K by %d needs %lld bytes of scratch, above its %lld-byte "
@@ -979,7 +982,8 @@ struct SoftRow {
       if (k + EV <= n) {
         uint32_t w[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] = BF ? pack_bf16x2(v[i][(2 * q) % EV], v[i][(2 * q + 1) % EV]) : __float_as_uint(v[i][q]);
+        for (int q = 0; q < 4; ++q)
+          w[q] = BF ? pack_bf16x2(v[i][(2 * q) % EV], v[i][(2 * q + 1) % EV]) : __float_as_uint(v[i][q]);
         __builtin_memcpy((char*)p + (base + k) * (BF ? 2 : 4), w, 16);
       } else {
 #pragma unroll
@@ -1863,10 +1867,12 @@ int mi_gemm_describe(int transA, int transB, int64_t M, int64_t N, int64_t K, in
   const int64_t a_contig = transA ? M : K, b_contig = transB ? K : N;
   const bool dwords = packed_dwords(dtype_in, transA, transB, M, N, K);
   const bool fast = K == 0 || (a_contig % ch == 0 && b_contig % ch == 0) || (dwords && mode != MODE_PROLOGUE);
-  const SkinnyPlan sk = plan_skinny(dtype_in, transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode, K == 0 || dwords, ws, cus);
+  const SkinnyPlan sk = plan_skinny(dtype_in, transA, transB, M, N, K, batch, 1, MI_CAUSAL_NONE, mode,
+                                    K == 0 || dwords, ws, cus);
   const Plan pl = sk.take ? skinny_as_plan(sk)
-                          : make_plan(dtype_in, transA && !transB ? MI_F32 : dtype_in, transA, transB, M, N, K, batch, mode,
-                                      direct_kind(transA, transB, M, N, K, true, false), false, ws > 0, ws, cus, fast);
+                          : make_plan(dtype_in, transA && !transB ? MI_F32 : dtype_in, transA, transB, M, N, K,
+                                      batch, mode, direct_kind(transA, transB, M, N, K, true, false), false,
+                                      ws > 0, ws, cus, fast);
   describe_plan(buf, buf_len, dtype_in, fast, pl, transA, transB, batch);
   return MI_OK;
 }

@@ -82,8 +82,8 @@ __device__ __forceinline__ int mc_unswz(int kr, int p) {
 __device__ __forceinline__ int mc_swz32(int kr, int q) { return q ^ (((kr >> 2) & 1) << 3); }
 
 // Row-contiguous tiles whose row is not a power of two (192 columns), or is a single
-// granule (64 columns of bf16), are stored in 128-byte granules, column block by column block: granule G holds k-row
-// G % BK of the 64-column block G / BK, so consecutive k-rows of one column block
+// granule (64 columns of bf16), are stored in 128-byte granules, column block by column
+// block: granule G holds k-row G % BK of the 64-column block G / BK, so consecutive k-rows of one column block
 // are 128 bytes apart and any four of them cover both halves of a 256-byte bank
 // window; the two 64-byte halves of a granule swap on k-rows 2 and 3 (mod 4), so
 // the four k-rows one transpose read touches land in four different 64-byte bank

@@ -67,10 +67,11 @@ typedef float elem_t;
 #if MI_DT_BF16
 // bf16 direct-to-LDS kernels of one variant (K tile and LDS ring depth:
 // MI_DLDS_BK / MI_DLDS_STAGES for 256x256, MI_S_BK / MI_S_STAGES of the A layout for 128x128;
-// the dual-B tiles are the plain ones with B's columns shared by the two matrices).  256x256 runs 8 waves (2 x 4, wave tiles 128x64): two
-// waves per SIMD, so one wave's MFMAs issue while the other waits on LDS or DMA issue
-// (8192x2048x5632 NT: 147 vs 161 us with 4 waves of 128x128; 8192x5632x2048 NN 157 vs
-// 166; 2048x5632x8192 TN 170 vs 180; bit-identical results).
+// the dual-B tiles are the plain ones with B's columns shared by the two matrices).
+// 256x256 runs 8 waves (2 x 4, wave tiles 128x64): two waves per SIMD, so one wave's MFMAs
+// issue while the other waits on LDS or DMA issue (8192x2048x5632 NT: 147 vs 161 us with
+// 4 waves of 128x128; 8192x5632x2048 NN 157 vs 166; 2048x5632x8192 TN 170 vs 180;
+// bit-identical results).
 template <bool AK, bool BK, int V>
 KernelFn dlds_kernel(int cfg) {
   if constexpr ((V & DLDS_ROWSCALE) != 0) {

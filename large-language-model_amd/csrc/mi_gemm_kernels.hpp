@@ -13,16 +13,16 @@ typedef void (*KernelFn)(Params);
 //         DUAL_L 256x128 of each B (L's waves and LDS with two B tiles of half the width),
 //         DUAL_M 192x128 of each (8 waves of 96x32 of each), DUAL_S and DUAL_W 128x64 of
 //         each (S and W likewise), DUAL 256x128 of each register-staged, PRO 256x256 with
-//         the SiLU-gate A prologue, W 128x128 with wave-level split-K (8 waves: two groups of 4 waves of
-//         64x64, each over half of every K tile, summed through LDS),
+//         the SiLU-gate A prologue, W 128x128 with wave-level split-K (8 waves: two
+//         groups of 4 waves of 64x64, each over half of every K tile, summed through LDS),
 //         M 256x192 (8 waves of 64x96), V 128x192 with wave-level split-K (two
 //         groups of 4 waves of 64x96).
 //   SKINNY (either type): products of up to 64 rows and small fp32 ones in blocks of 64
 //         rows, mi_skinny.hip (the shape is in skinny_plan).
 //   fp32: V 64x128, M 64x64 and DUAL_S 64x64 of each B direct-to-LDS (four waves);
 //         register-staged S 128x128, DUAL 128x64, PRO 128x128.
-enum Cfg { CFG_L = 0, CFG_S = 1, CFG_DUAL = 2, CFG_PRO = 3, CFG_W = 4, CFG_M = 5, CFG_V = 6, CFG_SKINNY = 7, CFG_DUAL_S = 8,
-           CFG_DUAL_W = 9, CFG_DUAL_M = 10, CFG_DUAL_L = 11 };
+enum Cfg { CFG_L = 0, CFG_S = 1, CFG_DUAL = 2, CFG_PRO = 3, CFG_W = 4, CFG_M = 5, CFG_V = 6, CFG_SKINNY = 7,
+           CFG_DUAL_S = 8, CFG_DUAL_W = 9, CFG_DUAL_M = 10, CFG_DUAL_L = 11 };
 
 struct CfgShape {
   int bm, bn;
@@ -60,9 +60,10 @@ inline CfgShape cfg_shape(bool bf16, int cfg) {
 // the fast (buffer-load) or the element-granular loader, or nullptr when the
 // combination does not exist (prologue with transA = 1).  The element-granular
 // variant of the plain configurations exists only for CFG_S.  ktail: the K
-// extent is not whole K tiles (2: nor whole 16-byte chunks of a K-contiguous operand); fast_epi: the epilogue is alpha (SiLU
-// gate), beta*C and the output conversion only, with no split-K (1: on whole 32x32
-// blocks, 2: and the row scale, 3: with blocks cut by the matrix edge).
+// extent is not whole K tiles (2: nor whole 16-byte chunks of a K-contiguous
+// operand); fast_epi: the epilogue is alpha (SiLU gate), beta*C and the output
+// conversion only, with no split-K (1: on whole 32x32 blocks, 2: and the row scale,
+// 3: with blocks cut by the matrix edge).
 #define MI_DECL_PICK(dt, ta, tb) \
   KernelFn pick_##dt##_##ta##tb(int cfg, bool fast, int ktail, int fast_epi);
 MI_DECL_PICK(bf16, 0, 0)

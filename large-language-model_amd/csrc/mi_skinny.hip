@@ -81,7 +81,8 @@ constexpr int lane_dwords(bool part, bool bkc, int es, int mb) {
 // MB: blocks of 16 rows; ND: B matrices of a workgroup (2: both of a dual product, PART
 // false only); PART: the workgroup takes a part of K, as do the waves of one that does not.
 template <typename T, bool BKC, int MB, int ND, bool PART>
-__global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))) skinny_kernel(Params p, int dual_parts) {
+__global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND)))
+    skinny_kernel(Params p, int dual_parts) {
   constexpr int NW = PART ? PART_WAVES : whole_waves(MB, ND);
   constexpr int ES = (int)sizeof(T);
   constexpr int KL = 16 / ES;                    // k of one lane per step
@@ -118,7 +119,8 @@ __global__ void __launch_bounds__(64 * (PART ? PART_WAVES : whole_waves(MB, ND))
   for (int i = 0; i < MB; ++i) ao[i] = (uint32_t)((m0 + 16 * i + cr) * lda + gr * 16);
   if constexpr (BKC) {
 #pragma unroll
-    for (int j = 0; j < CB; ++j) bo[j] = n0 + 16 * j + cr < p.N ? (uint32_t)((n0 + 16 * j + cr) * ldb + gr * 16) : kBufOOB;
+    for (int j = 0; j < CB; ++j)
+      bo[j] = n0 + 16 * j + cr < p.N ? (uint32_t)((n0 + 16 * j + cr) * ldb + gr * 16) : kBufOOB;
   } else {
     // the columns past N of a lane that straddles it are not stored
     bo[0] = n0 + CB * c < p.N ? (uint32_t)((n0 + CB * c) * ES + g * KL * ldb) : kBufOOB;
@@ -327,7 +329,8 @@ void launch_rows(const Params& p, const SkinnyPlan& pl, bool both, hipStream_t s
 
 }  // namespace
 
-SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems, int cus) {
+SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems,
+                       int cus) {
   SkinnyPlan pl{};
   const int64_t es = bf16 ? 2 : 4, nd = dual ? 2 : 1;
   pl.blocks = (int)((M + 63) / 64);
@@ -377,7 +380,8 @@ SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, 
   return pl;
 }
 
-hipError_t launch_skinny(const Params& p, const SkinnyPlan& pl, bool bf16, bool transB, bool dual, hipStream_t stream) {
+hipError_t launch_skinny(const Params& p, const SkinnyPlan& pl, bool bf16, bool transB, bool dual,
+                         hipStream_t stream) {
   const bool both = dual && !pl.part;
   if (bf16)
     transB ? launch_rows<__bf16, true>(p, pl, both, stream) : launch_rows<__bf16, false>(p, pl, both, stream);

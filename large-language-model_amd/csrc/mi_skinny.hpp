@@ -31,10 +31,12 @@ struct SkinnyPlan {
 
 // Plan for C[M, N] = A[M, K] op(B) on a chip of `cus` compute units.  ws_elems: fp32 partials
 // the workspace holds.
-SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems, int cus);
+SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, int64_t K, int64_t ws_elems,
+                       int cus);
 
 // p as for the GEMM kernels (op(A) not transposed, one problem, one K segment, no causal
 // structure, p.splits set to the plan's); dual: p.B2 holds the second B of the SiLU gate.
-hipError_t launch_skinny(const Params& p, const SkinnyPlan& pl, bool bf16, bool transB, bool dual, hipStream_t stream);
+hipError_t launch_skinny(const Params& p, const SkinnyPlan& pl, bool bf16, bool transB, bool dual,
+                         hipStream_t stream);
 
 }  // namespace mig
