@@ -370,13 +370,25 @@ SkinnyPlan skinny_plan(bool bf16, bool transB, bool dual, int64_t M, int64_t N, 
   pl.cols = cols_of(pl.part);
   pl.strips = (int)strips_of(pl.part);
   // Strips past two or three to a CU are short work for a workgroup each, and 128-row tiles
-  // leave no CU idle either: the tile kernels take them, but for a few rows only while K is
-  // short (us, skinny and tile: 2 x 32000 x 112 bf16 NT 11.5 and 6.6, 3 x 32000 x 1152 19.3
-  // and 17.1, 8 x 32000 x 2048 cold 0.8 of the tile's time, 7 x 32000 x 64 fp32 NT 13.1 and
-  // 7.1; 26 x 32000 x 2424 fp32 NT 119 and 84; 64 x 32000 x 192 bf16 dual 16.9 and 12.9).
-  const int64_t per_cu = M > 32 ? (dual ? 1 : 2) : M > 16 ? 3 : 2;
-  pl.take = pl.part || M > SKINNY_MAX_M || pl.strips <= per_cu * cus ||
-            (M <= 16 && K * es >= (pl.strips > 4 * cus ? 3072 : 1024));
+  // leave no CU idle either.  Where whole-K workgroups then have the lower time, by bytes of a
+  // row of K, skinny over tile with B in the caches and cold: M <= 16 NN bf16 1.31 / 1.39 at
+  // 256, 0.96 / 1.07 at 2048, fp32 1.19 / - at 256, 0.79 / 0.77 at 1024; NT past 4 strips a CU
+  // bf16 1.37 / 1.14 at 1024, 0.94 / 0.80 at 4096, fp32 1.11 at 1024, 0.90 / 0.98 at 2048;
+  // M <= 32 NN 1.0 / 1.2 at 256, 0.8 / 1.0 at 1024, 1.03 / 1.2 at 8192 (fp32 0.72 / 0.94), NT
+  // past 4 strips 1.4 at 512, 1.0 / 1.35 at 2048; M <= 64 NT bf16 0.85 / 0.96 at 512, 0.8 / 0.93
+  // to 4 strips at 1024, else past 1.1 (2 x 32000 x 112 bf16 NT 11.5 us, tile 6.6; 26 x 32000 x
+  // 2424 fp32 NT 119 and 84; 20 x 32000 x 768 fp32 NN 20.6 and 27.5).
+  const int64_t row = K * es, s = pl.strips, big = (int64_t)1 << 40;
+  auto within = [&](int64_t lo, int64_t hi) { return lo <= row && row <= hi; };
+  if (pl.part || M > SKINNY_MAX_M) pl.take = true;
+  else if (M > 32)
+    pl.take = s <= (dual && !transB ? cus : 2 * cus) ||
+              (bf16 && transB && !dual && within(0, s <= 4 * cus ? 1024 : 512));
+  else if (s <= 3 * cus) pl.take = true;
+  else if (transB && s > 4 * cus) pl.take = M <= 16 && !(bf16 && dual) && within(bf16 ? 4096 : 1536, big);
+  else if (transB) pl.take = within(768, big);
+  else if (bf16) pl.take = M <= 16 ? !dual && within(2048, big) : within(512, 4096);
+  else pl.take = within(512, M <= 16 ? big : 8192);
   return pl;
 }
 
