@@ -294,12 +294,14 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
     // through HBM: whole blocks 0.82 and 0.81 at 64, 0.92 and 0.90 at 320, 0.93 and 1.00 at
     // 640, 0.97 and 1.01 at 896, 1.06 and 1.08 at 1024 to 1216; cut blocks 0.91 up to 128, 1.02
     // at 192; general epilogue 1.1 at 64.
-    // fp32 C: as many rounding chains (two in a W tile) as S tiles split to fill the CUs once.
+    // fp32 C: at least half as many rounding chains (two in a W tile) as S tiles split to fill
+    // the CUs once (error against 64 bits up to 1.4 times theirs, 1.4e-7 at K = 1000; as many
+    // chains would cost a second launch: TN 64 x 1984 x 752 8.8 us whole, 12.1 split 2).
     if (fast && (tilesS * 2 < cus || (Ktot < 1024 && tilesS * 4 <= 3 * cus))) {
       const int even = tilesS * 2 < cus ? split_of(tilesS, 32, false) : 1;
       const bool short_k = direct == 1 ? Ktot < 1024 : direct == 3 && Ktot <= 128;
       if (short_k && (even == 1 || dtype_c != MI_F32)) return plan_for(CFG_S, 1);
-      int least = dtype_c == MI_F32 ? (even + 1) / 2 : 1;
+      int least = dtype_c == MI_F32 ? (even + 3) / 4 : 1;
       while (!fits(least)) --least;
       const double kt = (double)cdiv(Ktot, 64);
       int best = least;
@@ -369,7 +371,9 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
   // 40-2048 rows: 0.9 % faster than the share's plan and never more than 5 % slower, error
   // against 64 bits no larger; without the bound on the chains 1.2 %, but up to 9 % slower and
   // an error up to 2.2 times as large (256 x 3180 x 4288 NN: 64x128 split 5 64.6 us, 3.7e-7;
-  // 64x64 whole 72, 5.8e-7).
+  // 64x64 whole 72, 5.8e-7).  Where that asks for two splits of a product that three or four
+  // would share evenly, the 64x64 tile with four chains (Q) may still take it whole, by the same
+  // time (384 x 1664 x 640 TN: 64x128 split 3 19.5 us, whole 14.9; 236 x 2485 x 984 26 and 21).
   // Causally cut products (the attention's) take 64x64 tiles, which waste less on the diagonal:
   // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304;
   // uncut batches do not (47 of 1536 x 256 x 61 TN 64x64 34.5 us, 64x128 30.3; 48 of 1152 x
@@ -381,15 +385,15 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
   // 47 78 67 83 65 73 76 71; 36 tiles: 16 28 37 44 49 52 54 41).
   if (fast) {
     int best_cfg = CFG_M, best_sp = 1;
-    // the best plan of at least `least` splits by its time, else by its share; false if the
-    // workspace (of the timed pass) holds none
+    // the best plan of at least `least` splits by its time, else by its share, and its score
+    // (1e300 if the workspace, of the timed pass, holds none)
     auto search = [&](bool timed, int least) {
       double best_score = 1e300;
       for (int cfg : {CFG_V, CFG_M}) {
         if (cfg == CFG_V && cut) continue;
         const CfgShape t = shape_of(dtype_in, cfg);
         const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
-        for (int sp = least; sp <= (allow_split ? 8 : 1); ++sp) {
+        for (int sp = least; sp <= (allow_split || !timed ? 8 : 1); ++sp) {
           const int64_t units = tiles * sp;
           if (sp > 1) {
             if (units > 3 * (int64_t)cus || (timed && (int64_t)sp * M * N * batch > ws_limit_elems)) continue;
@@ -406,10 +410,18 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
           if (wins) best_cfg = cfg, best_sp = sp, best_score = score;
         }
       }
-      return best_score < 1e300;
+      return best_score;
     };
     search(false, 1);
-    for (int least = (best_sp + 1) / 2; !search(true, least); --least) {}
+    const int even = best_sp;
+    double best = 1e300;
+    for (int least = (even + 1) / 2; best == 1e300; --least) best = search(true, least);
+    if (even > 2 && even <= 4) {
+      const int64_t tiles = cdiv(M, 64) * cdiv(N, 64) * batch;
+      const double whole = (double)cdiv(tiles, cus) * 64 * 64 * (double)Ktot / (128 * 2100.0);
+      // no room for its splits: whole it is, in four chains as with the room
+      if (2 * best_sp < even ? batch == 1 : best_sp > 1 && whole < best) return plan_for(CFG_Q, 1);
+    }
     return plan_for(best_cfg, best_sp);
   }
   if (tilesS * 8 >= (int64_t)cus * 5 || !allow_split) return plan_for(CFG_S, 1);
@@ -459,6 +471,7 @@ void describe_plan(char* buf, size_t len, int dtype_in, bool fast, const Plan& p
   const CfgShape sh = shape_of(dtype_in, pl.cfg);
   const char* kind = (dtype_in == MI_BF16 && fast && pl.cfg != CFG_PRO)
                          ? (pl.cfg == CFG_W || pl.cfg == CFG_V || pl.cfg == CFG_DUAL_W ? "dlds-kg2" : "dlds")
+                     : dtype_in != MI_BF16 && fast && pl.cfg == CFG_Q ? "dlds-c4"
                      : (dtype_in != MI_BF16 && fast && (pl.cfg == CFG_V || pl.cfg == CFG_M || pl.cfg == CFG_DUAL_S))
                          ? "dlds"
                          : "regstage";

@@ -292,8 +292,9 @@ struct DldsOperand {
 // (STRADDLE, with KTAIL: the rest of the chunk that straddles the end is zeroed in LDS), and
 // the problem takes the direct epilogue (every tile full, epilogue alpha / SiLU
 // gate, beta*C and the output conversion only, no split-K).  One kernel holding
-// both epilogues would need the accumulators in two places at once.
-enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4, DLDS_EDGE = 8, DLDS_STRADDLE = 16 };
+// both epilogues would need the accumulators in two places at once.  CHAINS4 (fp32): K in
+// four rounding chains instead of two.
+enum { DLDS_KTAIL = 1, DLDS_FAST_EPI = 2, DLDS_ROWSCALE = 4, DLDS_EDGE = 8, DLDS_STRADDLE = 16, DLDS_CHAINS4 = 32 };
 
 // GEMM of WGM x WGN waves, wave tile (BM/WGM) x (BN/WGN) of 32x32 MFMA blocks: bf16
 // (ES = 2, one 32x32x16 MFMA per block and substep) or fp32 (ES = 4, four 32x32x2).
@@ -421,20 +422,25 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  // fp32: every other MFMA of a fragment pair sums into accumulators of its own, joined at
-  // the end: each rounding chain is half as long, as if K were split in two, which keeps the
-  // products that the planner splits less than it could as close to their 64-bit values as
-  // the split would.  LDS bounds the workgroups per CU (5 of 64x64, 3 of 64x128), so the
-  // registers are there; held in VGPRs (waves_per_eu above) they cost no time, where moving
-  // both sets out of accumulation registers at a tile's end cost 1.5 % (training block on 2048
-  // tokens 771-779 us; here 776, one set 776).  Error against 64 bits: that block 8.1e-7 ->
-  // 5.7e-7, the materialised attention 5.6e-7 -> 4.0e-7.
-  f32x16_t acc_odd[ES == 4 ? TM : 1][ES == 4 ? NB : 1];
+  // fp32: every other MFMA of a fragment pair sums into accumulators of its own (CHAINS4:
+  // every one of the four), joined at the end: each rounding chain is half (a quarter) as
+  // long, as if K were split in two (four), which keeps the products that the planner splits
+  // less than it could as close to their 64-bit values as the split would.  LDS bounds the
+  // workgroups per CU (5 of 64x64, 3 of 64x128), so the registers are there (four chains of a
+  // 64x64 tile: 4 workgroups, on grids that rarely have as many); held in VGPRs (waves_per_eu
+  // above) they cost no time, where moving both sets out of accumulation registers at a
+  // tile's end cost 1.5 % (training block on 2048 tokens 771-779 us; here 776, one set 776).
+  // Error against 64 bits: that block 8.1e-7 -> 5.7e-7, the materialised attention 5.6e-7 ->
+  // 4.0e-7.
+  constexpr int NX = ES != 4 ? 0 : (VAR & DLDS_CHAINS4) != 0 ? 3 : 1;  // further sets
+  f32x16_t acc_x[NX ? NX : 1][ES == 4 ? TM : 1][ES == 4 ? NB : 1];
   if constexpr (ES == 4) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int x = 0; x < NX; ++x)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) acc_odd[i][j] = acc[i][j];
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc_x[x][i][j] = acc[i][j];
   }
 
   OpA oa;
@@ -554,9 +560,11 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
       // fp32: value t of both fragments is k = 8S + t (lanes 0-31) and 8S + 4 + t
       // (lanes 32-63), the two k of one 32x32x2 MFMA
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        (t & 1 ? acc_odd : acc)[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-            __uint_as_float(fb[set][j][t]), __uint_as_float(fa[set][i][t]), (t & 1 ? acc_odd : acc)[i][j], 0, 0, 0);
+      for (int t = 0; t < 4; ++t) {
+        f32x16_t& sum = t % (NX + 1) == 0 ? acc[i][j] : acc_x[t % (NX + 1) - 1][i][j];
+        sum = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[set][j][t]), __uint_as_float(fa[set][i][t]),
+                                                   sum, 0, 0, 0);
+      }
     }
   };
 
@@ -749,7 +757,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN * KG)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] += acc_odd[i][j][e];
+        for (int e = 0; e < 16; ++e) {
+          if constexpr (NX == 3) acc_x[0][i][j][e] += acc_x[2][i][j][e], acc[i][j][e] += acc_x[1][i][j][e];
+          acc[i][j][e] += acc_x[0][i][j][e];
+        }
   }
 
   // acc[i][j][4q + e] holds C[m][n + e] with

@@ -121,6 +121,7 @@ KernelFn dlds32_kernel(int cfg) {
   switch (cfg) {
     case CFG_V: return gemm_dlds_kernel<64, 128, 32, 2, AK, BK, MODE_PLAIN, V, 2, 2, 1, 4>;
     case CFG_M: return gemm_dlds_kernel<64, 64, 32, 2, AK, BK, MODE_PLAIN, V, 2, 2, 1, 4>;
+    case CFG_Q: return gemm_dlds_kernel<64, 64, 32, 2, AK, BK, MODE_PLAIN, V | DLDS_CHAINS4, 2, 2, 1, 4>;
     case CFG_DUAL_S: return gemm_dlds_kernel<64, 64, 32, 2, AK, BK, MODE_DUAL, V, 2, 2, 1, 4>;
     default: return nullptr;
   }

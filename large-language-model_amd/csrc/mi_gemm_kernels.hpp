@@ -19,10 +19,11 @@ typedef void (*KernelFn)(Params);
 //         groups of 4 waves of 64x96).
 //   SKINNY (either type): products of up to 64 rows and small fp32 ones in blocks of 64
 //         rows, mi_skinny.hip (the shape is in skinny_plan).
-//   fp32: V 64x128, M 64x64 and DUAL_S 64x64 of each B direct-to-LDS (four waves);
+//   fp32: V 64x128, M 64x64, Q 64x64 with four rounding chains instead of two, and DUAL_S
+//         64x64 of each B direct-to-LDS (four waves);
 //         register-staged S 128x128, DUAL 128x64, PRO 128x128.
 enum Cfg { CFG_L = 0, CFG_S = 1, CFG_DUAL = 2, CFG_PRO = 3, CFG_W = 4, CFG_M = 5, CFG_V = 6, CFG_SKINNY = 7,
-           CFG_DUAL_S = 8, CFG_DUAL_W = 9, CFG_DUAL_M = 10, CFG_DUAL_L = 11 };
+           CFG_DUAL_S = 8, CFG_DUAL_W = 9, CFG_DUAL_M = 10, CFG_DUAL_L = 11, CFG_Q = 12 };
 
 struct CfgShape {
   int bm, bn;
@@ -52,7 +53,7 @@ inline CfgShape cfg_shape(bool bf16, int cfg) {
   // others the register-staged kernel (four waves)
   return cfg == CFG_DUAL ? CfgShape{128, 64}
        : cfg == CFG_V    ? CfgShape{64, 128}
-       : cfg == CFG_M || cfg == CFG_DUAL_S ? CfgShape{64, 64}
+       : cfg == CFG_M || cfg == CFG_Q || cfg == CFG_DUAL_S ? CfgShape{64, 64}
                          : CfgShape{128, 128};
 }
 

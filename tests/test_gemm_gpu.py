@@ -970,3 +970,33 @@ def test_cut_blocks_of_transposed_a(mi, dev, bf16, M, N, K, want, tB):
         mi.gemm(A, B, C, M, N, K, transA=True, transB=bool(tB), beta=beta, ldc=ldc)
         assert torch.equal(C, (ref + 3.0 * beta).float()), (ldc, beta)
         assert buf[:, N:].isnan().all()
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)], ids=["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("M,N,K", [(384, 1664, 640), (375, 1545, 468), (236, 2488, 984), (384, 1668, 645)])
+def test_fp32_four_chains(mi, dev, tA, tB, M, N, K):
+    """The fp32 tile with four rounding chains on whole and cut blocks, K in whole tiles, whole chunks
+    and neither, in the direct and the general epilogue: integers bit for bit; and random values no
+    further from 64 bits than K in four parts, whose sums' errors grow as sqrt(K / 4): a partial sum
+    of k products rounds by at most 2^-24 sqrt(k) of their rms, in all 2^-24 sqrt(K / 8) of the
+    result's rms, doubled for the spread."""
+    import torch
+
+    assert mi.describe(tA, tB, M, N, K, mi.MI_F32).startswith("dlds-c4 f32 64x64")
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    bias = torch.randint(-3, 4, (N,), generator=g, device=dev).float()
+    for draw in ("integers", "normal"):
+        mk = (lambda *s: torch.randint(-4, 5, s, generator=g, device=dev).float()) if draw == "integers" else (
+            lambda *s: torch.randn(s, generator=g, device=dev))  # noqa: E731
+        a, b = mk(M, K), mk(K, N)
+        A, B = (a.T if tA else a).contiguous(), (b.T if tB else b).contiguous()
+        ref = a.double() @ b.double()
+        for kw in ({}, {"bias": bias}):
+            C = torch.full((M, N), float("nan"), device=dev)
+            mi.gemm(A, B, C, M, N, K, transA=bool(tA), transB=bool(tB), **kw)
+            want = ref + bias.double() if kw else ref
+            if draw == "integers":
+                assert torch.equal(C.double(), want)
+            else:
+                rel = ((C.double() - want).norm() / want.norm()).item()
+                assert rel <= 2.0 ** -24 * 2 * (K / 8) ** 0.5, rel
