@@ -373,7 +373,8 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
   // an error up to 2.2 times as large (256 x 3180 x 4288 NN: 64x128 split 5 64.6 us, 3.7e-7;
   // 64x64 whole 72, 5.8e-7).  Where that asks for two splits of a product that three or four
   // would share evenly, the 64x64 tile with four chains (Q) may still take it whole, by the same
-  // time (384 x 1664 x 640 TN: 64x128 split 3 19.5 us, whole 14.9; 236 x 2485 x 984 26 and 21).
+  // time and a tenth (384 x 1664 x 640 TN: 64x128 split 3 18.9 us, 2.7e-7, whole 13.2, 2.3e-7;
+  // 375 x 1545 x 468 NN 13.9; 1664 x 392 x 2184 TN: 64x64 split 4 36.8, whole 40.9).
   // Causally cut products (the attention's) take 64x64 tiles, which waste less on the diagonal:
   // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304;
   // uncut batches do not (47 of 1536 x 256 x 61 TN 64x64 34.5 us, 64x128 30.3; 48 of 1152 x
@@ -418,7 +419,7 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
     for (int least = (even + 1) / 2; best == 1e300; --least) best = search(true, least);
     if (even > 2 && even <= 4) {
       const int64_t tiles = cdiv(M, 64) * cdiv(N, 64) * batch;
-      const double whole = (double)cdiv(tiles, cus) * 64 * 64 * (double)Ktot / (128 * 2100.0);
+      const double whole = 1.1 * (double)cdiv(tiles, cus) * 64 * 64 * (double)Ktot / (128 * 2100.0);
       // no room for its splits: whole it is, in four chains as with the room
       if (2 * best_sp < even ? batch == 1 : best_sp > 1 && whole < best) return plan_for(CFG_Q, 1);
     }
