@@ -374,7 +374,13 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
   // 64x64 whole 72, 5.8e-7).  Where that asks for two splits of a product that three or four
   // would share evenly, the 64x64 tile with four chains (Q) may still take it whole, by the same
   // time and a tenth (384 x 1664 x 640 TN: 64x128 split 3 18.9 us, 2.7e-7, whole 13.2, 2.3e-7;
-  // 375 x 1545 x 468 NN 13.9; 1664 x 392 x 2184 TN: 64x64 split 4 36.8, whole 40.9).
+  // 375 x 1545 x 468 NN 13.9; 1664 x 392 x 2184 TN: 64x64 split 4 36.8, whole 40.9).  In place of
+  // five and more even splits Q takes half as many as the other two would, its time counted a
+  // twentieth higher (1424 such NN, TN: 0.88 of the time at the median; 561 x 510 x 971 TN 64x128
+  // split 6 21.8 us, Q split 3 16.4, error 1.7e-7 both).  Not at a long K, which a lone workgroup
+  // on a CU walks slower in Q (1152 x 384 x 3968 NN split 7 36.4, Q split 2 42.4), and not NT,
+  // where it would be quicker (0.86) but 1.07 times further from 64 bits, up to 1.3, than the even
+  // splits that such products have run in.
   // Causally cut products (the attention's) take 64x64 tiles, which waste less on the diagonal:
   // forward and backward of 48 heads of 512 x 64 149 -> 143 us, 16 of 1000 x 128 323 -> 304;
   // uncut batches do not (47 of 1536 x 256 x 61 TN 64x64 34.5 us, 64x128 30.3; 48 of 1152 x
@@ -385,16 +391,17 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
   // tiles at K = 2048: splits 1..8 ran 43 71 59 74 83 66 69 76 TFLOP/s; 108 tiles:
   // 47 78 67 83 65 73 76 71; 36 tiles: 16 28 37 44 49 52 54 41).
   if (fast) {
-    int best_cfg = CFG_M, best_sp = 1;
+    int best_cfg = CFG_M, best_sp = 1, even = 1;
     // the best plan of at least `least` splits by its time, else by its share, and its score
     // (1e300 if the workspace, of the timed pass, holds none)
     auto search = [&](bool timed, int least) {
       double best_score = 1e300;
-      for (int cfg : {CFG_V, CFG_M}) {
+      for (int cfg : {CFG_V, CFG_M, CFG_Q}) {
         if (cfg == CFG_V && cut) continue;
+        if (cfg == CFG_Q && (!timed || even <= 4 || batch > 1 || Ktot > 3072 || (!transA && transB))) continue;
         const CfgShape t = shape_of(dtype_in, cfg);
         const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn) * batch;
-        for (int sp = least; sp <= (allow_split || !timed ? 8 : 1); ++sp) {
+        for (int sp = cfg == CFG_Q ? (least + 1) / 2 : least; sp <= (allow_split || !timed ? 8 : 1); ++sp) {
           const int64_t units = tiles * sp;
           if (sp > 1) {
             if (units > 3 * (int64_t)cus || (timed && (int64_t)sp * M * N * batch > ws_limit_elems)) continue;
@@ -402,7 +409,7 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
           }
           double score = (double)cdiv(units, cus) * t.bm * t.bn / sp;
           if (timed) {
-            score *= (double)Ktot / (128 * 2100.0);
+            score *= (cfg == CFG_Q ? 1.05 : 1.0) * (double)Ktot / (128 * 2100.0);
             if (sp > 1) score += 2.5 + 8.0 * (double)(sp * M * N * batch) / 3e6;
           }
           const bool wins = score < best_score ||
@@ -414,7 +421,7 @@ Plan make_plan(int dtype_in, int dtype_c, int transA, int transB, int64_t M, int
       return best_score;
     };
     search(false, 1);
-    const int even = best_sp;
+    even = best_sp;
     double best = 1e300;
     for (int least = (even + 1) / 2; best == 1e300; --least) best = search(true, least);
     if (even > 2 && even <= 4) {
@@ -472,13 +479,14 @@ void describe_plan(char* buf, size_t len, int dtype_in, bool fast, const Plan& p
   const CfgShape sh = shape_of(dtype_in, pl.cfg);
   const char* kind = (dtype_in == MI_BF16 && fast && pl.cfg != CFG_PRO)
                          ? (pl.cfg == CFG_W || pl.cfg == CFG_V || pl.cfg == CFG_DUAL_W ? "dlds-kg2" : "dlds")
-                     : dtype_in != MI_BF16 && fast && pl.cfg == CFG_Q ? "dlds-c4"
-                     : (dtype_in != MI_BF16 && fast && (pl.cfg == CFG_V || pl.cfg == CFG_M || pl.cfg == CFG_DUAL_S))
+                     : (dtype_in != MI_BF16 && fast &&
+                        (pl.cfg == CFG_V || pl.cfg == CFG_M || pl.cfg == CFG_Q || pl.cfg == CFG_DUAL_S))
                          ? "dlds"
                          : "regstage";
-  std::snprintf(buf, len, "%s %s %dx%d %s%s split%d tiles%lld", kind,
+  std::snprintf(buf, len, "%s %s %dx%d %s%s split%d tiles%lld%s", kind,
                 dtype_in == MI_BF16 ? "bf16" : "f32", sh.bm, sh.bn, transA ? "T" : "N",
-                transB ? "T" : "N", pl.splits, (long long)pl.tiles_m * pl.tiles_n * batch);
+                transB ? "T" : "N", pl.splits, (long long)pl.tiles_m * pl.tiles_n * batch,
+                pl.cfg == CFG_Q ? " chains4" : "");
 }
 
 // ---- per-call GEMM profiler ----------------------------------------------------

@@ -313,7 +313,8 @@ def test_loader_follows_alignment(mi, dt, M, N, K):
 def test_fp32_plans_keep_their_chains(mi):
     """The fp32 planner sums K in as many rounding chains (splits x the two or four of a tile) as the
     plan that shares the work most evenly among the CUs splits it into, so that a quicker plan is
-    never a less accurate one; and it plans NN, NT and TN alike."""
+    never a less accurate one; and it plans NN, NT and TN alike but for splits of the four-chain
+    tile, which NT does not take."""
     cus, deeper = 256, 0
 
     def even_split(M, N, K):
@@ -334,12 +335,14 @@ def test_fp32_plans_keep_their_chains(mi):
     shapes += [tuple(int(x) for x in np.exp(rng.uniform(np.log(65), np.log(4096), 3))) for _ in range(300)]
     for M, N, K in shapes:
         texts = [mi.describe(tA, tB, M, N, K, mi.MI_F32, workspace_bytes=1 << 34) for tA, tB in ((0, 0), (0, 1), (1, 0))]
-        assert texts[1].replace("NT", "TN") == texts[2], (M, N, K, texts)
+        if not (texts[2].endswith("chains4") and "split1 " not in texts[2]):  # NT sums in more chains there
+            assert texts[1].replace("NT", "TN") == texts[2], (M, N, K, texts)
         if not texts[0].startswith("skinny"):
             assert texts[0].replace("NN", "TN") == texts[2], (M, N, K, texts)
         need = even_split(M, N, K)
-        chains = int(re.search(r"split(\d+)", texts[2]).group(1)) * (4 if texts[2].startswith("dlds-c4") else 2)
-        assert chains >= need, (M, N, K, texts[2], need)
+        for text in texts[1:]:
+            chains = int(re.search(r"split(\d+)", text).group(1)) * (4 if text.endswith("chains4") else 2)
+            assert chains >= need, (M, N, K, text, need)
         own = mi.workspace_size(1, 0, M, N, K, mi.MI_F32, mi.MI_F32)  # no room beyond the plan's own partials
         assert mi.describe(1, 0, M, N, K, mi.MI_F32, workspace_bytes=own) == texts[2], (M, N, K, own)
         deeper += need > 2

@@ -7,6 +7,7 @@ benchmark configurations are checked on sampled rows against the oracle and on
 every element through row/column checksums.
 """
 import itertools
+import re
 
 import numpy as np
 import pytest
@@ -982,7 +983,7 @@ def test_fp32_four_chains(mi, dev, tA, tB, M, N, K):
     result's rms, doubled for the spread."""
     import torch
 
-    assert mi.describe(tA, tB, M, N, K, mi.MI_F32).startswith("dlds-c4 f32 64x64")
+    assert re.match("dlds f32 64x64 .* chains4", mi.describe(tA, tB, M, N, K, mi.MI_F32))
     g = torch.Generator(device=dev).manual_seed(M + K)
     bias = torch.randint(-3, 4, (N,), generator=g, device=dev).float()
     for draw in ("integers", "normal"):
@@ -1000,3 +1001,33 @@ def test_fp32_four_chains(mi, dev, tA, tB, M, N, K):
             else:
                 rel = ((C.double() - want).norm() / want.norm()).item()
                 assert rel <= 2.0 ** -24 * 2 * (K / 8) ** 0.5, rel
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (1, 0), (1, 1)], ids=["NN", "TN", "TT"])
+@pytest.mark.parametrize("M,N,K,split", [(512, 768, 1088, 2), (220, 1134, 1280, 3), (561, 510, 971, 3)])
+def test_fp32_four_chains_split(mi, dev, tA, tB, M, N, K, split):
+    """The four-chain tile with K in parts: integers bit for bit, with beta and without, the workspace
+    NaN on entry; and random values no further from 64 bits than a sum in 4 x split parts, as in
+    test_fp32_four_chains."""
+    import torch
+
+    assert re.match("dlds f32 64x64 .* chains4", mi.describe(tA, tB, M, N, K, mi.MI_F32, workspace_bytes=1 << 30))
+    need = mi.workspace_size(tA, tB, M, N, K, mi.MI_F32, mi.MI_F32)
+    assert need == split * M * N * 4
+    ws = torch.full((need // 4,), float("nan"), device=dev)
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    for draw in ("integers", "normal"):
+        mk = (lambda *s: torch.randint(-4, 5, s, generator=g, device=dev).float()) if draw == "integers" else (
+            lambda *s: torch.randn(s, generator=g, device=dev))  # noqa: E731
+        a, b = mk(M, K), mk(K, N)
+        A, B = (a.T if tA else a).contiguous(), (b.T if tB else b).contiguous()
+        ref = a.double() @ b.double()
+        for beta in (0.0, 1.0):
+            C = torch.full((M, N), 3.0 if beta else float("nan"), device=dev)
+            mi.gemm(A, B, C, M, N, K, transA=bool(tA), transB=bool(tB), beta=beta, workspace=ws)
+            want = ref + 3.0 * beta
+            if draw == "integers":
+                assert torch.equal(C.double(), want)
+            else:
+                rel = ((C.double() - want).norm() / want.norm()).item()
+                assert rel <= 2.0 ** -24 * 2 * (K / (8 * split)) ** 0.5 + 2.0 ** -24, rel
